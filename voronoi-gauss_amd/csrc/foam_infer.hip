@@ -15,149 +15,16 @@
 #include <cmath>
 #include <type_traits>
 
-#include "vgr_abi.h"
-#include "vgr_device.h"
+#include "vgr_foam.h"
 
 namespace vgr {
 namespace {
 
 constexpr int kBlock = 64;  // one wave64 per workgroup = one 8x8 ray tile
-constexpr int kLazy = VGR_COLOR_LAZY, kBaked = VGR_COLOR_BAKED, kFused = VGR_COLOR_FUSED;
 // Fused colours over the indexed edge records (vgr_foam_index_pack): the neighbour's index in the fourth word of its
 // edge record and its cut-off word in attr[:, 7], so a neighbour round loads no separate index. An internal mode of
 // this file: it blends exactly as kFused.
 constexpr int kFusedIdx = 3;
-
-struct FoamScene {
-    const float4* __restrict__ points;  // (N) p, w unused
-    const int* __restrict__ offsets;    // (N + 1) self-first
-    const int* __restrict__ nbr;        // (E)
-    const float4* __restrict__ edge;    // (E) p_j, half2(r2_j, lam_j)
-    const float4* __restrict__ attr;    // (N, 5)
-    const float4* __restrict__ sh;      // (N, 12) fp32 or (N, 6) fp16
-    const int* __restrict__ orig;       // (N) or null
-    const int4* __restrict__ slots;     // (N, 4) slot table (vgr_foam_slot_table) or null
-    const float4* __restrict__ rows;    // site rows (the first 16 attr columns) or null, row_stride float4 apart
-    int n_sites;
-    int row_stride;  // float4 from one site row to the next: 4 (64-byte rows) or 16 (256-byte site blocks)
-    int sh_stride;   // float4 from one SH row to the next: 12 (fp32), 6 (fp16) or 16 (the SH rows of site blocks)
-};
-
-struct FoamParams {
-    float t_thresh, w_thresh, color_cut;
-    int sh_deg;
-};
-
-struct FoamRays {
-    const float* __restrict__ o;
-    const float* __restrict__ d;
-    const int* __restrict__ start;
-    const float* __restrict__ t_near;
-    const float* __restrict__ t_far;
-    const int* __restrict__ cap;
-    int64_t n;
-    const int* __restrict__ order;  // processing order of the rays (a permutation of 0 .. n - 1), or null
-};
-
-struct FoamOut {
-    float* __restrict__ rgb;
-    float* __restrict__ T;
-    float* __restrict__ depth;
-    int* __restrict__ stats;
-    int* __restrict__ trace;
-    int64_t trace_cap;
-};
-
-// Running normalised colour blend (fused / baked modes).
-struct Blend {
-    float m, a, r, g, b;
-};
-
-__device__ __forceinline__ void blend_init(Blend& B) { B.m = kInf, B.a = B.r = B.g = B.b = 0.f; }
-
-// k precedes j in the tie-breaking order: the smaller original index.
-__device__ __forceinline__ bool before(const FoamScene& S, int k, int j) {
-    return S.orig != nullptr ? S.orig[k] < S.orig[j] : k < j;
-}
-
-// (r2, lam) half2 packed in the 4th component of an edge record.
-__device__ __forceinline__ float2 cutoffs(float w) {
-    const uint32_t u = __float_as_uint(w);
-    const _Float16 lo = __builtin_bit_cast(_Float16, static_cast<uint16_t>(u & 0xffffu));
-    const _Float16 hi = __builtin_bit_cast(_Float16, static_cast<uint16_t>(u >> 16));
-    return make_float2(static_cast<float>(lo), static_cast<float>(hi));
-}
-
-// ------------------------------------------------------------------ field arithmetic (explicit FMA)
-// The density, colour and blend arithmetic below fuses chosen products and sums into one FMA (fmaf), which rounds
-// once where the CPU oracle rounds twice: each term moves by at most an ulp of its magnitude, and the colours and
-// transmittances by a few ulps of 1 (about 1e-6), well inside the 1e-4 parity bar. The fusions are written out, not
-// left to the compiler's contraction, so every kernel of this file that composes these terms rounds them the same
-// way whatever the surrounding code and register schedule. The traversal arithmetic (walk distances, exit planes)
-// is never fused, so the visited cells stay bit-exact.
-
-__device__ __forceinline__ void blend_add(Blend& B, float m, float r, float g, float b) {
-    if (m < B.m) {
-        const float s = fexp(-0.5f * (B.m - m));
-        B.a *= s, B.r *= s, B.g *= s, B.b *= s, B.m = m;
-    }
-    const float w = fexp(-0.5f * (m - B.m));
-    B.a += w, B.r = fmaf(w, r, B.r), B.g = fmaf(w, g, B.g), B.b = fmaf(w, b, B.b);
-}
-
-// (vx, vy, vz) A (vx, vy, vz)^T for the symmetric conic A = (p.x p.y p.z / . p.w q.x / . . q.y)
-__device__ __forceinline__ float maha_f(const float4& p, const float4& q, float vx, float vy, float vz) {
-    const float diag = fmaf(p.x * vx, vx, fmaf(p.w * vy, vy, q.y * vz * vz));
-    const float cross = fmaf(p.y * vx, vy, fmaf(p.z * vx, vz, q.x * vy * vz));
-    return fmaf(2.f, cross, diag);
-}
-
-// Sample point o + t d, used by the field terms only (the traversal never reads it).
-__device__ __forceinline__ void sample_point(const float (&o)[3], const float (&d)[3], float t, float (&x)[3]) {
-    x[0] = fmaf(t, d[0], o[0]), x[1] = fmaf(t, d[1], o[1]), x[2] = fmaf(t, d[2], o[2]);
-}
-
-__device__ __forceinline__ void offset_of(const float (&x)[3], const float4& p, float& v0, float& v1, float& v2,
-                                          float& r2) {
-    v0 = x[0] - p.x, v1 = x[1] - p.y, v2 = x[2] - p.z;
-    r2 = fmaf(v0, v0, fmaf(v1, v1, v2 * v2));
-}
-
-// rho_k G_k(x) from the density record (q0 = xx xy xz yy, q1 = yz zz min(raw, 30) 0).
-__device__ __forceinline__ float density_term(const float4& q0, const float4& q1, float v0, float v1, float v2) {
-    return fexp(fmaf(-0.5f, maha_f(q0, q1, v0, v1, v2), q1.z));
-}
-
-__device__ __forceinline__ float weight_of(float m, float mmin) { return fexp(-0.5f * (m - mmin)); }
-
-__device__ __forceinline__ void accumulate(float& A, float& r, float& g, float& bl, float w, const float (&c)[3]) {
-    A += w, r = fmaf(w, c[0], r), g = fmaf(w, c[1], g), bl = fmaf(w, c[2], bl);
-}
-
-// Adds blocks q0 .. q0 + 3 (those below nv) of a site's SH coefficients (fp32, or fp16 pairs) to c: the colour
-// SH_k(d) accumulates over the coefficients in storage order, coefficient i of channel i mod 3 times basis i / 3.
-template <bool HALF, int CH = 4>
-__device__ __forceinline__ void sh_accumulate(const float4 (&f)[CH], int q0, int nv, const float (&b)[16],
-                                              float (&c)[3]) {
-#pragma unroll
-    for (int uq = 0; uq < CH; ++uq) {
-        const int q = q0 + uq;
-        if (q >= nv) break;
-        const float fv[4] = {f[uq].x, f[uq].y, f[uq].z, f[uq].w};
-        if (HALF) {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const float2 p = cutoffs(fv[u]);
-                const int i0 = 8 * q + 2 * u, i1 = i0 + 1;
-                c[i0 % 3] = fmaf(b[i0 / 3], p.x, c[i0 % 3]);
-                c[i1 % 3] = fmaf(b[i1 / 3], p.y, c[i1 % 3]);
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) c[(4 * q + u) % 3] = fmaf(b[(4 * q + u) / 3], fv[u], c[(4 * q + u) % 3]);
-        }
-    }
-}
 
 // ------------------------------------------------------------------ traversal arithmetic (never contracted)
 
@@ -196,11 +63,6 @@ template <int SLOTS>
 __device__ __forceinline__ int slot_of(int k) {
     return static_cast<int>(static_cast<uint32_t>(k) % SLOTS);
 }
-
-// Entry e of a neighbourhood [e0, e1) for a load issued ahead of the loop that may not run: clamped into the cell,
-// and for an empty cell (no self entry, which no pack_foam pack has) to the entry before it, so the load stays in
-// bounds whatever the offsets.
-__device__ __forceinline__ int entry_in(int e, int e1) { return max(min(e, e1 - 1), 0); }
 
 // Volatile ints typed as LDS: the election and tag accesses stay ds_read / ds_write. Through a generic pointer
 // they would be flat accesses, after each of which the wave waits for all of its outstanding global loads.
@@ -509,13 +371,6 @@ __device__ __forceinline__ int tags_finish(const FoamScene& S, PassLog& L) { ret
 __device__ __forceinline__ int tags_pass(const FoamScene& S, SlotTags<1>& T, int c) { return table_hits<1>(S, c, 0, T); }
 __device__ __forceinline__ int tags_finish(const FoamScene&, SlotTags<1>&) { return 0; }
 
-// Number of float4 a colour fetch reads: the blocks holding coefficients of degree <= DEG (the others multiply a
-// zero basis value, so leaving them out changes no finite colour).
-template <bool HALF, int DEG>
-constexpr int sh_vec4() {
-    return HALF ? sh_vec4_f16(DEG) : sh_vec4_f32(DEG);
-}
-
 // Greedy walk to the lexicographic argmin of (|x - p|^2, tie order) over {c} U adj(c), repeated. IDX: the edge
 // records carry the neighbour index (indexed pack).
 template <bool IDX = false>
@@ -740,11 +595,6 @@ __device__ void color_lazy(const FoamScene& S, const FoamParams& P, int c, float
     C[0] = r * inv, C[1] = g * inv, C[2] = bl * inv;
 }
 
-template <bool TRACE>
-__device__ __forceinline__ void trace_cell(const FoamScene& S, const FoamOut& O, int64_t r, int s, int c) {
-    if (TRACE && s < O.trace_cap) O.trace[r * O.trace_cap + s] = S.orig != nullptr ? S.orig[c] : c;
-}
-
 // The register allocation is bounded for waves_for waves per SIMD (Tune<COLOR>::waves unless the LDS allows fewer).
 // Six waves per SIMD is the fastest occupancy measured for the fused fp32 degree-3 kernel on config 3 although it
 // spills: 80 VGPRs, the rest of the ray's state (accumulated colour and depth, the basis) stored to scratch once
@@ -878,33 +728,6 @@ __global__ void __launch_bounds__(kBlock, (waves_for<COLOR, kBlock, TABLE>(STAGE
 // (a few ulps). Per lane this layout runs the same face and field arithmetic as one ray per lane, but 64 / G rays
 // per wave keep more independent loads in flight per wave, and a wave's loads of one cell are contiguous.
 
-
-__device__ __forceinline__ bool wave_any(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0; }
-
-// k precedes j in the tie order, INT_MAX (no face) after every site.
-__device__ __noinline__ bool before_or_none(const FoamScene& S, int k, int j) {
-    if (j == INT_MAX) return k != INT_MAX;
-    if (k == INT_MAX) return false;
-    return before(S, k, j);
-}
-
-// Keeps the lexicographic minimum of (t, k) and the candidate (u, j). Exact ties in t are rare: they take a
-// wave-uniform branch, inside which only the tied lanes look up the tie order.
-__device__ __forceinline__ void keep_min(const FoamScene& S, float u, int j, float& t, int& k) {
-    bool take = u < t;
-    const bool tie = u == t && j != k;
-    if (wave_any(tie)) {
-        if (tie) take = before_or_none(S, j, k);
-    }
-    if (take) t = u, k = j;
-}
-
-template <int CTRL>
-__device__ __forceinline__ void min_step(const FoamScene& S, float& t, int& k) {
-    const float u = row_perm<CTRL>(t);
-    const int j = row_perm<CTRL>(k);
-    keep_min(S, u, j, t, k);
-}
 
 template <int G>
 __device__ __forceinline__ void group_min(const FoamScene& S, float& t, int& k) {
@@ -1349,6 +1172,20 @@ inline int default_lanes(int64_t stage, int64_t color_mode) {
     return stage < 2 || color_mode == kLazy ? 4 : 1;
 }
 
+// Below this many rays the default layout of the full rendering (stage 2) is 16 lanes per ray (foam_wide.hip): one ray
+// per lane, or four lanes, leaves a launch as long as its longest ray's chain of dependent reads, whatever its size.
+// Measured on a scene of 131k sites with large cells (90 samples per ray) and one of 1M (160 samples), 8x8 tiles, ms of
+// the render call, 16 lanes against the other layout:
+//   exact and fused colours, fp32 SH  8192 rays 0.65 : 9.9, 1.1 : 23.7; 131072 6.8 : 7.4, 8.9 : 20.0; 262144 10.1 : 8.3,
+//                                     14.0 : 21.4
+//   baked colours                     8192 rays 0.53 : 1.83, 1.09 : 4.3; 65536 1.33 : 1.92, 2.4 : 5.0; 131072 2.7 : 2.1,
+//                                     4.2 : 5.2
+//   exact with a finite cut-off       65536 rays 2.7 : 3.6, 3.8 : 8.7; 131072 6.5 : 5.4, 8.5 : 11.8
+// The lines lie where the worse of the two scenes breaks even.
+inline int64_t wide_rays(int64_t color_mode, bool finite_cut) {
+    return color_mode == kBaked || (color_mode == kLazy && finite_cut) ? 98304 : 131072;
+}
+
 int foam_entry(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t* nbr, const float* edge,
                int64_t n_edges, const float* attr, const void* sh, int32_t sh_half, int64_t sh_deg, const float* o,
                const float* d, const int32_t* start, const float* near_t, const float* far_t, int64_t n_rays,
@@ -1365,6 +1202,7 @@ int foam_entry(const float* points, int64_t n_sites, const int32_t* offsets, con
                              color_mode == kLazy && one_lane && std::isinf(color_cut) && color_cut > 0;
     const bool indexed = exact_blend || (edge_i != nullptr && attr_i != nullptr && stage == 2 &&
                                          color_mode == kFused && one_lane);
+    const bool wide = lanes == kDefaultLanes && stage == 2 && n_rays <= wide_rays(color_mode, !(std::isinf(color_cut) && color_cut > 0));
     if (indexed) lanes = 1;
     if (lanes == kDefaultLanes) lanes = default_lanes(stage, color_mode);
     VGR_REQUIRE(lanes == 1 || lanes == 2 || lanes == 4 || lanes == 8,
@@ -1395,13 +1233,14 @@ int foam_entry(const float* points, int64_t n_sites, const int32_t* offsets, con
     // 64-byte rows); the two-pass exact colours with 4 lanes per ray ran slower on them (268.9 against 258.3 ms on
     // config 3) and keep the attr rows, as the one-ray-per-lane kernels do. Site blocks also supply those kernels'
     // SH rows, 16 float4 apart after each 4-float4 record.
-    const bool rows_used = rows != nullptr && !indexed && stage == 2 && color_mode == kFused && lanes > 1;
+    const bool rows_used =
+        rows != nullptr && stage == 2 && (wide || (!indexed && color_mode == kFused && lanes > 1));
     const bool blocks = rows_used && row_floats == 64;
     const FoamScene S{reinterpret_cast<const float4*>(points),
                       offsets,
                       nbr,
-                      reinterpret_cast<const float4*>(indexed ? edge_i : edge),
-                      reinterpret_cast<const float4*>(indexed ? attr_i : attr),
+                      reinterpret_cast<const float4*>(indexed && !wide ? edge_i : edge),
+                      reinterpret_cast<const float4*>(indexed && !wide ? attr_i : attr),
                       !needs_sh ? nullptr
                       : blocks  ? reinterpret_cast<const float4*>(rows) + 4
                                 : reinterpret_cast<const float4*>(sh),
@@ -1421,6 +1260,7 @@ int foam_entry(const float* points, int64_t n_sites, const int32_t* offsets, con
     // (incoherent batches, bound by DRAM) the table's reads cost more than the per-lookup tags, which need only
     // 256 bytes of LDS per wave there: config 5's batch ran 2437.6 ms with the table, 2298.0 ms with the tags.
     const bool table = slots != nullptr && std::isinf(color_cut) && color_cut > 0 && lanes != 8;
+    if (wide) return launch_foam_wide(S, P, R, O, int(color_mode), sh_half != 0, s);
     if (indexed)
         return sh_half != 0 ? dispatch_indexed<true>(trace != nullptr, table, exact_blend, S, P, R, O, s)
                             : dispatch_indexed<false>(trace != nullptr, table, exact_blend, S, P, R, O, s);
