@@ -323,6 +323,21 @@ int vgr_grid_build(const float* points, int64_t n_sites, int32_t stride, const f
                    const int32_t* res, int32_t* cell_start, int32_t* cell_sites, int32_t* work, void* stream);
 
 /*
+ * vgr_grid_build that also writes the cell-ordered copy of vgr_grid_cell_points (cell_points f32 (N, 4), 16-byte
+ * aligned) in the same pass.
+ */
+int vgr_grid_build_points(const float* points, int64_t n_sites, int32_t stride, const float* lo, const float* cell,
+                          const int32_t* res, int32_t* cell_start, int32_t* cell_sites, float* cell_points,
+                          int32_t* work, void* stream);
+
+/*
+ * Bounding box of points f32 (n, stride), xyz first, n >= 1: box[0 .. 6) = (min xyz, max xyz), NaN where any coordinate
+ * of that axis is NaN. box: vgr_points_box_floats() floats on the device (the rest is scratch).
+ */
+int64_t vgr_points_box_floats(void);
+int vgr_points_box(const float* points, int64_t n, int32_t stride, float* box, void* stream);
+
+/*
  * Coherent processing order of a ray batch, for the `order` argument of vgr_foam_infer_lanes and
  * vgr_march_forward_lanes. No counterpart in the reference, which traces rays in the order given (config 5's
  * incoherent batch: origins uniform in a cube, directions uniform on the sphere). A permutation sorting the rays
@@ -433,6 +448,16 @@ int vgr_grid_cell_points(const float* points, int64_t n_sites, int32_t stride, c
 int vgr_grid_nearest_points(const float* cell_points, int64_t n_sites, const float* lo, const float* cell,
                             const int32_t* res, const int32_t* cell_start, const float* queries, int64_t n_queries,
                             const int32_t* order, int32_t* site, void* stream);
+
+/*
+ * vgr_grid_nearest_points for large batches: the queries are first binned into the same grid (a counting sort into work,
+ * with their positions), so that consecutive lanes scan the same cells and read their queries in order. The same answers.
+ * work: vgr_grid_binned_work_size(m, G) bytes, 16-byte aligned; m < 2^31.
+ */
+int64_t vgr_grid_binned_work_size(int64_t n_queries, int64_t n_cells);
+int vgr_grid_nearest_binned(const float* cell_points, int64_t n_sites, const float* lo, const float* cell,
+                            const int32_t* res, const int32_t* cell_start, const float* queries, int64_t n_queries,
+                            void* work, int64_t work_bytes, int32_t* site, void* stream);
 
 #ifdef __cplusplus
 }

@@ -109,3 +109,42 @@ def test_camera_and_ray_batch_starts_match_host(gpu):
 	centers = np.stack([c.eye for c in c3.cameras]).astype(np.float32)
 	np.testing.assert_array_equal(sites.nearest_sites(T(c3.points, gpu), T(centers, gpu)).cpu().numpy(),
 								  sites.nearest_sites(c3.points, centers))
+
+
+@pytest.mark.parametrize('m', [65537, 65600, 200003])
+@pytest.mark.parametrize('kind', ['spread', 'one point', 'outside', 'two cells'])
+def test_binned_batches_match_unbinned(gpu, m, kind):
+	"""Batches above 65,536 queries are binned into the grid's cells first (take_place shares a wave's atomics where its
+	lanes share a cell): the same answers as query by query, for spread queries, a batch from one camera, queries outside
+	the grid (all in its boundary cells), and two cells mixed."""
+	rng = np.random.default_rng(15)
+	pts = rng.uniform(-1, 1, (30000, 3)).astype(np.float32)
+	q = rng.uniform(-1.1, 1.1, (m, 3))
+	if kind == 'one point':
+		q[:] = [0.2, -0.4, 3.0]
+	elif kind == 'outside':
+		q[:, 0] += 7
+	elif kind == 'two cells':
+		q = np.array([[0.5, 0.5, 0.5], [-0.5, 0.25, 0.1]])[rng.integers(0, 2, m)] + rng.uniform(-0.01, 0.01, (m, 3))
+	q = q.astype(np.float32)
+	g = grid.SiteGrid(T(pts, gpu))
+	binned = g.nearest(T(q, gpu))
+	plain = torch.cat([g.nearest(T(q[a:a + 65536], gpu)) for a in range(0, m, 65536)])
+	assert torch.equal(binned, plain)
+	np.testing.assert_array_equal(binned.cpu().numpy()[:2000], dense.nearest_brute(pts, q[:2000]))
+
+
+@pytest.mark.parametrize('n', [1, 255, 256, 257, 131072, 131073, 300001])
+@pytest.mark.parametrize('stride', [3, 4])
+def test_points_box(gpu, n, stride):
+	"""The bounding box equals torch's min and max bit for bit, a NaN coordinate reaching its axis as it does there."""
+	from vgr import _lib
+	pts = torch.randn(n, stride, device=gpu)
+	for nan in (False, True):
+		if nan:
+			pts[n // 2, 1] = float('nan')
+		box = torch.empty(int(_lib.load().vgr_points_box_floats()), device=gpu)
+		_lib.call('vgr_points_box', _lib.ptr(pts), n, stride, _lib.ptr(box), _lib.stream_of(gpu))
+		want = torch.cat([pts[:, :3].amin(0), pts[:, :3].amax(0)])
+		assert torch.equal(torch.isnan(box[:6]), torch.isnan(want))
+		assert torch.equal(box[:6].nan_to_num(7.0), want.nan_to_num(7.0))

@@ -67,11 +67,16 @@ SIGNATURES = {
 	'vgr_grid_nearest': [_P, _I64, _I32, _P, _P, _P, _P, _P, _P, _I64, _P, _P],
 	'vgr_grid_cell_points': [_P, _I64, _I32, _P, _P, _P],
 	'vgr_grid_nearest_points': [_P, _I64, _P, _P, _P, _P, _P, _I64, _P, _P, _P],
+	'vgr_grid_build_points': [_P, _I64, _I32, _P, _P, _P, _P, _P, _P, _P, _P],
+	'vgr_points_box_floats': [],
+	'vgr_points_box': [_P, _I64, _I32, _P, _P],
+	'vgr_grid_binned_work_size': [_I64, _I64],
+	'vgr_grid_nearest_binned': [_P, _I64, _P, _P, _P, _P, _P, _I64, _P, _I64, _P, _P],
 	'vgr_abi_version': [],
 	'vgr_last_error': [],
 }
 
-ABI_VERSION = 27
+ABI_VERSION = 28
 _lib = None
 
 
@@ -97,6 +102,8 @@ def load():
 		lib.vgr_pack_work_size.restype = ctypes.c_int64
 		lib.vgr_morton_work_size.restype = ctypes.c_int64
 		lib.vgr_ray_order_work_size.restype = ctypes.c_int64
+		lib.vgr_points_box_floats.restype = ctypes.c_int64
+		lib.vgr_grid_binned_work_size.restype = ctypes.c_int64
 		if lib.vgr_abi_version() != ABI_VERSION:
 			raise RuntimeError(f'{LIB_PATH} has ABI {lib.vgr_abi_version()}, expected {ABI_VERSION}: rebuild it')
 		_lib = lib

@@ -1,5 +1,5 @@
 """Start-cell locator on the GPU: a uniform grid over the sites and exact nearest-site queries (libvgr's
-vgr_grid_build, vgr_grid_cell_points, vgr_grid_nearest_points).
+vgr_points_box, vgr_grid_build_points, vgr_grid_nearest_points, vgr_grid_nearest_binned).
 
 It replaces the host-side cKDTree query of the reference's nearest_sites (sites.py:38-39), which finds the start
 site of the traversal per camera centre (bench_infer.py:60, eval_scene.py:69) and per ray origin of a ray batch.
@@ -11,6 +11,10 @@ import math
 import torch
 
 from . import _lib
+
+
+# Batches above this many queries are binned before they are answered.
+BINNED_QUERIES = 65536
 
 
 class SiteGrid:
@@ -28,8 +32,10 @@ class SiteGrid:
 			raise RuntimeError('SiteGrid needs at least one site')
 		self.points, self.stride, self.n = points, points.shape[1], n
 		dev = points.device
-		lo = points[:, :3].amin(0).double().cpu()
-		hi = points[:, :3].amax(0).double().cpu()
+		lib = _lib.load()
+		box = torch.empty(int(lib.vgr_points_box_floats()), dtype=torch.float32, device=dev)
+		_lib.call('vgr_points_box', _lib.ptr(points), n, self.stride, _lib.ptr(box), _lib.stream_of(dev))
+		lo, hi = box[:6].cpu().double().view(2, 3)
 		ext = torch.clamp(hi - lo, min=1e-6)
 		lo = lo - 1e-6 * ext
 		ext = ext * (1 + 2e-6)
@@ -41,23 +47,21 @@ class SiteGrid:
 		self.cell = [float(e) / r for e, r in zip(ext, res)]
 		self.res = res
 		n_cells = res[0] * res[1] * res[2]
-		lib = _lib.load()
 		self.cell_start = torch.empty(n_cells + 1, dtype=torch.int32, device=dev)
 		self.cell_sites = torch.empty(n, dtype=torch.int32, device=dev)
 		work = torch.empty(int(lib.vgr_grid_work_size(n, n_cells)), dtype=torch.int32, device=dev)
 		self._geom = (_floats(self.lo), _floats(self.cell), _ints(self.res))
-		_lib.call('vgr_grid_build', _lib.ptr(points), n, self.stride, *self._geom, _lib.ptr(self.cell_start),
-				  _lib.ptr(self.cell_sites), _lib.ptr(work), _lib.stream_of(dev))
-		self._work = work  # released once the asynchronous build has run (caching allocator, same stream)
 		# the sites in cell order, (x, y, z, bits of the index) each, which the queries scan (a snapshot of points)
 		self.cell_points = torch.empty(n, 4, dtype=torch.float32, device=dev)
-		_lib.call('vgr_grid_cell_points', _lib.ptr(points), n, self.stride, _lib.ptr(self.cell_sites),
-				  _lib.ptr(self.cell_points), _lib.stream_of(dev))
+		_lib.call('vgr_grid_build_points', _lib.ptr(points), n, self.stride, *self._geom, _lib.ptr(self.cell_start),
+				  _lib.ptr(self.cell_sites), _lib.ptr(self.cell_points), _lib.ptr(work), _lib.stream_of(dev))
+		self._work = work  # released once the asynchronous build has run (caching allocator, same stream)
 
 	def nearest(self, queries, order=None):
 		"""Index (int32) of the nearest site of every query point: queries (m, 3) float32 CUDA tensor. order:
 		optional int32 (m,) permutation of 0 .. m - 1, the order in which the queries are answered (query_order
-		gives a coherent one); the answers do not depend on it."""
+		gives a coherent one); the answers do not depend on it. Without an order, batches above 65,536 queries are
+		binned into the grid's cells first and answered cell by cell."""
 		if not (isinstance(queries, torch.Tensor) and queries.is_cuda):
 			raise RuntimeError('queries must be a CUDA tensor')
 		if queries.dtype != torch.float32 or queries.dim() != 2 or queries.shape[1] != 3 or not queries.is_contiguous():
@@ -66,6 +70,13 @@ class SiteGrid:
 									  and order.shape == (len(queries),) and order.is_contiguous()):
 			raise RuntimeError('order must be a contiguous int32 CUDA tensor of one entry per query')
 		out = torch.empty(len(queries), dtype=torch.int32, device=queries.device)
+		if order is None and BINNED_QUERIES < len(queries) < 2 ** 31:
+			wb = int(_lib.load().vgr_grid_binned_work_size(len(queries), len(self.cell_start) - 1))
+			work = torch.empty(wb, dtype=torch.uint8, device=queries.device)
+			_lib.call('vgr_grid_nearest_binned', _lib.ptr(self.cell_points), self.n, *self._geom,
+					  _lib.ptr(self.cell_start), _lib.ptr(queries), len(queries), _lib.ptr(work), wb, _lib.ptr(out),
+					  _lib.stream_of(queries.device))
+			return out
 		_lib.call('vgr_grid_nearest_points', _lib.ptr(self.cell_points), self.n, *self._geom, _lib.ptr(self.cell_start),
 				  _lib.ptr(queries), len(queries), _lib.ptr(order), _lib.ptr(out), _lib.stream_of(queries.device))
 		return out
