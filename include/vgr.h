@@ -288,6 +288,29 @@ int vgr_conic_backward(const float* log_scale, const float* quat, int64_t n, dou
 int64_t vgr_pack_work_size(int64_t n_sites);
 
 /*
+ * vgr_pack_foam with the derived records of vgr_foam_index_pack and vgr_foam_slot_table and the site rows of
+ * vgr_foam_infer_indexed written by the same passes: edge_i f32 (M + N, 4), attr_i f32 (N, 20), slots i32 (N, 16), rows
+ * f32 (N, row_floats), row_floats 16 or 64 (with the fp32 SH row), slots and rows 16-byte aligned. The SH rows come from
+ * sh f32 (N, 16, 3), or, when sh is NULL, from sh_dc f32 (N, 3) and sh_rest f32 (N, 15, 3). work as for vgr_pack_foam.
+ */
+int vgr_pack_foam_indexed(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t* adj,
+                          int64_t n_adj, const float* raw, const float* d_log_scale, const float* c_log_scale,
+                          const float* dA, const float* cA, const float* sh, const float* sh_dc, const float* sh_rest,
+                          const int32_t* perm, double scale_floor, double eps_density, float* points4,
+                          int32_t* offsets_sf, int32_t* nbr, float* edge, float* attr, float* sh32, void* sh16,
+                          float* edge_i, float* attr_i, int32_t* slots, float* rows, int64_t row_floats, void* work,
+                          int64_t work_bytes, void* stream);
+
+/*
+ * The renumbering of morton_order() (render.py:168-176): the stable sort of the points' Z-order keys (vgr_morton_codes,
+ * bits <= 10) -> perm32 i32 (n) and perm i64 (n), new -> old, and its inverse inv i64 (n) (NULL = none).
+ * work: vgr_morton_order_work_size(n) bytes, 256-byte aligned.
+ */
+int64_t vgr_morton_order_work_size(int64_t n);
+int vgr_morton_order(const float* points, int64_t n, int32_t bits, int32_t* perm32, int64_t* perm, int64_t* inv,
+                     void* work, int64_t work_bytes, void* stream);
+
+/*
  * Z-order keys of points f32 (n, 3) over their bounding box, bits per axis (<= 21): the keys morton_order()
  * (render.py:168-176) sorts to renumber the sites, with its arithmetic (q = trunc((p - lo) / max(hi - lo, 1e-12) *
  * (2^bits - 1)), bit b of axis a at bit 3 b + a) -> code i64 (n). work: vgr_morton_work_size(n) bytes.

@@ -133,3 +133,35 @@ def test_native_pack_errors(gpu):
 					  torch.zeros(4, 6, device=gpu), torch.zeros(4, 6, device=gpu), torch.zeros(4, 16, 3, device=gpu),
 					  eps_density=-1.0)
 	assert np.isfinite(0.0)
+
+
+@pytest.mark.parametrize('n', [20, 63, 64, 65, 255, 257, 3000])
+@pytest.mark.parametrize('sh_half', [False, True])
+def test_derived_records_of_the_pack_match_their_own_kernels(gpu, n, sh_half):
+	"""pack_foam(index=True), whose passes write the derived records too (edge_i, attr_i, slot table, site rows, SH rows
+	read from the field's two parameters), bit for bit against pack_foam(index=False) followed by index_pack, at the edges
+	of its waves and blocks; and the renumbering against a stable sort of the keys."""
+	from helpers import Field
+	from vgr.model import VoronoiGaussField
+	f = Field(seed=n, n=n)
+	T = lambda a: torch.as_tensor(a, device=gpu)  # noqa: E731
+	m = VoronoiGaussField(T(f.points), T(f.offsets), T(f.adj), torch.zeros(f.n, 3, device=gpu),
+						  torch.ones(f.n, device=gpu))
+	with torch.no_grad():
+		for name, v in (('raw', f.raw), ('d_log_scale', f.d_log_scale), ('d_quat', f.d_quat),
+						('c_log_scale', f.c_log_scale), ('c_quat', f.c_quat), ('sh_dc', f.sh[:, :1]),
+						('sh_rest', f.sh[:, 1:])):
+			getattr(m, name).copy_(T(np.ascontiguousarray(v)))
+	for reorder in (False, True):
+		a = render.pack_foam(m, eps_density=1e-3, sh_half=sh_half, reorder=reorder)
+		b = render.index_pack(render.pack_foam(m, eps_density=1e-3, sh_half=sh_half, reorder=reorder, index=False))
+		assert set(a) == set(b)
+		for k, v in b.items():
+			if not isinstance(v, torch.Tensor):
+				assert a[k] is None and v is None, k
+				continue
+			assert a[k].dtype == v.dtype and a[k].shape == v.shape and a[k].is_contiguous(), k
+			assert torch.equal(a[k].view(torch.uint8), v.view(torch.uint8)), k
+		if reorder:
+			assert torch.equal(a['perm'], torch.sort(render.morton_codes(m.graph.points), stable=True)[1])
+			assert torch.equal(a['inv'][a['perm']], torch.arange(f.n, device=gpu))

@@ -69,7 +69,7 @@ __global__ void __launch_bounds__(kBlock) grid_count(const float* __restrict__ p
 
 // Scatter: point i goes to slot start[its cell] + its place: its index to cell_sites and (x, y, z, bits of i) to cp,
 // either of which may be null. The cell is computed again from the position (12 bytes) rather than kept (4 written, 4
-// read); with the place known the scatter needs no second round of atomics: 1M sites 125 -> 75 us for both passes.
+// read); with the place known the scatter needs no second round of atomics: 1M sites 125 -> 76 us for both passes.
 __global__ void __launch_bounds__(kBlock)
     grid_fill(const float* __restrict__ pts, int stride, int64_t n, Geom g, const int* __restrict__ start,
               const int* __restrict__ place, int* __restrict__ cell_sites, float4* __restrict__ cp) {
@@ -279,7 +279,7 @@ namespace {
 
 // Bounding box of n points of `stride` floats, (min xyz, max xyz), NaN where a coordinate is NaN on that axis: kBoxBlocks
 // blocks sweep the points, then one block reduces their boxes. (torch's amin and amax over the rows of an (N, 3) tensor
-// take 0.76 ms for 1M points; this reads them once, 8 us.)
+// take 0.76 ms for 1M points, this 12 us.)
 constexpr int kBoxBlocks = 512;
 
 __device__ __forceinline__ float nan_min(float a, float b) { return b < a || b != b ? b : a; }

@@ -447,35 +447,70 @@ def traverse_faces(points, offsets, nbr, edge, o, d, start, near, far, cap=None,
 
 
 def pack_foam(points, offsets, adj, raw, d_log_scale, c_log_scale, dA, cA, sh, perm=None, scale_floor=0.0,
-			  eps_density=0.0, sh_half=False):
+			  eps_density=0.0, sh_half=False, index=False):
 	"""The inference records on the GPU (vgr_pack_foam, render.py:179-225) from the model's device tensors and the
-	conics; perm (N,) new -> old renumbers the sites (None: none). -> points (N, 4), offsets (N + 1), nbr (E),
-	edge (E, 4), attr (N, 20), sh32 (N, 16, 3) fp32, sh16 (N, 16, 3) fp16 or None, all in the new numbering."""
+	conics; perm (N,) new -> old renumbers the sites (None: none). sh: the (N, 16, 3) rows, or the pair of their parts
+	(sh_dc (N, 1, 3), sh_rest (N, 15, 3)). -> points (N, 4), offsets (N + 1), nbr (E), edge (E, 4), attr (N, 20),
+	sh32 (N, 16, 3) fp32, sh16 (N, 16, 3) fp16 or None, all in the new numbering. index: also the records of index_pack,
+	slot_table and the site rows, written by the same kernels (vgr_pack_foam_indexed): edge_i, attr_i, slots and rows
+	((N, 64) site blocks, (N, 16) with sh_half)."""
 	for t, n, dt in ((points, 'points', torch.float32), (offsets, 'offsets', torch.int32), (adj, 'adj', torch.int32),
 					 (raw, 'raw', torch.float32), (d_log_scale, 'd_log_scale', torch.float32),
-					 (c_log_scale, 'c_log_scale', torch.float32), (dA, 'dA', torch.float32), (cA, 'cA', torch.float32),
-					 (sh, 'sh', torch.float32)):
+					 (c_log_scale, 'c_log_scale', torch.float32), (dA, 'dA', torch.float32), (cA, 'cA', torch.float32)):
 		_check(t, n, dt)
 	n, m = points.size(0), adj.numel()
-	_require(sh.dim() == 3 and sh.size(0) == n and sh.size(1) == 16 and sh.size(2) == 3, 'sh must be (N, 16, 3)')
+	dc, rest = (None, None) if isinstance(sh, torch.Tensor) else sh
+	if dc is None:
+		_check(sh, 'sh', torch.float32)
+		_require(sh.dim() == 3 and sh.size(0) == n and sh.size(1) == 16 and sh.size(2) == 3, 'sh must be (N, 16, 3)')
+	else:
+		_check(dc, 'sh_dc', torch.float32)
+		_check(rest, 'sh_rest', torch.float32)
+		_require(dc.shape == (n, 1, 3) and rest.shape == (n, 15, 3), 'sh_dc must be (N, 1, 3) and sh_rest (N, 15, 3)')
+		sh = None
 	dev = points.device
 	p32 = None
 	if perm is not None:
 		p32 = perm.to(torch.int32).contiguous()
 		_check(p32, 'perm', torch.int32)
 	f = dict(dtype=torch.float32, device=dev)
-	out = {'points': torch.empty(n, 4, **f), 'offsets': torch.empty(n + 1, dtype=torch.int32, device=dev),
-		   'nbr': torch.empty(m + n, dtype=torch.int32, device=dev), 'edge': torch.empty(m + n, 4, **f),
-		   'attr': torch.empty(n, 20, **f), 'sh32': torch.empty(n, 16, 3, **f),
+	i = dict(dtype=torch.int32, device=dev)
+	out = {'points': torch.empty(n, 4, **f), 'offsets': torch.empty(n + 1, **i), 'nbr': torch.empty(m + n, **i),
+		   'edge': torch.empty(m + n, 4, **f), 'attr': torch.empty(n, 20, **f), 'sh32': torch.empty(n, 16, 3, **f),
 		   'sh16': torch.empty(n, 16, 3, dtype=torch.float16, device=dev) if sh_half else None}
 	wb = int(_lib.load().vgr_pack_work_size(n))
 	work = torch.empty(wb, dtype=torch.uint8, device=dev)
+	field = [ptr(points), n, ptr(offsets), ptr(adj), m, ptr(raw), ptr(d_log_scale), ptr(c_log_scale), ptr(dA), ptr(cA)]
+	records = [ptr(out[k]) for k in ('points', 'offsets', 'nbr', 'edge', 'attr', 'sh32', 'sh16')]
+	floor_eps = (float(scale_floor), float(eps_density))
 	with torch.cuda.device(dev):
-		call('vgr_pack_foam', ptr(points), n, ptr(offsets), ptr(adj), m, ptr(raw), ptr(d_log_scale), ptr(c_log_scale),
-			 ptr(dA), ptr(cA), ptr(sh), ptr(p32), float(scale_floor), float(eps_density), ptr(out['points']),
-			 ptr(out['offsets']), ptr(out['nbr']), ptr(out['edge']), ptr(out['attr']), ptr(out['sh32']),
-			 ptr(out['sh16']), ptr(work), wb, stream_of(dev))
+		if index or dc is not None:
+			out.update(edge_i=torch.empty(m + n, 4, **f), attr_i=torch.empty(n, 20, **f), slots=torch.empty(n, 16, **i),
+					   rows=torch.empty(n, 16 if sh_half else 64, **f))
+			call('vgr_pack_foam_indexed', *field, ptr(sh), ptr(dc), ptr(rest), ptr(p32), *floor_eps, *records,
+				 *[ptr(out[k]) for k in ('edge_i', 'attr_i', 'slots', 'rows')], out['rows'].size(1), ptr(work), wb,
+				 stream_of(dev))
+		else:
+			call('vgr_pack_foam', *field, ptr(sh), ptr(p32), *floor_eps, *records, ptr(work), wb, stream_of(dev))
 	return out
+
+
+def morton_order(points, bits=10):
+	"""The stable Z-order renumbering of points (N, 3) (vgr_morton_order, bits <= 10, render.py:168-176) -> perm (N,)
+	int64 new -> old, inv (N,) int64, perm32 (N,) int32."""
+	_check(points, 'points', torch.float32)
+	n, dev = points.size(0), points.device
+	_require(points.dim() == 2 and points.size(1) == 3, 'points must be (N, 3)')
+	perm32 = torch.empty(n, dtype=torch.int32, device=dev)
+	perm, inv = torch.empty(n, dtype=torch.int64, device=dev), torch.empty(n, dtype=torch.int64, device=dev)
+	if n == 0:
+		return perm, inv, perm32
+	wb = int(_lib.load().vgr_morton_order_work_size(n))
+	work = torch.empty(wb, dtype=torch.uint8, device=dev)
+	with torch.cuda.device(dev):
+		call('vgr_morton_order', ptr(points), n, int(bits), ptr(perm32), ptr(perm), ptr(inv), ptr(work), wb,
+			 stream_of(dev))
+	return perm, inv, perm32
 
 
 def morton_codes(points, bits=10):

@@ -11,6 +11,7 @@ import torch
 import torch.nn.functional as F
 
 from . import ext
+from .model import VoronoiGaussField
 
 # ---------------------------------------------------------------------------------------------------- ray bounds
 
@@ -302,19 +303,24 @@ def pack_foam(model, scale_floor=0.0, eps_density=0.0, sh_half=False, reorder=Fa
 	g = model.graph
 	dA = ext.conic(model.d_log_scale, model.d_quat, scale_floor)
 	cA = ext.conic(model.c_log_scale, model.c_quat, scale_floor)
-	perm = inv = None
+	perm = inv = orig = None
 	if reorder:
-		perm = morton_order(g.points)
-		inv = torch.empty_like(perm)
-		inv[perm] = torch.arange(len(perm), device=perm.device)
+		perm, inv, orig = ext.morton_order(g.points)
+	# a field's SH rows are read from its two parameters, without the copy that joins them
+	parts = isinstance(model, VoronoiGaussField) and type(model).sh is VoronoiGaussField.sh and index
+	sh = (model.sh_dc.detach().contiguous(), model.sh_rest.detach().contiguous()) if parts else \
+		model.sh().detach().float().contiguous()
+	if parts and any(t.dtype != torch.float32 for t in sh):
+		sh = model.sh().detach().float().contiguous()
 	out = ext.pack_foam(g.points, g.offsets, g.adj, *[t.detach().contiguous() for t in (
-		model.raw, model.d_log_scale, model.c_log_scale, dA, cA)], model.sh().detach().float().contiguous(), perm,
-		scale_floor, eps_density, sh_half)
-	empty = torch.empty(0, device=g.points.device)
+		model.raw, model.d_log_scale, model.c_log_scale, dA, cA)], sh, orig, scale_floor, eps_density, sh_half, index)
+	empty = torch.empty(0, dtype=torch.int32, device=g.points.device)
 	pack = {'points': out['points'], 'offsets': out['offsets'], 'nbr': out['nbr'], 'edge': out['edge'],
 			'attr': out['attr'], 'sh': out['sh16'] if sh_half else out['sh32'], 'sh32': out['sh32'], 'perm': perm,
-			'inv': inv, 'orig': (empty if perm is None else perm).int().contiguous(), 'baked_center': None}
-	return index_pack(pack) if index else pack
+			'inv': inv, 'orig': empty if orig is None else orig, 'baked_center': None}
+	if index:
+		pack.update({k: out[k] for k in ('edge_i', 'attr_i', 'slots', 'rows')})
+	return pack
 
 
 @torch.no_grad()
