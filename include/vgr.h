@@ -165,6 +165,29 @@ int vgr_march_backward(const float* points, int64_t n_sites, const int32_t* offs
                        int64_t blocks_ready, void* work, int64_t work_bytes, void* stream);
 
 /*
+ * The march of a training step with 16 lanes per ray (vgr_march_forward_lanes) that leaves visit records for its backward:
+ * visits f32 (B, visit_cap, 8), per run of at most 32 samples in one cell (cell bits, index of its first sample bits,
+ * transmittance and composited rgb before it, unused x 2), and n_visits i32 (B), the runs of each ray (0: not traced, more
+ * than visit_cap: its records are incomplete). vgr_march_backward_visits replays the runs independently of each other, rays
+ * with incomplete records as vgr_march_backward does, and takes the forward's stats; n_rays <= 2^22.
+ */
+int vgr_march_forward_visits(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t* adj,
+                             int64_t n_adj, const float* raw, const float* dA, const float* cA, const float* sh,
+                             int64_t sh_deg, const float* o, const float* d, const int32_t* start, const float*
+                             near_t, const float* mid_t, const float* far_t, int64_t n_rays, double dt, int64_t
+                             n_bg, double t_thresh, double w_thresh, float* rgb, float* T, float* depth, int32_t*
+                             stats, void* work, int64_t work_bytes, float* visits, int64_t visit_cap, int32_t*
+                             n_visits, void* stream);
+int vgr_march_backward_visits(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t* adj,
+                              int64_t n_adj, const float* raw, const float* dA, const float* cA, const float* sh,
+                              int64_t sh_deg, const float* o, const float* d, const int32_t* start, const float*
+                              near_t, const float* mid_t, const float* far_t, int64_t n_rays, double dt, int64_t
+                              n_bg, double t_thresh, double w_thresh, const float* rgb, const float* T, const float*
+                              g_rgb, const float* g_T, float* g_raw, float* g_dA, float* g_cA, float* g_sh, int64_t
+                              blocks_ready, void* work, int64_t work_bytes, const float* visits, int64_t visit_cap,
+                              const int32_t* n_visits, const int32_t* stats, void* stream);
+
+/*
  * The training renderer: rendering at the ray's crossings of the Voronoi faces with a record of every sample, and
  * its backward. Replaces foam_forward() / foam_backward() of csrc/foam.cu:471-531 (kernels :345-469, exports
  * :533-536), bound by ext.foam (ext.py:185-216), the renderer train.py uses by default (render_rays_foam).
@@ -192,6 +215,21 @@ int vgr_foam_backward(const float* points, int64_t n_sites, const int32_t* offse
                       const float* T, const float* g_rgb, const float* g_T, const float* rec, int64_t record_cap,
                       const int32_t* stats, float* g_raw, float* g_dA, float* g_cA, float* g_sh,
                       int64_t blocks_ready, void* work, int64_t work_bytes, void* stream);
+
+/*
+ * vgr_foam_backward with scratch for recorded rays (NULL = none): their samples' gradients are first computed ray by ray
+ * from the records, then scattered sample by sample, so that a training batch fills the GPU; the same sums in another order.
+ * scratch: vgr_foam_scratch_size(B, record_cap) bytes, 16-byte aligned, as rec must then be.
+ */
+int64_t vgr_foam_scratch_size(int64_t n_rays, int64_t record_cap);
+int vgr_foam_backward_scratch(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t* adj,
+                              int64_t n_adj, const float* raw, const float* dA, const float* cA, const float* sh,
+                              int64_t sh_deg, const float* o, const float* d, const int32_t* start,
+                              const float* near_t, const float* far_t, int64_t n_rays, double t_thresh,
+                              double w_thresh, const float* rgb, const float* T, const float* g_rgb, const float* g_T,
+                              const float* rec, int64_t record_cap, const int32_t* stats, float* g_raw, float* g_dA,
+                              float* g_cA, float* g_sh, int64_t blocks_ready, void* work, int64_t work_bytes,
+                              void* scratch, int64_t scratch_bytes, void* stream);
 
 /*
  * Nearest site of every sorted ray sample o + z d by a greedy walk (strict <). Replaces walk() of

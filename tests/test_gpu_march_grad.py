@@ -116,3 +116,35 @@ def test_march_backward_edge_cases(gpu):
 		fx.march_backward(*field, 4, *rt, DT, NBG, 1e-4, 1e-4, rgb, Tt, ones3, ones)
 	with pytest.raises(RuntimeError, match='g_rgb'):
 		fx.march_backward(*field, 3, *rt, DT, NBG, 1e-4, 1e-4, rgb, Tt, ones3[:3], ones)
+
+
+@pytest.mark.parametrize('n_rays', [1, 3, 65, 130])
+@pytest.mark.parametrize('cap', [1, 24, 256])
+@pytest.mark.parametrize('dt', [1 / 16, 1 / 256])
+def test_backward_of_recorded_visits(gpu, n_rays, cap, dt):
+	"""The backward from the forward's visit records (runs of up to 32 samples in a cell, replayed on their own) against the
+	backward that marches every ray again: records that all fit, some and none, steps longer than a cell and many steps per
+	cell. The samples replay with the forward's bits and the sums run in another order: 1e-5. The forward's outputs do not
+	depend on the records."""
+	f = Field(seed=9, n=300)
+	o, d, start, near, mid, far = f.rays(B=n_rays, seed=9)
+	start = start.copy()
+	start[:1] = f.n if n_rays > 1 else start[:1]  # a ray that is not traced
+	dA, cA = f.conics(0.01)
+	t = lambda a: torch.as_tensor(np.ascontiguousarray(a), device=gpu)  # noqa: E731
+	args = [t(a) for a in (f.points, f.offsets, f.adj, f.raw, dA, cA, f.sh)] + [3] + \
+		[t(a) for a in (o, d, start, near, mid, far)] + [dt, 16, 1e-4, 1e-4]
+	fx = ext.march_extension()
+	visits = (torch.full((n_rays, cap, 8), float('nan'), device=gpu), torch.full((n_rays,), -1, dtype=torch.int32,
+																				 device=gpu))
+	outs = fx.march_forward(*args, lanes=16, visits=visits)
+	plain = fx.march_forward(*args, lanes=16)
+	for a, b in zip(outs, plain):
+		assert torch.equal(a, b)
+	assert (visits[1] >= 0).all()
+	g = torch.Generator(device=gpu).manual_seed(2)
+	up = torch.randn(n_rays, 3, device=gpu, generator=g), torch.randn(n_rays, device=gpu, generator=g)
+	got = fx.march_backward(*args, outs[0], outs[1], *up, lanes=16, visits=visits, stats=outs[3])
+	want = fx.march_backward(*args, outs[0], outs[1], *up, lanes=16)
+	for a, b in zip(got, want):
+		assert torch.isfinite(a).all() and (a.double() - b.double()).norm() <= 1e-5 * b.double().norm() + 1e-30

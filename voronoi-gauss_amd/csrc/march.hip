@@ -607,6 +607,40 @@ __device__ void grad_pass_wave(const MarchField& F, const MarchGradOut& G, int i
     }
 }
 
+// add_rows by a whole wave: lane t adds float t of every row, from two LDS words whose places it knows beforehand
+// (slot[t] alone below 13, b_j times dc_c from 16 on), two rows at a time so that one row's LDS reads cover the other's.
+struct RowLane {
+    int a, b;  // words of the slot: value = slot[a] * (b >= 0 ? slot[b] : 1)
+    bool on;
+};
+
+__device__ __forceinline__ RowLane row_lane(int nb) {
+    const int t = threadIdx.x & 63;
+    if (t < 13) return {t, -1, true};
+    const int q = t - kGradSh;
+    return {16 + max(q, 0) / 3, 13 + max(q, 0) % 3, q >= 0 && q / 3 < nb};
+}
+
+__device__ __forceinline__ void add_rows_wave(const MarchGradOut& G, const float* __restrict__ slots, uint64_t rows,
+                                              int k, const RowLane& R) {
+    const int t = threadIdx.x & 63;
+    while (rows != 0) {
+        const int L0 = __builtin_amdgcn_readfirstlane(__ffsll(static_cast<unsigned long long>(rows)) - 1);
+        rows &= rows - 1;
+        const bool two = rows != 0;
+        const int L1 = two ? __builtin_amdgcn_readfirstlane(__ffsll(static_cast<unsigned long long>(rows)) - 1) : L0;
+        rows &= rows - 1;
+        const float* s0 = slots + kSlot * L0;
+        const float* s1 = slots + kSlot * L1;
+        const float a0 = s0[R.a], a1 = s1[R.a];
+        const float b0 = R.b >= 0 ? s0[R.b] : 1.f, b1 = R.b >= 0 ? s1[R.b] : 1.f;
+        const int64_t k0 = __builtin_amdgcn_readlane(k, L0), k1 = __builtin_amdgcn_readlane(k, L1);
+        const float v0 = a0 * b0, v1 = a1 * b1;
+        if (R.on && v0 != 0.f) unsafeAtomicAdd(G.block + kGradBlock * k0 + t, v0);
+        if (two && R.on && v1 != 0.f) unsafeAtomicAdd(G.block + kGradBlock * k1 + t, v1);
+    }
+}
+
 // Colour blend of the coloured samples of a pass (flush's sums): A_s and the unnormalised channel sums.
 template <int NV>
 __device__ void blend_sums(const MarchField& F, int i, const float (&o)[3], const float (&d)[3], const float (&b)[16],
@@ -804,18 +838,21 @@ __device__ __forceinline__ void group_round(const MarchField& F, int i, const fl
 }
 
 // The neighbourhood of the group's current cell, as the lanes hold it: lane g's slots are neighbours g and g + 16
-// (k = -1 past the end) with their unclamped colours 1/2 + SH_k(d) . b, which depend only on the site and the ray,
-// evaluated once per cell visit at its first coloured sample. Neighbours beyond the two slots (cells of more than 32
-// neighbours) are read directly at every sample.
+// (k = -1 past the end) with their records, read once per cell visit (a march takes about ten samples per cell, so most
+// rounds then read no memory), and their unclamped colours 1/2 + SH_k(d) . b, which depend only on the site and the ray,
+// evaluated once per visit at its first coloured sample. Neighbours beyond the two slots (cells of more than 32 neighbours)
+// are read directly at every sample.
 constexpr int kSlots = 2;
 
 struct GroupCell {
     int cell, e0, n;
     int k[kSlots];
+    SiteRec rc[kSlots];
     float c[kSlots][3];
     bool col_ok;
 };
 
+template <int BLK>
 __device__ __forceinline__ void enter_cell(const MarchField& F, int cell, int g, GroupCell& C) {
     C.cell = cell, C.e0 = F.offsets[cell], C.n = F.offsets[cell + 1] - C.e0 + 1, C.col_ok = false;
 #pragma unroll
@@ -823,6 +860,9 @@ __device__ __forceinline__ void enter_cell(const MarchField& F, int cell, int g,
         const int e = g + kGroup * s;
         C.k[s] = e < C.n ? neighbor(F, cell, C.e0, e) : -1;
     }
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s)
+        if (C.k[s] >= 0) C.rc[s] = site_rec<BLK>(F, C.k[s]);
 }
 
 template <int NV>
@@ -845,11 +885,9 @@ __device__ __forceinline__ void group_colour(const MarchField& F, GroupCell& Cc,
 #pragma unroll
     for (int s = 0; s < kSlots; ++s) {
         if (Cc.k[s] >= 0) {
-            const float4* r = F.rec + block_vec4(NV) * static_cast<int64_t>(Cc.k[s]);
-            const float4 p = r[0], c0 = r[2], c1 = r[3];
             float v[3];
-            offset_to(p, x, v);
-            const float a = fexp(-0.5f * (color_m(c0, c1, v) - mmin));
+            offset_to(Cc.rc[s].q0, x, v);
+            const float a = fexp(-0.5f * (color_m(Cc.rc[s].q2, Cc.rc[s].q3, v) - mmin));
             A += a;
 #pragma unroll
             for (int ch = 0; ch < 3; ++ch) cs[ch] += a * fmaxf(Cc.c[s][ch], 0.f);
@@ -877,7 +915,7 @@ __device__ __forceinline__ void group_colour(const MarchField& F, GroupCell& Cc,
 // same order, same butterflies), and resolves the leading samples at which the site wins (march_ray's batching in
 // the group layout). The coloured samples among them are blended by one colour round. Same bits as one sample per
 // round; up to kGroupBatch times fewer rounds.
-constexpr int kGroupBatch = 4;
+constexpr int kGroupBatch = 3;
 
 struct GroupRoundN {
     float sigma[kGroupBatch], mmin[kGroupBatch];
@@ -885,16 +923,14 @@ struct GroupRoundN {
 };
 
 template <int BLK>
-__device__ __forceinline__ void group_round_n(const MarchField& F, int i, const float (&o)[3], const float (&d)[3],
-                                              const float (&t)[kGroupBatch], int g, GroupRoundN& Q) {
-    const int e0 = F.offsets[i], n = F.offsets[i + 1] - e0 + 1;
+__device__ __forceinline__ void group_round_n(const MarchField& F, const GroupCell& C, const float (&o)[3],
+                                              const float (&d)[3], const float (&t)[kGroupBatch], int g,
+                                              GroupRoundN& Q) {
     float bd[kGroupBatch], s[kGroupBatch], mm[kGroupBatch];
     int bk[kGroupBatch];
 #pragma unroll
     for (int j = 0; j < kGroupBatch; ++j) bd[j] = kInf, s[j] = 0.f, mm[j] = kInf, bk[j] = INT_MAX;
-    for (int e = g; e < n; e += kGroup) {
-        const int k = neighbor(F, i, e0, e);
-        const SiteRec rc = site_rec<BLK>(F, k);
+    const auto visit = [&](int k, const SiteRec& rc) {
 #pragma unroll
         for (int j = 0; j < kGroupBatch; ++j) {
             float x[3], v[3];
@@ -905,6 +941,13 @@ __device__ __forceinline__ void group_round_n(const MarchField& F, int i, const 
             s[j] += fexp(rc.q0.w - 0.5f * density_m(rc, v));
             mm[j] = fminf(mm[j], color_m(rc.q2, rc.q3, v));
         }
+    };
+#pragma unroll
+    for (int u = 0; u < kSlots; ++u)
+        if (C.k[u] >= 0) visit(C.k[u], C.rc[u]);
+    for (int e = g + kGroup * kSlots; e < C.n; e += kGroup) {
+        const int k = neighbor(F, C.cell, C.e0, e);
+        visit(k, site_rec<BLK>(F, k));
     }
 #pragma unroll
     for (int j = 0; j < kGroupBatch; ++j) {
@@ -926,15 +969,13 @@ __device__ __forceinline__ void group_colour_n(const MarchField& F, GroupCell& C
 #pragma unroll
     for (int s = 0; s < kSlots; ++s) {
         if (Cc.k[s] >= 0) {
-            const float4* r = F.rec + block_vec4(NV) * static_cast<int64_t>(Cc.k[s]);
-            const float4 p = r[0], c0 = r[2], c1 = r[3];
 #pragma unroll
             for (int j = 0; j < kGroupBatch; ++j) {
                 if ((mask >> j) & 1u) {
                     float x[3], v[3];
                     point_at(o, d, t[j], x);
-                    offset_to(p, x, v);
-                    const float a = fexp(-0.5f * (color_m(c0, c1, v) - mmin[j]));
+                    offset_to(Cc.rc[s].q0, x, v);
+                    const float a = fexp(-0.5f * (color_m(Cc.rc[s].q2, Cc.rc[s].q3, v) - mmin[j]));
                     A[j] += a;
 #pragma unroll
                     for (int ch = 0; ch < 3; ++ch) cs[j][ch] += a * fmaxf(Cc.c[s][ch], 0.f);
@@ -971,10 +1012,26 @@ __device__ __forceinline__ void group_colour_n(const MarchField& F, GroupCell& C
     }
 }
 
+// The visits a forward leaves for its backward: per ray up to `cap` records of 8 floats, one per run of at most
+// kVisitSamples samples in one cell: the cell and the index of its first sample (bits), the transmittance and the colour
+// composited before it. n: the records of each ray (more than cap: the ray's records are incomplete).
+constexpr int kVisitSamples = 32;
+constexpr int kVisitFloats = 8;
+struct MarchVisits {
+    float* __restrict__ rec;  // (B, cap, 8) or null
+    int* __restrict__ n;      // (B)
+    int cap;
+};
+
+// Waves per SIMD: with the cell's records in registers, 3 samples per round fit three waves. 160,000 camera rays / a training
+// step of 4,096 (forward and backward): 3 samples and 3 waves 28.3 / 4.29 ms, 4 and 2 36.3 / 4.18, 4 and 3 31.4 / 4.30, 2 and
+// 4 31.1 / 4.65, 4 and 4 59.0 / 5.44 (spills); reading the records every round, 4 samples, 31.0 / 4.4.
+constexpr int kGroupWaves = 3;
+
 // Per ray: the sample loop of march_ray, kGroupBatch samples per round.
 template <int NV, bool TRACE>
 __device__ void march_ray_group(const MarchField& F, const MarchParams& M, const MarchRays& R, const MarchOut& O,
-                                int64_t r, int cur, int g) {
+                                const MarchVisits& V, int64_t r, int cur, int g) {
     const float o[3] = {R.o[3 * r], R.o[3 * r + 1], R.o[3 * r + 2]};
     const float d[3] = {R.d[3 * r], R.d[3 * r + 1], R.d[3 * r + 2]};
     const float near = R.t_near[r], mid = R.t_mid[r], far = R.t_far[r];
@@ -987,14 +1044,17 @@ __device__ void march_ray_group(const MarchField& F, const MarchParams& M, const
     float T = 1.f, acc[3] = {0.f, 0.f, 0.f}, dep = 0.f;
     GroupCell Cc;
     Cc.cell = -1;
+    int n_visits = 0, visit_cell = -1, visit_k = 0;
     bool live = true;
     for (int k = 0; live && k < n_total;) {
+        if (Cc.cell != cur) enter_cell<block_vec4(NV)>(F, cur, g, Cc);
         float t[kGroupBatch], delta[kGroupBatch], w[kGroupBatch];
 #pragma unroll
         for (int j = 0; j < kGroupBatch; ++j)
             sample_at(near, mid, far, n_in, M, min(k + j, n_total - 1), t[j], delta[j]);
         GroupRoundN Q;
-        group_round_n<block_vec4(NV)>(F, cur, o, d, t, g, Q);
+        group_round_n<block_vec4(NV)>(F, Cc, o, d, t, g, Q);
+        const float T_before = T;
         int nres = 0, next = cur;
         unsigned coloured = 0u;
         bool run = true;
@@ -1015,8 +1075,19 @@ __device__ void march_ray_group(const MarchField& F, const MarchParams& M, const
                 next = Q.k[j], run = false;
             }
         }
+        if (V.rec != nullptr && nres > 0 && (visit_cell != cur || k - visit_k >= kVisitSamples)) {
+            if (n_visits < V.cap && g < kVisitFloats) {
+                const float v = g == 0 ? __int_as_float(cur)
+                              : g == 1 ? __int_as_float(k)
+                              : g == 2 ? T_before
+                              : g == 3 ? acc[0]
+                              : g == 4 ? acc[1]
+                                       : acc[2];
+                V.rec[(r * V.cap + n_visits) * kVisitFloats + g] = v;
+            }
+            visit_cell = cur, visit_k = k, ++n_visits;
+        }
         if (coloured) {
-            if (Cc.cell != cur) enter_cell(F, cur, g, Cc);
             float C[kGroupBatch][3], inv[kGroupBatch];
             group_colour_n<NV>(F, Cc, o, d, t, Q.mmin, coloured, b, nb, g, C, inv);
 #pragma unroll
@@ -1038,11 +1109,13 @@ __device__ void march_ray_group(const MarchField& F, const MarchParams& M, const
         O.T[r] = T;
         O.depth[r] = dep;
         O.stats[3 * r] = n_samples, O.stats[3 * r + 1] = n_color, O.stats[3 * r + 2] = walk_steps;
+        if (V.rec != nullptr) V.n[r] = n_visits;
     }
 }
 
 template <bool TRACE>
-__global__ void __launch_bounds__(kBlock) march_group_kernel(MarchField F, MarchParams M, MarchRays R, MarchOut O) {
+__global__ void __launch_bounds__(kBlock, kGroupWaves)
+    march_group_kernel(MarchField F, MarchParams M, MarchRays R, MarchOut O, MarchVisits V) {
     const int64_t i = (xcd_block_id() * kBlock + threadIdx.x) / kGroup;
     const int g = threadIdx.x % kGroup;
     if (i >= R.n) return;
@@ -1054,14 +1127,15 @@ __global__ void __launch_bounds__(kBlock) march_group_kernel(MarchField F, March
             O.rgb[3 * r] = O.rgb[3 * r + 1] = O.rgb[3 * r + 2] = 0.f;
             O.T[r] = 1.f, O.depth[r] = 0.f;
             O.stats[3 * r] = O.stats[3 * r + 1] = O.stats[3 * r + 2] = 0;
+            if (V.rec != nullptr) V.n[r] = 0;
         }
         return;
     }
     switch (F.sh_deg) {
-        case 0: march_ray_group<sh_vec4_f32(0), TRACE>(F, M, R, O, r, cur, g); break;
-        case 1: march_ray_group<sh_vec4_f32(1), TRACE>(F, M, R, O, r, cur, g); break;
-        case 2: march_ray_group<sh_vec4_f32(2), TRACE>(F, M, R, O, r, cur, g); break;
-        default: march_ray_group<sh_vec4_f32(3), TRACE>(F, M, R, O, r, cur, g); break;
+        case 0: march_ray_group<sh_vec4_f32(0), TRACE>(F, M, R, O, V, r, cur, g); break;
+        case 1: march_ray_group<sh_vec4_f32(1), TRACE>(F, M, R, O, V, r, cur, g); break;
+        case 2: march_ray_group<sh_vec4_f32(2), TRACE>(F, M, R, O, V, r, cur, g); break;
+        default: march_ray_group<sh_vec4_f32(3), TRACE>(F, M, R, O, V, r, cur, g); break;
     }
 }
 
@@ -1184,7 +1258,7 @@ __device__ void march_ray_group_backward(const MarchField& F, const MarchParams&
             continue;
         }
         moves = 0;
-        if (Cc.cell != cur) flush(), enter_cell(F, cur, g, Cc);
+        if (Cc.cell != cur) flush(), enter_cell<block_vec4(NV)>(F, cur, g, Cc);
         const float alpha = 1.f - fexp(-Q.sigma * delta);
         const float w = T * alpha;
         const float T_next = T * (1.f - alpha);
@@ -1203,7 +1277,7 @@ __device__ void march_ray_group_backward(const MarchField& F, const MarchParams&
 #pragma unroll
         for (int s = 0; s < kSlots; ++s) {
             if (Cc.k[s] >= 0) {
-                const SiteRec rc = site_rec<block_vec4(NV)>(F, Cc.k[s]);
+                const SiteRec& rc = Cc.rc[s];
                 const float c[3] = {Cc.col_ok ? Cc.c[s][0] : 0.f, Cc.col_ok ? Cc.c[s][1] : 0.f,
                                     Cc.col_ok ? Cc.c[s][2] : 0.f};
                 sample_grad(rc, x, c, gR, gsig, coloured, w, Q.mmin, inv_a, grc, S[s]);
@@ -1228,12 +1302,14 @@ __device__ void march_ray_group_backward(const MarchField& F, const MarchParams&
 }
 
 __global__ void __launch_bounds__(kBlock)
-    march_group_backward_kernel(MarchField F, MarchParams M, MarchRays R, MarchGradIn GI, MarchGradOut G) {
+    march_group_backward_kernel(MarchField F, MarchParams M, MarchRays R, MarchGradIn GI, MarchGradOut G,
+                                MarchVisits V) {
     static_assert(kBlock == 64, "the gradient slots are per wave: one wave per workgroup");
     __shared__ float slots[kSlot * 64];
     const int64_t r = (xcd_block_id() * kBlock + threadIdx.x) / kGroup;
     const int g = threadIdx.x % kGroup;
     if (r >= R.n) return;
+    if (V.rec != nullptr && V.n[r] > 0 && V.n[r] <= V.cap) return;  // march_visits_kernel's
     const int cur = R.start[r];
     if (cur < 0 || cur >= F.n_sites) return;
     switch (F.sh_deg) {
@@ -1241,6 +1317,137 @@ __global__ void __launch_bounds__(kBlock)
         case 1: march_ray_group_backward<sh_vec4_f32(1)>(F, M, R, GI, G, r, cur, g, slots); break;
         case 2: march_ray_group_backward<sh_vec4_f32(2)>(F, M, R, GI, G, r, cur, g, slots); break;
         default: march_ray_group_backward<sh_vec4_f32(3)>(F, M, R, GI, G, r, cur, g, slots); break;
+    }
+}
+
+// ------------------------------------------------------------------------ march backward of recorded visits
+//
+// march_ray_group_backward walks a ray again sample by sample, a chain of hundreds to thousands of rounds for a batch that
+// fills one wave per SIMD. With the forward's visit records the runs of a ray are independent: each has its cell (no walk),
+// its first sample, and the transmittance and colour before it, from which the run's samples replay with the forward's
+// bits. A group of 16 lanes takes a run, kVisitWaves waves of 4 groups per ray: it reads its neighbourhood once, keeps its
+// gradients in registers over the run, and adds them as rows shared by the wave. The arithmetic is
+// march_ray_group_backward's. 4,096 rays among 256k sites, steps of 1/512: 8.40 ms walking the rays again, 1.1 ms by visits;
+// bound by instructions (each sample's terms, sums and gradients over the group).
+constexpr int kVisitWaves = 8;
+
+template <int NV>
+__device__ void march_visits(const MarchField& F, const MarchParams& M, const MarchRays& R, const MarchGradIn& GI,
+                             const MarchGradOut& G, const MarchVisits& V, int n_samples, int64_t r, int first,
+                             float* __restrict__ slots) {
+    const float o[3] = {R.o[3 * r], R.o[3 * r + 1], R.o[3 * r + 2]};
+    const float d[3] = {R.d[3 * r], R.d[3 * r + 1], R.d[3 * r + 2]};
+    const float near = R.t_near[r], mid = R.t_mid[r], far = R.t_far[r];
+    const int n_in = mid > near ? static_cast<int>(ceilf((mid - near) / M.dt)) : 0;
+    const int nb = (F.sh_deg + 1) * (F.sh_deg + 1), lane = threadIdx.x & 63, g = lane % kGroup;
+    const int n_visits = V.n[r];
+    float b[16];
+    sh_basis(d[0], d[1], d[2], F.sh_deg, b);
+    const float gR[3] = {GI.g_rgb[3 * r], GI.g_rgb[3 * r + 1], GI.g_rgb[3 * r + 2]};
+    const float fg[3] = {GI.rgb[3 * r], GI.rgb[3 * r + 1], GI.rgb[3 * r + 2]};
+    const float gT_final = GI.g_T[r] * GI.T[r];
+    const RowLane RL = row_lane(nb);
+    float* mine = slots + kSlot * lane;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) mine[16 + j] = b[j];
+    for (int base = first; base < n_visits; base += 4 * kVisitWaves) {
+        const int v = base + lane / kGroup;
+        GroupCell Cc;
+        SlotGrad S[kSlots];
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) clear_slot(S[s]), Cc.k[s] = -1;
+        Cc.cell = -1, Cc.col_ok = false;
+        if (v < n_visits) {
+            const float* p = V.rec + (r * V.cap + v) * kVisitFloats;
+            const int k0 = __float_as_int(p[1]);
+            const int k1 = v + 1 < n_visits ? __float_as_int(p[kVisitFloats + 1]) : n_samples;
+            float T = p[2], acc[3] = {p[3], p[4], p[5]};
+            enter_cell<block_vec4(NV)>(F, __float_as_int(p[0]), g, Cc);
+            for (int k = k0; k < k1; ++k) {
+                float t, delta, x[3];
+                sample_at(near, mid, far, n_in, M, k, t, delta);
+                point_at(o, d, t, x);
+                float sg = 0.f, mm = kInf;
+                const auto terms = [&](const SiteRec& rc) {
+                    float u[3];
+                    offset_to(rc.q0, x, u);
+                    sg += fexp(rc.q0.w - 0.5f * density_m(rc, u));
+                    mm = fminf(mm, color_m(rc.q2, rc.q3, u));
+                };
+#pragma unroll
+                for (int s = 0; s < kSlots; ++s)
+                    if (Cc.k[s] >= 0) terms(Cc.rc[s]);
+                for (int e = g + kGroup * kSlots; e < Cc.n; e += kGroup)
+                    terms(site_rec<block_vec4(NV)>(F, neighbor(F, Cc.cell, Cc.e0, e)));
+                const float sigma = row_sum(sg), mmin = row_min(mm);
+                const float alpha = 1.f - fexp(-sigma * delta);
+                const float w = T * alpha;
+                const float T_next = T * (1.f - alpha);
+                const bool coloured = w > M.w_thresh;
+                float inv_a = 0.f, C[3] = {0.f, 0.f, 0.f}, grc = 0.f;
+                if (coloured) {
+                    group_colour<NV>(F, Cc, x, b, nb, mmin, g, inv_a, C);
+#pragma unroll
+                    for (int a = 0; a < 3; ++a) acc[a] += w * C[a];
+                    grc = gR[0] * C[0] + gR[1] * C[1] + gR[2] * C[2];
+                }
+                float gs = 0.f;
+#pragma unroll
+                for (int a = 0; a < 3; ++a) gs += gR[a] * (T_next * C[a] - (fg[a] - acc[a]));
+                const float gsig = delta * (gs - gT_final);
+#pragma unroll
+                for (int s = 0; s < kSlots; ++s) {
+                    if (Cc.k[s] >= 0) {
+                        const float c[3] = {Cc.col_ok ? Cc.c[s][0] : 0.f, Cc.col_ok ? Cc.c[s][1] : 0.f,
+                                            Cc.col_ok ? Cc.c[s][2] : 0.f};
+                        sample_grad(Cc.rc[s], x, c, gR, gsig, coloured, w, mmin, inv_a, grc, S[s]);
+                    }
+                }
+                for (int e = g + kGroup * kSlots; e < Cc.n; e += kGroup) {
+                    const int kk = neighbor(F, Cc.cell, Cc.e0, e);
+                    const float4* rp = F.rec + block_vec4(NV) * static_cast<int64_t>(kk);
+                    const SiteRec rc = {rp[0], rp[1], rp[2], rp[3]};
+                    float c[3] = {0.f, 0.f, 0.f};
+                    if (coloured) sh_eval_n<NV>(rp + kRec, b, nb, c);
+                    SlotGrad A;
+                    clear_slot(A);
+                    sample_grad(rc, x, c, gR, gsig, coloured, w, mmin, inv_a, grc, A);
+                    flush_slot(G, kk, c, b, nb, gR, A);
+                }
+                T = T_next;
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < kSlots; ++s) {
+            const bool row = Cc.k[s] >= 0 && (S[s].dens || S[s].col);
+            if (row) {
+                mine[0] = S[s].raw;
+#pragma unroll
+                for (int u = 0; u < 6; ++u) mine[1 + u] = S[s].dA[u], mine[7 + u] = S[s].cA[u];
+#pragma unroll
+                for (int ch = 0; ch < 3; ++ch) mine[13 + ch] = S[s].col && Cc.c[s][ch] > 0.f ? gR[ch] * S[s].aw : 0.f;
+            }
+            __builtin_amdgcn_wave_barrier();
+            add_rows_wave(G, slots, __ballot(row), Cc.k[s], RL);
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+}
+
+__global__ void __launch_bounds__(kBlock, 3)
+    march_visits_kernel(MarchField F, MarchParams M, MarchRays R, MarchGradIn GI, MarchGradOut G, MarchVisits V,
+                        const int* __restrict__ stats) {
+    __shared__ float slots[kSlot * 64];
+    const int64_t id = xcd_block_id(), r = id / kVisitWaves;
+    const int first = 4 * static_cast<int>(id % kVisitWaves);
+    const int n = V.n[r];
+    if (n > V.cap || first >= n) return;
+    const int n_samples = stats[3 * r];
+    switch (F.sh_deg) {
+        case 0: march_visits<sh_vec4_f32(0)>(F, M, R, GI, G, V, n_samples, r, first, slots); break;
+        case 1: march_visits<sh_vec4_f32(1)>(F, M, R, GI, G, V, n_samples, r, first, slots); break;
+        case 2: march_visits<sh_vec4_f32(2)>(F, M, R, GI, G, V, n_samples, r, first, slots); break;
+        default: march_visits<sh_vec4_f32(3)>(F, M, R, GI, G, V, n_samples, r, first, slots); break;
     }
 }
 
@@ -1443,7 +1650,7 @@ __global__ void __launch_bounds__(kBlock)
 // (scattered fp32 atomics, one per lane and float, ran this kernel at ~16 G atomics/s, where a row is one atomic
 // instruction on two lines). The neighbour rounds run in step across the wave: every active lane takes part in
 // every round, lanes of rays with fewer neighbours (or nothing to add) idle.
-template <int NV>
+template <int NV, bool WAVE = false>
 __device__ void train_scatter(const MarchField& F, const MarchGradOut& G, const float (&o)[3], const float (&d)[3],
                               const float (&b)[16], int nb, const TrainSample& S, float gs, const float (&gC)[3],
                               int g, float* __restrict__ slots) {
@@ -1458,6 +1665,7 @@ __device__ void train_scatter(const MarchField& F, const MarchGradOut& G, const 
     const uint64_t act = __ballot(1);
     const int n_act = __popcll(act);
     const int rank = __popcll(act & ((uint64_t(1) << lane) - 1));
+    const RowLane RL = WAVE ? row_lane(nb) : RowLane{};
     for (int base = 0; __ballot(base < n) != 0; base += kGroup) {
         const int e = base + g;
         int k = 0;
@@ -1496,7 +1704,8 @@ __device__ void train_scatter(const MarchField& F, const MarchGradOut& G, const 
             }
         }
         __builtin_amdgcn_wave_barrier();
-        add_rows(G, slots, __ballot(row), k, nb, rank, n_act);
+        if constexpr (WAVE) add_rows_wave(G, slots, __ballot(row), k, RL);
+        else add_rows(G, slots, __ballot(row), k, nb, rank, n_act);
         __builtin_amdgcn_wave_barrier();
     }
 }
@@ -1572,18 +1781,141 @@ __device__ void train_ray_backward(const MarchField& F, const MarchParams& M, co
 
 __global__ void __launch_bounds__(kBlock)
     train_backward_kernel(MarchField F, MarchParams M, TrainRays R, MarchGradIn GI, MarchGradOut G,
-                          const float* __restrict__ rec, int K, const int* __restrict__ stats) {
+                          const float* __restrict__ rec, int K, const int* __restrict__ stats,
+                          const int* __restrict__ count) {
     static_assert(kBlock == 64, "the gradient slots are per wave: one wave per workgroup");
     __shared__ float slots[kSlot * 64];
     const int64_t r = (xcd_block_id() * kBlock + threadIdx.x) / kGroup;
     const int g = threadIdx.x % kGroup;
     if (r >= R.n) return;
+    if (count != nullptr && count[r] > 0) return;  // scattered sample by sample
     if (R.start[r] < 0 || R.start[r] >= F.n_sites) return;  // not traced: no gradient
     switch (F.sh_deg) {
         case 0: train_ray_backward<sh_vec4_f32(0)>(F, M, R, GI, G, rec, K, stats, r, g, slots); break;
         case 1: train_ray_backward<sh_vec4_f32(1)>(F, M, R, GI, G, rec, K, stats, r, g, slots); break;
         case 2: train_ray_backward<sh_vec4_f32(2)>(F, M, R, GI, G, rec, K, stats, r, g, slots); break;
         default: train_ray_backward<sh_vec4_f32(3)>(F, M, R, GI, G, rec, K, stats, r, g, slots); break;
+    }
+}
+
+// ------------------------------------------------------------ backward of recorded rays, one sample per 16 lanes
+//
+// train_ray_backward walks a ray's samples in turn, so a batch of 4,096 rays is 1,024 waves (one per SIMD), each a chain of
+// about 100 samples times the latency of a neighbourhood and of the rows' LDS reads. Only two scalars of that chain depend
+// on the order, the transmittance and the composited colour: train_grads_kernel runs them over a ray's records (one lane per
+// ray, four records in flight) and leaves each sample's dL/dsigma and dL/dC; then the samples of all rays are independent
+// and train_samples_kernel scatters them, kSampleWaves waves per ray, 4 samples per wave at a time. The arithmetic is
+// train_ray_backward's. count[r] is the number of samples scattered; 0 leaves the ray to train_backward_kernel (no
+// records, more samples than fit, or a segment whose weight passes w_thresh here and did not in the forward).
+// 4,096 rays among 442k sites, 65 samples per ray: 3.43 ms walking the rays, 0.07 + 0.48 ms split; bound now by the
+// records gathered per neighbour and the rows' atomics.
+constexpr int kSampleWaves = 8;
+constexpr int kAhead = 4;
+constexpr int64_t kSplitRays = int64_t(1) << 22;  // 8 waves (512 threads) per ray stay below 2^32
+
+__global__ void __launch_bounds__(kBlock)
+    train_grads_kernel(MarchParams M, const int* __restrict__ start, int n_sites, MarchGradIn GI,
+                       const float4* __restrict__ rec, int K, const int* __restrict__ stats, int64_t n_rays,
+                       float4* __restrict__ grads, int* __restrict__ count) {
+    const int64_t r = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    if (r >= n_rays) return;
+    const int n = stats[3 * r] <= K && start[r] >= 0 && start[r] < n_sites ? stats[3 * r] : 0;
+    if (n <= 0) {
+        count[r] = 0;
+        return;
+    }
+    const float gR[3] = {GI.g_rgb[3 * r], GI.g_rgb[3 * r + 1], GI.g_rgb[3 * r + 2]};
+    const float fg[3] = {GI.rgb[3 * r], GI.rgb[3 * r + 1], GI.rgb[3 * r + 2]};
+    const float gT_final = GI.g_T[r] * GI.T[r];
+    const float4* p = rec + 2 * (r * K);  // (t, site, sigma, C0), (C1, C2, mmin, inv_a)
+    float4* out = grads + r * K;
+    float4 A0 = p[0], A1 = p[1], q0[kAhead], q1[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+        const int s = min(1 + u, n - 1);
+        q0[u] = p[2 * s], q1[u] = p[2 * s + 1];
+    }
+    float T = 1.f, acc[3] = {0.f, 0.f, 0.f}, gs_pending = 0.f, gC_pending[3] = {0.f, 0.f, 0.f};
+    int done = 0;  // samples whose gradients are out
+    bool open = n > 1, redo = false;
+    for (int base = 1; open; base += kAhead) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const int s = base + u;  // segment s - 1 .. s
+            if (open && s < n) {
+                const float4 B0 = q0[u], B1 = q1[u];
+                const int ahead = min(s + kAhead, n - 1);
+                q0[u] = p[2 * ahead], q1[u] = p[2 * ahead + 1];
+                const float delta = B0.x - A0.x;
+                const float alpha = 1.f - fexp(-0.5f * (A0.z + B0.z) * delta);
+                const float w = T * alpha;
+                const float T_next = T * (1.f - alpha);
+                const bool active = w > M.w_thresh;
+                float c[3] = {0.f, 0.f, 0.f};
+                if (active) {
+                    redo = redo || !(A1.w > 0.f) || !(B1.w > 0.f);
+                    const float CA[3] = {A0.w, A1.x, A1.y}, CB[3] = {B0.w, B1.x, B1.y};
+#pragma unroll
+                    for (int a = 0; a < 3; ++a) c[a] = 0.5f * (CA[a] + CB[a]), acc[a] += w * c[a];
+                }
+                float g_sbar = 0.f;
+#pragma unroll
+                for (int a = 0; a < 3; ++a) g_sbar += gR[a] * (T_next * c[a] - (fg[a] - acc[a]));
+                g_sbar = delta * (g_sbar - gT_final);
+                float gc_half[3];
+#pragma unroll
+                for (int a = 0; a < 3; ++a) gc_half[a] = active ? 0.5f * w * gR[a] : 0.f;
+                out[s - 1] = make_float4(gs_pending + 0.5f * g_sbar, gC_pending[0] + gc_half[0],
+                                         gC_pending[1] + gc_half[1], gC_pending[2] + gc_half[2]);
+                gs_pending = 0.5f * g_sbar;
+#pragma unroll
+                for (int a = 0; a < 3; ++a) gC_pending[a] = gc_half[a];
+                T = T_next, A0 = B0, A1 = B1, done = s;
+                if (s + 1 >= n || T < M.t_thresh) open = false;
+            }
+        }
+    }
+    out[done] = make_float4(gs_pending, gC_pending[0], gC_pending[1], gC_pending[2]);
+    count[r] = redo ? 0 : done + 1;
+}
+
+template <int NV>
+__device__ void train_samples(const MarchField& F, const TrainRays& R, const MarchGradOut& G,
+                              const float* __restrict__ rec, int K, const float4* __restrict__ grads, int n, int64_t r,
+                              int first, float* __restrict__ slots) {
+    const float o[3] = {R.o[3 * r], R.o[3 * r + 1], R.o[3 * r + 2]};
+    const float d[3] = {R.d[3 * r], R.d[3 * r + 1], R.d[3 * r + 2]};
+    const int nb = (F.sh_deg + 1) * (F.sh_deg + 1), lane = threadIdx.x & 63, g = lane % kGroup;
+    float b[16];
+    sh_basis(d[0], d[1], d[2], F.sh_deg, b);
+#pragma unroll
+    for (int j = 0; j < 16; ++j) slots[kSlot * lane + 16 + j] = b[j];
+    for (int base = first; base < n; base += 4 * kSampleWaves) {
+        const int s = base + lane / kGroup;
+        TrainSample S{};
+        float gs = 0.f, gC[3] = {0.f, 0.f, 0.f};
+        if (s < n) {
+            train_load(rec, r, K, s, S);
+            const float4 v = grads[r * K + s];
+            gs = v.x, gC[0] = v.y, gC[1] = v.z, gC[2] = v.w;
+        }
+        train_scatter<NV, true>(F, G, o, d, b, nb, S, gs, gC, g, slots);
+    }
+}
+
+__global__ void __launch_bounds__(kBlock)
+    train_samples_kernel(MarchField F, TrainRays R, MarchGradOut G, const float* __restrict__ rec, int K,
+                         const float4* __restrict__ grads, const int* __restrict__ count) {
+    __shared__ float slots[kSlot * 64];
+    const int64_t id = xcd_block_id(), r = id / kSampleWaves;
+    const int first = 4 * static_cast<int>(id % kSampleWaves);
+    const int n = count[r];
+    if (first >= n) return;
+    switch (F.sh_deg) {
+        case 0: train_samples<sh_vec4_f32(0)>(F, R, G, rec, K, grads, n, r, first, slots); break;
+        case 1: train_samples<sh_vec4_f32(1)>(F, R, G, rec, K, grads, n, r, first, slots); break;
+        case 2: train_samples<sh_vec4_f32(2)>(F, R, G, rec, K, grads, n, r, first, slots); break;
+        default: train_samples<sh_vec4_f32(3)>(F, R, G, rec, K, grads, n, r, first, slots); break;
     }
 }
 
@@ -1621,16 +1953,15 @@ int64_t march_lanes(int64_t lanes, int64_t n_rays) { return lanes != 0 ? lanes :
 }  // namespace
 }  // namespace vgr
 
-extern "C" int vgr_march_forward_lanes(const float* points, int64_t n_sites, const int32_t* offsets,
-                                       const int32_t* adj, int64_t n_adj, const float* raw, const float* dA,
-                                       const float* cA, const float* sh, int64_t sh_deg, const float* o,
-                                       const float* d, const int32_t* start, const float* near_t,
-                                       const float* mid_t, const float* far_t, int64_t n_rays, double dt,
-                                       int64_t n_bg, double t_thresh, double w_thresh, float* rgb, float* T,
-                                       float* depth, int32_t* stats, int32_t* trace, int64_t trace_cap,
-                                       const int32_t* order, int64_t lanes_per_ray, void* work, int64_t work_bytes,
-                                       void* stream) {
-    using namespace vgr;
+namespace vgr {
+namespace {
+
+int march_forward(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t* adj, int64_t n_adj,
+                  const float* raw, const float* dA, const float* cA, const float* sh, int64_t sh_deg, const float* o,
+                  const float* d, const int32_t* start, const float* near_t, const float* mid_t, const float* far_t,
+                  int64_t n_rays, double dt, int64_t n_bg, double t_thresh, double w_thresh, float* rgb, float* T,
+                  float* depth, int32_t* stats, int32_t* trace, int64_t trace_cap, const int32_t* order, int64_t
+                  lanes_per_ray, void* work, int64_t work_bytes, const MarchVisits& V, void* stream) {
     VGR_REQUIRE(lanes_per_ray == 0 || lanes_per_ray == 1 || lanes_per_ray == kGroup,
                 "march_forward: lanes_per_ray must be 0 (by batch size), 1 or 16 (got %lld)",
                 static_cast<long long>(lanes_per_ray));
@@ -1657,9 +1988,9 @@ extern "C" int vgr_march_forward_lanes(const float* points, int64_t n_sites, con
     if (march_lanes(lanes_per_ray, n_rays) == kGroup) {
         const dim3 grid(grid_for(n_rays * kGroup, kBlock));
         if (trace != nullptr)
-            hipLaunchKernelGGL(march_group_kernel<true>, grid, dim3(kBlock), 0, as_stream(stream), F, M, R, O);
+            hipLaunchKernelGGL(march_group_kernel<true>, grid, dim3(kBlock), 0, as_stream(stream), F, M, R, O, V);
         else
-            hipLaunchKernelGGL(march_group_kernel<false>, grid, dim3(kBlock), 0, as_stream(stream), F, M, R, O);
+            hipLaunchKernelGGL(march_group_kernel<false>, grid, dim3(kBlock), 0, as_stream(stream), F, M, R, O, V);
         return launch_status("march_group_kernel");
     }
     if (trace != nullptr)
@@ -1669,6 +2000,36 @@ extern "C" int vgr_march_forward_lanes(const float* points, int64_t n_sites, con
         hipLaunchKernelGGL(march_forward_kernel<false>, dim3(grid_for(n_rays, kBlock)), dim3(kBlock), 0,
                            as_stream(stream), F, M, R, O);
     return launch_status("march_forward_kernel");
+}
+
+}  // namespace
+}  // namespace vgr
+
+extern "C" int vgr_march_forward_lanes(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t*
+                                       adj, int64_t n_adj, const float* raw, const float* dA, const float* cA, const
+                                       float* sh, int64_t sh_deg, const float* o, const float* d, const int32_t*
+                                       start, const float* near_t, const float* mid_t, const float* far_t, int64_t
+                                       n_rays, double dt, int64_t n_bg, double t_thresh, double w_thresh, float* rgb,
+                                       float* T, float* depth, int32_t* stats, int32_t* trace, int64_t trace_cap,
+                                       const int32_t* order, int64_t lanes_per_ray, void* work, int64_t work_bytes,
+                                       void* stream) {
+    return vgr::march_forward(points, n_sites, offsets, adj, n_adj, raw, dA, cA, sh, sh_deg, o, d, start, near_t,
+        mid_t, far_t, n_rays, dt, n_bg, t_thresh, w_thresh, rgb, T, depth, stats, trace, trace_cap, order,
+        lanes_per_ray, work, work_bytes, vgr::MarchVisits{}, stream);
+}
+
+extern "C" int vgr_march_forward_visits(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t*
+                                        adj, int64_t n_adj, const float* raw, const float* dA, const float* cA, const
+                                        float* sh, int64_t sh_deg, const float* o, const float* d, const int32_t*
+                                        start, const float* near_t, const float* mid_t, const float* far_t, int64_t
+                                        n_rays, double dt, int64_t n_bg, double t_thresh, double w_thresh, float* rgb,
+                                        float* T, float* depth, int32_t* stats, void* work, int64_t work_bytes, float*
+                                        visits, int64_t visit_cap, int32_t* n_visits, void* stream) {
+    VGR_REQUIRE(visits && n_visits && visit_cap > 0 && visit_cap <= INT_MAX,
+                "march_forward_visits: visits and n_visits are required, visit_cap in [1, 2^31)");
+    return vgr::march_forward(points, n_sites, offsets, adj, n_adj, raw, dA, cA, sh, sh_deg, o, d, start, near_t,
+        mid_t, far_t, n_rays, dt, n_bg, t_thresh, w_thresh, rgb, T, depth, stats, nullptr, 0, nullptr, vgr::kGroup,
+        work, work_bytes, vgr::MarchVisits{visits, n_visits, int(visit_cap)}, stream);
 }
 
 extern "C" int vgr_march_forward(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t* adj,
@@ -1683,15 +2044,16 @@ extern "C" int vgr_march_forward(const float* points, int64_t n_sites, const int
                                    trace_cap, nullptr, 0, work, work_bytes, stream);
 }
 
-extern "C" int vgr_march_backward(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t* adj,
-                                  int64_t n_adj, const float* raw, const float* dA, const float* cA, const float* sh,
-                                  int64_t sh_deg, const float* o, const float* d, const int32_t* start,
-                                  const float* near_t, const float* mid_t, const float* far_t, int64_t n_rays,
-                                  double dt, int64_t n_bg, double t_thresh, double w_thresh, const float* rgb,
-                                  const float* T, const float* g_rgb, const float* g_T, float* g_raw, float* g_dA,
-                                  float* g_cA, float* g_sh, int64_t lanes_per_ray, int64_t blocks_ready, void* work,
-                                  int64_t work_bytes, void* stream) {
-    using namespace vgr;
+namespace vgr {
+namespace {
+
+int march_backward(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t* adj, int64_t n_adj,
+                   const float* raw, const float* dA, const float* cA, const float* sh, int64_t sh_deg, const float*
+                   o, const float* d, const int32_t* start, const float* near_t, const float* mid_t, const float*
+                   far_t, int64_t n_rays, double dt, int64_t n_bg, double t_thresh, double w_thresh, const float* rgb,
+                   const float* T, const float* g_rgb, const float* g_T, float* g_raw, float* g_dA, float* g_cA,
+                   float* g_sh, int64_t lanes_per_ray, int64_t blocks_ready, void* work, int64_t work_bytes, const
+                   MarchVisits& V, const int32_t* stats, void* stream) {
     VGR_REQUIRE(lanes_per_ray == 0 || lanes_per_ray == 1 || lanes_per_ray == kGroup,
                 "march_backward: lanes_per_ray must be 0 (by batch size), 1 or 16 (got %lld)",
                 static_cast<long long>(lanes_per_ray));
@@ -1730,10 +2092,14 @@ extern "C" int vgr_march_backward(const float* points, int64_t n_sites, const in
     // wave-shared atomics once the launch holds at least one wave per CU (16384 rays); per-lane atomics below, where
     // the launch is bound by the latency of its few waves (config 5: 4096 rays 85 against 158 ms, 65536 rays 456
     // against 193 ms)
-    if (march_lanes(lanes_per_ray, n_rays) == kGroup)
+    if (march_lanes(lanes_per_ray, n_rays) == kGroup) {
+        if (V.rec != nullptr)
+            hipLaunchKernelGGL(march_visits_kernel, dim3(static_cast<unsigned>(n_rays * kVisitWaves)), dim3(kBlock),
+                0, s, F,
+                               M, R, GI, G, V, stats);
         hipLaunchKernelGGL(march_group_backward_kernel, dim3(grid_for(n_rays * kGroup, kBlock)), dim3(kBlock), 0, s,
-                           F, M, R, GI, G);
-    else if (n_rays >= kCoopRays)
+                           F, M, R, GI, G, V);
+    } else if (n_rays >= kCoopRays)
         hipLaunchKernelGGL(march_backward_kernel<true>, dim3(grid_for(n_rays, kBlock)), dim3(kBlock), 0, s, F, M, R,
                            GI, G);
     else
@@ -1742,6 +2108,41 @@ extern "C" int vgr_march_backward(const float* points, int64_t n_sites, const in
     hipLaunchKernelGGL(grad_unpack_kernel, dim3(grid_for(kGradBlock * n_sites, 256)), dim3(256), 0, s, block, n_sites,
                        g_raw, g_dA, g_cA, g_sh);
     return launch_status("march_backward_kernel");
+}
+
+}  // namespace
+}  // namespace vgr
+
+extern "C" int vgr_march_backward(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t* adj,
+                                  int64_t n_adj, const float* raw, const float* dA, const float* cA, const float* sh,
+                                  int64_t sh_deg, const float* o, const float* d, const int32_t* start, const float*
+                                  near_t, const float* mid_t, const float* far_t, int64_t n_rays, double dt, int64_t
+                                  n_bg, double t_thresh, double w_thresh, const float* rgb, const float* T, const
+                                  float* g_rgb, const float* g_T, float* g_raw, float* g_dA, float* g_cA, float* g_sh,
+                                  int64_t lanes_per_ray, int64_t blocks_ready, void* work, int64_t work_bytes, void*
+                                  stream) {
+    return vgr::march_backward(points, n_sites, offsets, adj, n_adj, raw, dA, cA, sh, sh_deg, o, d, start, near_t,
+        mid_t, far_t, n_rays, dt, n_bg, t_thresh, w_thresh, rgb, T, g_rgb, g_T, g_raw, g_dA, g_cA, g_sh,
+        lanes_per_ray, blocks_ready, work, work_bytes, vgr::MarchVisits{}, nullptr, stream);
+}
+
+extern "C" int vgr_march_backward_visits(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t*
+                                        adj, int64_t n_adj, const float* raw, const float* dA, const float* cA, const
+                                        float* sh, int64_t sh_deg, const float* o, const float* d, const int32_t*
+                                        start, const float* near_t, const float* mid_t, const float* far_t, int64_t
+                                        n_rays, double dt, int64_t n_bg, double t_thresh, double w_thresh, const
+                                        float* rgb, const float* T, const float* g_rgb, const float* g_T, float*
+                                        g_raw, float* g_dA, float* g_cA, float* g_sh, int64_t blocks_ready, void*
+                                        work, int64_t work_bytes, const float* visits, int64_t visit_cap, const
+                                        int32_t* n_visits, const int32_t* stats, void* stream) {
+    VGR_REQUIRE(n_rays == 0 || (visits && n_visits && stats && visit_cap > 0 && visit_cap <= INT_MAX),
+                "march_backward_visits: visits, n_visits and stats are required, visit_cap in [1, 2^31)");
+    VGR_REQUIRE(n_rays <= vgr::kSplitRays, "march_backward_visits: at most %lld rays", static_cast<long
+        long>(vgr::kSplitRays));
+    return vgr::march_backward(points, n_sites, offsets, adj, n_adj, raw, dA, cA, sh, sh_deg, o, d, start, near_t,
+        mid_t, far_t, n_rays, dt, n_bg, t_thresh, w_thresh, rgb, T, g_rgb, g_T, g_raw, g_dA, g_cA, g_sh, vgr::kGroup,
+        blocks_ready, work, work_bytes, vgr::MarchVisits{const_cast<float*>(visits), const_cast<int32_t*>(n_visits),
+        int(visit_cap)}, stats, stream);
 }
 
 extern "C" int64_t vgr_foam_work_size(int64_t n_sites, int64_t sh_deg) {
@@ -1794,15 +2195,21 @@ extern "C" int vgr_foam_forward(const float* points, int64_t n_sites, const int3
     return launch_status("train_forward_kernel");
 }
 
-extern "C" int vgr_foam_backward(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t* adj,
+extern "C" int64_t vgr_foam_scratch_size(int64_t n_rays, int64_t record_cap) {
+    return n_rays > 0 && record_cap > 0 ? n_rays * (16 * record_cap + 4) : 0;
+}
+
+namespace vgr {
+namespace {
+
+int foam_backward(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t* adj,
                                  int64_t n_adj, const float* raw, const float* dA, const float* cA, const float* sh,
                                  int64_t sh_deg, const float* o, const float* d, const int32_t* start,
                                  const float* near_t, const float* far_t, int64_t n_rays, double t_thresh,
                                  double w_thresh, const float* rgb, const float* T, const float* g_rgb,
                                  const float* g_T, const float* rec, int64_t record_cap, const int32_t* stats,
                                  float* g_raw, float* g_dA, float* g_cA, float* g_sh, int64_t blocks_ready,
-                                 void* work, int64_t work_bytes, void* stream) {
-    using namespace vgr;
+                                 void* work, int64_t work_bytes, void* scratch, int64_t scratch_bytes, void* stream) {
     VGR_REQUIRE(n_sites > 0 && n_sites <= INT_MAX, "foam_backward: n_sites must be in [1, 2^31)");
     VGR_REQUIRE(g_raw && g_dA && g_cA && g_sh, "foam_backward: null gradient pointer");
     const hipStream_t s = as_stream(stream);
@@ -1828,9 +2235,55 @@ extern "C" int vgr_foam_backward(const float* points, int64_t n_sites, const int
     const TrainRays R{o, d, start, near_t, far_t, n_rays};
     const MarchGradIn GI{rgb, T, g_rgb, g_T};
     const MarchGradOut G{block};
+    int* count = nullptr;
+    if (scratch != nullptr && record_cap > 0 && n_rays <= kSplitRays) {
+        VGR_REQUIRE(scratch_bytes >= vgr_foam_scratch_size(n_rays, record_cap) &&
+                        reinterpret_cast<uintptr_t>(scratch) % 16 == 0,
+                    "foam_backward: scratch must hold vgr_foam_scratch_size(B, record_cap) = %lld bytes, 16-byte "
+                    "aligned",
+                    static_cast<long long>(vgr_foam_scratch_size(n_rays, record_cap)));
+        VGR_REQUIRE(reinterpret_cast<uintptr_t>(rec) % 16 == 0, "foam_backward: rec must be 16-byte aligned");
+        float4* grads = static_cast<float4*>(scratch);
+        count = reinterpret_cast<int*>(grads + n_rays * record_cap);
+        hipLaunchKernelGGL(train_grads_kernel, dim3(grid_for(n_rays, kBlock)), dim3(kBlock), 0, s, M, start,
+                           int(n_sites), GI, reinterpret_cast<const float4*>(rec), int(record_cap), stats, n_rays, grads, count);
+        hipLaunchKernelGGL(train_samples_kernel, dim3(static_cast<unsigned>(n_rays * kSampleWaves)), dim3(kBlock), 0,
+            s, F,
+                           R, G, rec, int(record_cap), grads, count);
+    }
     hipLaunchKernelGGL(train_backward_kernel, dim3(grid_for(n_rays * kGroup, kBlock)), dim3(kBlock), 0, s, F, M, R,
-                       GI, G, record_cap > 0 ? rec : nullptr, int(record_cap), stats);
+                       GI, G, record_cap > 0 ? rec : nullptr, int(record_cap), stats, count);
     hipLaunchKernelGGL(grad_unpack_kernel, dim3(grid_for(kGradBlock * n_sites, 256)), dim3(256), 0, s, block, n_sites,
                        g_raw, g_dA, g_cA, g_sh);
     return launch_status("train_backward_kernel");
+}
+
+}  // namespace
+}  // namespace vgr
+
+extern "C" int vgr_foam_backward(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t* adj,
+                                 int64_t n_adj, const float* raw, const float* dA, const float* cA, const float* sh,
+                                 int64_t sh_deg, const float* o, const float* d, const int32_t* start,
+                                 const float* near_t, const float* far_t, int64_t n_rays, double t_thresh,
+                                 double w_thresh, const float* rgb, const float* T, const float* g_rgb,
+                                 const float* g_T, const float* rec, int64_t record_cap, const int32_t* stats,
+                                 float* g_raw, float* g_dA, float* g_cA, float* g_sh, int64_t blocks_ready,
+                                 void* work, int64_t work_bytes, void* stream) {
+    return vgr::foam_backward(points, n_sites, offsets, adj, n_adj, raw, dA, cA, sh, sh_deg, o, d, start, near_t, far_t,
+                              n_rays, t_thresh, w_thresh, rgb, T, g_rgb, g_T, rec, record_cap, stats, g_raw, g_dA, g_cA,
+                              g_sh, blocks_ready, work, work_bytes, nullptr, 0, stream);
+}
+
+extern "C" int vgr_foam_backward_scratch(const float* points, int64_t n_sites, const int32_t* offsets,
+                                         const int32_t* adj, int64_t n_adj, const float* raw, const float* dA,
+                                         const float* cA, const float* sh, int64_t sh_deg, const float* o,
+                                         const float* d, const int32_t* start, const float* near_t, const float* far_t,
+                                         int64_t n_rays, double t_thresh, double w_thresh, const float* rgb,
+                                         const float* T, const float* g_rgb, const float* g_T, const float* rec,
+                                         int64_t record_cap, const int32_t* stats, float* g_raw, float* g_dA,
+                                         float* g_cA, float* g_sh, int64_t blocks_ready, void* work, int64_t work_bytes,
+                                         void* scratch, int64_t scratch_bytes, void* stream) {
+    return vgr::foam_backward(points, n_sites, offsets, adj, n_adj, raw, dA, cA, sh, sh_deg, o, d, start, near_t, far_t,
+                              n_rays, t_thresh, w_thresh, rgb, T, g_rgb, g_T, rec, record_cap, stats, g_raw, g_dA, g_cA,
+                              g_sh, blocks_ready, work, work_bytes, scratch, scratch_bytes, stream);
 }

@@ -67,6 +67,14 @@ SIGNATURES = {
 	'vgr_grid_nearest': [_P, _I64, _I32, _P, _P, _P, _P, _P, _P, _I64, _P, _P],
 	'vgr_grid_cell_points': [_P, _I64, _I32, _P, _P, _P],
 	'vgr_grid_nearest_points': [_P, _I64, _P, _P, _P, _P, _P, _I64, _P, _P, _P],
+	'vgr_march_forward_visits': [_P, _I64, _P, _P, _I64, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _P, _I64,
+								_F64, _I64, _F64, _F64, _P, _P, _P, _P, _P, _I64, _P, _I64, _P, _P],
+	'vgr_march_backward_visits': [_P, _I64, _P, _P, _I64, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _P,
+								_I64, _F64, _I64, _F64, _F64, _P, _P, _P, _P, _P, _P, _P, _P, _I64, _P, _I64, _P, _I64, _P, _P,
+								_P],
+	'vgr_foam_scratch_size': [_I64, _I64],
+	'vgr_foam_backward_scratch': [_P, _I64, _P, _P, _I64, _P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _I64, _F64, _F64, _P,
+								  _P, _P, _P, _P, _I64, _P, _P, _P, _P, _P, _I64, _P, _I64, _P, _I64, _P],
 	'vgr_pack_foam_indexed': [_P, _I64, _P, _P, _I64] + [_P] * 9 + [_F64, _F64] + [_P] * 11 + [_I64, _P, _I64, _P],
 	'vgr_morton_order_work_size': [_I64],
 	'vgr_morton_order': [_P, _I64, _I32, _P, _P, _P, _P, _I64, _P],
@@ -105,6 +113,7 @@ def load():
 		lib.vgr_pack_work_size.restype = ctypes.c_int64
 		lib.vgr_morton_work_size.restype = ctypes.c_int64
 		lib.vgr_ray_order_work_size.restype = ctypes.c_int64
+		lib.vgr_foam_scratch_size.restype = ctypes.c_int64
 		lib.vgr_morton_order_work_size.restype = ctypes.c_int64
 		lib.vgr_points_box_floats.restype = ctypes.c_int64
 		lib.vgr_grid_binned_work_size.restype = ctypes.c_int64

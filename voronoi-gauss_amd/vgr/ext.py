@@ -184,17 +184,40 @@ def _field_work(points, m, records):
 	return torch.empty(wb, dtype=torch.uint8, device=points.device), wb
 
 
+# march_visits allocates records of 32 bytes for MARCH_VISITS runs per ray (a cell, or 32 samples of one: cameras around the
+# unit ball with steps of 1/512 take about 100 cells and 60 further runs of long cells), for at most MARCH_VISIT_BYTES.
+MARCH_VISITS, MARCH_VISIT_BYTES = 256, 1 << 31
+
+
+def march_visits(n_rays, device):
+	"""Buffers of the visit records of n_rays rays for march_forward and march_backward, or None for batches whose records
+	would take more than MARCH_VISIT_BYTES."""
+	if not 0 < n_rays * MARCH_VISITS * 32 <= MARCH_VISIT_BYTES:
+		return None
+	return (torch.empty(n_rays, MARCH_VISITS, 8, dtype=torch.float32, device=device),
+			torch.empty(n_rays, dtype=torch.int32, device=device))
+
+
+def _check_visits(visits, B):
+	_check(visits[0], 'visits', torch.float32)
+	_check(visits[1], 'visit counts', torch.int32)
+	_require(visits[0].dim() == 3 and visits[0].size(0) == B and visits[0].size(1) > 0 and visits[0].size(2) == 8 and
+			 visits[1].shape == (B,), 'visits must be (B, cap, 8) with (B,) counts')
+
+
 # ============================================================================ march.cu forward
 
 class _MarchExtension:
 	@staticmethod
 	def march_forward(points, offsets, adj, raw, dA, cA, sh, sh_deg, o, d, start, near, mid, far, dt, n_bg,
-					  t_thresh, w_thresh, trace_cap=0, lanes=0, work=None, order=None):
+					  t_thresh, w_thresh, trace_cap=0, lanes=0, work=None, order=None, visits=None):
 		"""-> [rgb (B, 3), T (B,), depth (B,), stats (B, 3) int32] (+ trace (B, trace_cap) when trace_cap > 0).
 		lanes: 1 ray per lane (1), 16 lanes per ray (16) or by batch size (0). work: optional uint8 device workspace
 		(at least vgr_march_work_size bytes); a training step passes the backward's, which then reuses its blocks.
 		order: optional int32 (B,) permutation of 0 .. B - 1, the order in which the rays are traced
-		(a ray it leaves out keeps uninitialised outputs; VGR_CHECK_ORDER=1 verifies it) (ray_order); same results."""
+		(a ray it leaves out keeps uninitialised outputs; VGR_CHECK_ORDER=1 verifies it) (ray_order); same results.
+		visits: optional pair (records (B, cap, 8) float32, counts (B,) int32) that a 16-lane forward without trace or
+		order fills for march_backward (march_visits)."""
 		for t, n, dtp in ((points, 'points', torch.float32), (offsets, 'offsets', torch.int32),
 						  (adj, 'adj', torch.int32), (raw, 'raw', torch.float32), (dA, 'dA', torch.float32),
 						  (cA, 'cA', torch.float32), (sh, 'sh', torch.float32), (o, 'o', torch.float32),
@@ -218,6 +241,16 @@ class _MarchExtension:
 			work = torch.empty(max(work_bytes, 1), dtype=torch.uint8, device=dev)
 		else:
 			work_bytes = work.numel()
+		if visits is not None:
+			_require(lanes == 16 and trace is None and order is None, 'visits need lanes=16 and no trace or order')
+			_check_visits(visits, B)
+			with torch.cuda.device(dev):
+				call('vgr_march_forward_visits', ptr(points), points.numel() // 3, ptr(offsets), ptr(adj), adj.numel(),
+					 ptr(raw), ptr(dA), ptr(cA), ptr(sh), int(sh_deg), ptr(o), ptr(d), ptr(start), ptr(near), ptr(mid),
+					 ptr(far), B, float(dt), int(n_bg), float(t_thresh), float(w_thresh), ptr(rgb), ptr(T), ptr(depth),
+					 ptr(stats), ptr(work), work_bytes, ptr(visits[0]), visits[0].size(1), ptr(visits[1]),
+					 stream_of(dev))
+			return out
 		with torch.cuda.device(dev):
 			call('vgr_march_forward_lanes', ptr(points), points.numel() // 3, ptr(offsets), ptr(adj), adj.numel(),
 				 ptr(raw), ptr(dA), ptr(cA), ptr(sh), int(sh_deg), ptr(o), ptr(d), ptr(start), ptr(near), ptr(mid),
@@ -228,10 +261,11 @@ class _MarchExtension:
 
 	@staticmethod
 	def march_backward(points, offsets, adj, raw, dA, cA, sh, sh_deg, o, d, start, near, mid, far, dt, n_bg,
-					   t_thresh, w_thresh, rgb, T, g_rgb, g_T, lanes=0, work=None):
+					   t_thresh, w_thresh, rgb, T, g_rgb, g_T, lanes=0, work=None, visits=None, stats=None):
 		"""-> [g_raw (N,), g_dA (N, 6), g_cA (N, 6), g_sh (N, 16, 3)] (march.cu:405-428). lanes: the layout of the
 		forward that produced rgb and T. work: the forward's workspace (vgr_march_backward_work_size bytes), whose
-		site blocks are reused, or None to pack them again."""
+		site blocks are reused, or None to pack them again. visits: the records a 16-lane forward filled, with that
+		forward's stats, from which every run of samples is replayed on its own; None to march every ray again."""
 		for t, n, dtp in ((points, 'points', torch.float32), (offsets, 'offsets', torch.int32),
 						  (adj, 'adj', torch.int32), (raw, 'raw', torch.float32), (dA, 'dA', torch.float32),
 						  (cA, 'cA', torch.float32), (sh, 'sh', torch.float32), (o, 'o', torch.float32),
@@ -254,6 +288,18 @@ class _MarchExtension:
 			work_bytes = work.numel()
 		else:
 			work = torch.empty(max(work_bytes, 1), dtype=torch.uint8, device=dev)
+		if visits is not None and B > 0:
+			_require(lanes == 16 and stats is not None, 'visits need lanes=16 and the forward\'s stats')
+			_check_visits(visits, B)
+			_check(stats, 'stats', torch.int32)
+			_require(stats.shape == (B, 3), 'stats must be (B, 3)')
+			with torch.cuda.device(dev):
+				call('vgr_march_backward_visits', ptr(points), n, ptr(offsets), ptr(adj), adj.numel(), ptr(raw), ptr(dA),
+					 ptr(cA), ptr(sh), int(sh_deg), ptr(o), ptr(d), ptr(start), ptr(near), ptr(mid), ptr(far), B,
+					 float(dt), int(n_bg), float(t_thresh), float(w_thresh), ptr(rgb), ptr(T), ptr(g_rgb), ptr(g_T),
+					 *[ptr(x) for x in g], int(ready), ptr(work), work_bytes, ptr(visits[0]), visits[0].size(1),
+					 ptr(visits[1]), ptr(stats), stream_of(dev))
+			return g
 		with torch.cuda.device(dev):
 			call('vgr_march_backward', ptr(points), n, ptr(offsets), ptr(adj), adj.numel(), ptr(raw), ptr(dA),
 				 ptr(cA), ptr(sh), int(sh_deg), ptr(o), ptr(d), ptr(start), ptr(near), ptr(mid), ptr(far), B,
@@ -546,6 +592,11 @@ def bake_colors(points4, sh32, sh_deg, center, attr):
 
 # ============================================================================ foam.cu (training renderer)
 
+# foam_backward allocates 16 bytes per record for its samples' gradients up to this many records (4 GiB); beyond that the
+# rays are replayed one by one.
+REPLAY_SAMPLES = 1 << 28
+
+
 class _FoamExtension:
 	@staticmethod
 	def _check_args(points, offsets, adj, raw, dA, cA, sh, o, d, start, near, far):
@@ -613,11 +664,16 @@ class _FoamExtension:
 			wb = work.numel()
 		else:
 			work = torch.empty(max(wb, 1), dtype=torch.uint8, device=dev)
+		scratch, sb = None, 0
+		if replay and rec.data_ptr() % 16 == 0 and 0 < B * K <= REPLAY_SAMPLES and B <= 1 << 22:
+			sb = int(_lib.load().vgr_foam_scratch_size(B, K))
+			scratch = torch.empty(sb, dtype=torch.uint8, device=dev)
 		with torch.cuda.device(dev):
-			call('vgr_foam_backward', ptr(points), n, ptr(offsets), ptr(adj), adj.numel(), ptr(raw), ptr(dA),
+			call('vgr_foam_backward_scratch', ptr(points), n, ptr(offsets), ptr(adj), adj.numel(), ptr(raw), ptr(dA),
 				 ptr(cA), ptr(sh), int(sh_deg), ptr(o), ptr(d), ptr(start), ptr(near), ptr(far), B, float(t_thresh),
 				 float(w_thresh), ptr(rgb), ptr(T), ptr(g_rgb), ptr(g_T), ptr(rec) if replay else None, K,
-				 ptr(stats) if replay else None, *[ptr(x) for x in g], int(ready), ptr(work), wb, stream_of(dev))
+				 ptr(stats) if replay else None, *[ptr(x) for x in g], int(ready), ptr(work), wb, ptr(scratch), sb,
+				 stream_of(dev))
 		return g
 
 
@@ -699,7 +755,7 @@ def _evaluate(op, args, params):
 	params = [p.contiguous() for p in params]
 	if torch.is_grad_enabled() and any(p.requires_grad for p in params):
 		return _Differentiable.apply(op, args, *params)
-	return op.forward([p.detach() for p in params], args)[0]
+	return getattr(op, 'infer', op.forward)([p.detach() for p in params], args)[0]
 
 
 class _DensityOp:
@@ -748,7 +804,8 @@ class _ConicOp:
 class _MarchOp:
 	"""params (raw, dA, cA, sh); args (graph, rays (o, d, start, near, mid, far), (sh_deg, dt, n_bg, t_thresh,
 	w_thresh)). Under autograd both passes run 16 lanes per ray, the faster layout for a training step at every batch
-	size measured, and share one workspace: the backward reuses the site blocks the forward packed."""
+	size measured, and share one workspace: the backward reuses the site blocks the forward packed, and replays the
+	runs of samples that the forward recorded."""
 	n_diff = 2
 
 	@staticmethod
@@ -757,15 +814,24 @@ class _MarchOp:
 		n = g.points.numel() // 3
 		work = torch.empty(max(int(_lib.load().vgr_march_backward_work_size(n, cfg[0])), 1), dtype=torch.uint8,
 						   device=g.points.device)
+		visits = march_visits(rays[0].size(0), g.points.device)
 		outs = march_extension().march_forward(g.points, g.offsets, g.adj, *p, cfg[0], *rays, *cfg[1:], lanes=16,
-											   work=work)
-		return tuple(outs), (), work
+											   work=work, visits=visits)
+		return tuple(outs), (), (work, visits)
 
 	@staticmethod
-	def backward(p, a, outs, extra, grads, work):
+	def infer(p, a):
+		"""Without gradients: the layout by batch size, no visit records and no gradient blocks."""
 		g, rays, cfg = a
+		return tuple(march_extension().march_forward(g.points, g.offsets, g.adj, *p, cfg[0], *rays, *cfg[1:])), (), None
+
+	@staticmethod
+	def backward(p, a, outs, extra, grads, state):
+		g, rays, cfg = a
+		work, visits = (None, None) if state is None else state
 		return march_extension().march_backward(g.points, g.offsets, g.adj, *p, cfg[0], *rays, *cfg[1:], outs[0],
-												outs[1], grads[0], grads[1], lanes=16, work=work)
+												outs[1], grads[0], grads[1], lanes=16, work=work, visits=visits,
+												stats=outs[3])
 
 
 class _FoamOp:
