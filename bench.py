@@ -53,13 +53,15 @@ def copy_probe(dev):
 
 
 def source_hash(*names):
-	"""16 hex digits of SHA-256 over the named kernel sources, the two headers every kernel includes and the hipcc
-	flags: it names the build a DRAM-traffic profile was measured on."""
+	"""16 hex digits of SHA-256 over the named kernel sources (foam_infer.hip: with the files its entry point launches
+	from and their header), the two headers every kernel includes and the hipcc flags: it names the build a DRAM-traffic
+	profile was measured on."""
 	import hashlib
 
 	from vgr import build
 	h = hashlib.sha256()
-	for n in sorted(set(names) | {'vgr_device.h', 'vgr_abi.h'}):
+	foam = {'foam_tile.hip', 'foam_wide.hip', 'vgr_foam.h'} if 'foam_infer.hip' in names else set()
+	for n in sorted(set(names) | foam | {'vgr_device.h', 'vgr_abi.h'}):
 		h.update(n.encode())
 		with open(os.path.join(build.CSRC, n), 'rb') as f:
 			h.update(f.read())
@@ -386,13 +388,14 @@ def bench_foam(args):
 	if row_kind is not None:
 		key += '-rows64' if pack['rows'].size(1) == 16 else '-blocks256'
 	src = source_hash('foam_infer.hip')
-	log(f'kernel source hash (foam_infer.hip): {src}; workload key {key}')
+	log(f'kernel source hash (foam_infer.hip and its kernels): {src}; workload key {key}')
+	tile = lanes == 1 and not args.eps_color > 0 and (mode == 2 or exact_blend)
 	roofline = hbm_roofline(ms, key, src, abytes,
 							'cache-oblivious gather bytes from the per-ray counters: 56 B per ray + 24 B per sample + '
 							f'{80 if indexed else 84} B per neighbourhood edge + SH bytes per distinct blended site '
 							'(counts every L1/L2/LDS hit as a fetch, so it can exceed the HBM peak)',
-							'foam_infer_kernel' if lanes == 1 else 'foam_group_kernel')
-	if roofline['frac'] is not None and not fast and (mode == 2 or exact_blend) and lanes == 1:
+							'foam_tile_kernel' if tile else 'foam_infer_kernel' if lanes == 1 else 'foam_group_kernel')
+	if roofline['frac'] is not None and tile:
 		roofline['limiter'] = ('not HBM: the texture data path is busy 94 % of the launch and the L2 serves 93 % of '
 							   'the gathers (profiles/foam_infer_config3_counters.md)')
 

@@ -11,9 +11,10 @@
 // are cached per wave in LDS (the tile's rays read mostly the same sites); colours are evaluated per lane.
 // A second layout, a group of 2, 4 or 8 lanes per ray (foam_group_kernel below), splits each cell's
 // neighbourhood over the group's lanes; it is the faster one for traversal, density and lazy colours, one ray per
-// lane for fused and baked colours (default_lanes).
+// lane for fused and baked colours (default_lanes). Two more layouts have files of their own: small batches run 16 lanes
+// per ray (foam_wide.hip, the rule at kWideRays), fused and exact colours without a cut-off evaluate a wave's samples by
+// cell (foam_tile.hip, the rule in foam_entry).
 #include <cmath>
-#include <type_traits>
 
 #include "vgr_foam.h"
 
@@ -331,45 +332,6 @@ __device__ __forceinline__ int table_hits(const FoamScene& S, int c, int g, Slot
     return hits;
 }
 
-// One ray per lane with fused colours (one pass per sample): the cells of the passes whose cache hits are still to
-// be counted, and the ray's 8 tags, in the lane's private memory (the log is written at a varying index, so it and
-// the tags stay out of registers); every kPassLog passes, and at the end of the ray, the logged passes are counted
-// in order with the tags in registers for the while. Measured on config 3 against the tags in registers: 179.4 and
-// 179.3 ms (16 and 32 passes) against 179.8, 24 spilled VGPRs against 44; 64 passes 208.9 ms; for exact colours,
-// whose passes follow the samples' weights, 227.4 against 182.8 ms, so they keep the tags in registers.
-constexpr int kPassLog = 16;
-struct PassLog {
-    int mem[kPassLog + kRayTagSlots];  // cells of the logged passes, then the tags
-    int n;
-};
-
-__device__ __forceinline__ int log_flush(const FoamScene& S, PassLog& L) {
-    SlotTags<1> T;
-#pragma unroll
-    for (int s = 0; s < kRayTagSlots; ++s) T.t[s] = L.mem[kPassLog + s];
-    int hits = 0;
-    for (int i = 0; i < L.n; ++i) hits += table_hits<1>(S, L.mem[i], 0, T);
-#pragma unroll
-    for (int s = 0; s < kRayTagSlots; ++s) L.mem[kPassLog + s] = T.t[s];
-    L.n = 0;
-    return hits;
-}
-
-// The slot-table count of one ray per lane, with the tags behind a pass log (above) or in registers: set-up, a pass
-// over cell c that looked up every entry (returns the hits counted now: all of the log's when it fills up), and the
-// end of the ray (the hits not counted yet).
-__device__ __forceinline__ void tags_init(PassLog& L) {
-    L.n = 0;
-#pragma unroll
-    for (int s = 0; s < kRayTagSlots; ++s) L.mem[kPassLog + s] = -1;
-}
-__device__ __forceinline__ int tags_pass(const FoamScene& S, PassLog& L, int c) {
-    L.mem[L.n] = c;
-    return ++L.n == kPassLog ? log_flush(S, L) : 0;
-}
-__device__ __forceinline__ int tags_finish(const FoamScene& S, PassLog& L) { return log_flush(S, L); }
-__device__ __forceinline__ int tags_pass(const FoamScene& S, SlotTags<1>& T, int c) { return table_hits<1>(S, c, 0, T); }
-__device__ __forceinline__ int tags_finish(const FoamScene&, SlotTags<1>&) { return 0; }
 
 // Greedy walk to the lexicographic argmin of (|x - p|^2, tie order) over {c} U adj(c), repeated. IDX: the edge
 // records carry the neighbour index (indexed pack).
@@ -451,7 +413,7 @@ __device__ __forceinline__ SiteRec site_rec(const FoamScene& S, int k) {
 // Mahalanobis distance (lazy) or running colour blend (fused, baked), and, when want_exit, the exit face.
 // Pipelined (Tune): the edge record of e + 2 and the site records of e + 1 are loaded while edge e is evaluated,
 // indices clamped to the cell so every load stays in bounds.
-template <int STAGE, int COLOR, bool HALF, int DEG, bool TABLE>
+template <int STAGE, int COLOR, bool HALF, int DEG>
 __device__ void eval_cell(const FoamScene& S, const FoamParams& P, int c, float t, const float (&o)[3],
                           const float (&d)[3], const float (&b)[16], ColorCache<COLOR>& cache,
                           bool want_exit, CellEval& R, int& n_dens, int& n_sh) {
@@ -528,8 +490,7 @@ __device__ void eval_cell(const FoamScene& S, const FoamParams& P, int c, float 
                                 const float4 q4 = S.attr[5 * static_cast<int64_t>(k) + 4];
                                 c3[0] = q4.x, c3[1] = q4.y, c3[2] = q4.z;
                             } else {
-                                if constexpr (TABLE) ++n_sh;  // the pass's hits come off in table_hits
-                                else n_sh += ray_tag_miss(cache, k);
+                                n_sh += ray_tag_miss(cache, k);
                                 cached_colour<HALF, sh_vec4<HALF, DEG>()>(cache, S.sh, HALF ? 6 : 12, k, b, c3);
                             }
                             blend_add(R.B, m, c3[0], c3[1], c3[2]);
@@ -600,21 +561,12 @@ __device__ void color_lazy(const FoamScene& S, const FoamParams& P, int c, float
 // spills: 80 VGPRs, the rest of the ray's state (accumulated colour and depth, the basis) stored to scratch once
 // per sample, outside the neighbourhood loop; at 4 waves it needs no spills and ran 27 % slower, at 7 it spills
 // inside the loop.
-//
-// EXACT (fused colour modes, colour cut-off +inf, slot table): the exact (lazy) colour mode run by the one-pass blend.
-// The exact colour of a sample is sum_k exp(-(m_k - m_min) / 2) c_k / sum_k exp(-(m_k - m_min) / 2) over every
-// neighbour (the cut-off is +inf); the blend keeps the same two sums relative to the running minimum, rescaled as
-// it falls, so the colours agree to rounding. The statistics are the exact mode's: a colour pass counts only where
-// the exact mode runs one (segments with weight > w_thresh, for the segment's far sample and, when the segment
-// before was not coloured, its near sample), with that pass's lookups (every entry, as the blend's pass looks up)
-// and the ray's cache tags advanced by those passes alone.
-template <int STAGE, int COLOR, bool HALF, int DEG, bool TRACE, bool TABLE, bool EXACT = false>
+template <int STAGE, int COLOR, bool HALF, int DEG, bool TRACE, bool TABLE>
 __global__ void __launch_bounds__(kBlock, (waves_for<COLOR, kBlock, TABLE>(STAGE >= 2 && COLOR != kBaked)))
     foam_infer_kernel(FoamScene S, FoamParams P, FoamRays R, FoamOut O) {
-    static_assert(!EXACT || (TABLE && STAGE == 2 && (COLOR == kFused || COLOR == kFusedIdx)), "exact via the blend");
+    static_assert(!TABLE || COLOR == kLazy, "a blend without a cut-off runs in foam_tile.hip");
     constexpr bool kSH = STAGE >= 2 && COLOR != kBaked;
     constexpr bool BLEND = STAGE >= 2 && COLOR != kLazy;
-    constexpr bool FUSED_SH = BLEND && COLOR != kBaked;
     __shared__ float4 cache_lds[cache_vec4<COLOR, kBlock, TABLE>(kSH)];
     ColorCache<COLOR> cache{};  // set up by every lane of the block before any returns
     if (kSH) cache = make_cache<COLOR, kBlock, TABLE>(cache_lds, static_cast<int>(threadIdx.x));
@@ -640,16 +592,12 @@ __global__ void __launch_bounds__(kBlock, (waves_for<COLOR, kBlock, TABLE>(STAGE
     if (kSH) sh_basis(d[0], d[1], d[2], DEG, b);
 
     int walk_steps = 0, n_dens = 0, n_sh = 0;
-    std::conditional_t<TABLE && FUSED_SH && !EXACT, PassLog, SlotTags<1>> tags;
+    SlotTags<1> tags;
     tags_init(tags);
     int c = walk_to<COLOR == kFusedIdx>(S, start, o[0] + t_near * d[0], o[1] + t_near * d[1], o[2] + t_near * d[2],
                                         walk_steps);
     CellEval E;
-    int looks = 0, looksP = 0;  // EXACT: lookups of the latest pass and of the one before
-    bool litP = false;          // EXACT: the segment ending at the near sample was coloured
-    eval_cell<STAGE, COLOR, HALF, DEG, TABLE>(S, P, c, t_near, o, d, b, cache, true, E, n_dens,
-                                              EXACT ? looks : n_sh);
-    if (TABLE && FUSED_SH && !EXACT) n_sh -= tags_pass(S, tags, c);
+    eval_cell<STAGE, COLOR, HALF, DEG>(S, P, c, t_near, o, d, b, cache, true, E, n_dens, n_sh);
     trace_cell<TRACE>(S, O, r, 0, c);
     float sP = E.sigma, mP = E.mmin, tP = t_near, CP[3] = {0.f, 0.f, 0.f};
     bool hasP = false;
@@ -664,10 +612,7 @@ __global__ void __launch_bounds__(kBlock, (waves_for<COLOR, kBlock, TABLE>(STAGE
         const bool last = E.next == INT_MAX || E.t_exit >= t_far || n_samples + 1 >= max_samples;
         const float tQ = last ? t_far : fmaxf(E.t_exit, tP);
         const int cQ = last ? c : E.next;
-        looksP = looks, looks = 0;
-        eval_cell<STAGE, COLOR, HALF, DEG, TABLE>(S, P, cQ, tQ, o, d, b, cache, !last, E, n_dens,
-                                                  EXACT ? looks : n_sh);
-        if (TABLE && FUSED_SH && !EXACT) n_sh -= tags_pass(S, tags, cQ);
+        eval_cell<STAGE, COLOR, HALF, DEG>(S, P, cQ, tQ, o, d, b, cache, !last, E, n_dens, n_sh);
         trace_cell<TRACE>(S, O, r, n_samples, cQ);
         ++n_samples;
         const float sQ = E.sigma, mQ = E.mmin;
@@ -682,17 +627,13 @@ __global__ void __launch_bounds__(kBlock, (waves_for<COLOR, kBlock, TABLE>(STAGE
         }
         const bool lit = STAGE >= 2 && w > P.w_thresh;
         if (lit) {
-            if constexpr (EXACT) {
-                if (!litP) n_sh += looksP - tags_pass(S, tags, cP);
-                n_sh += looks - tags_pass(S, tags, cQ);
-            }
             if constexpr (!BLEND) {
                 if (!hasP) {
                     color_lazy<HALF, DEG, TABLE>(S, P, cP, tP, mP, o, d, b, cache, CP, n_sh);
-                    if (TABLE) n_sh -= tags_pass(S, tags, cP);
+                    if (TABLE) n_sh -= table_hits<1>(S, cP, 0, tags);
                 }
                 color_lazy<HALF, DEG, TABLE>(S, P, cQ, tQ, mQ, o, d, b, cache, CQ, n_sh);
-                if (TABLE) n_sh -= tags_pass(S, tags, cQ);
+                if (TABLE) n_sh -= table_hits<1>(S, cQ, 0, tags);
                 hasQ = true;
             }
 #pragma unroll
@@ -701,12 +642,11 @@ __global__ void __launch_bounds__(kBlock, (waves_for<COLOR, kBlock, TABLE>(STAGE
             ++n_color;
         }
         T *= 1.f - alpha;
-        tP = tQ, sP = sQ, mP = mQ, hasP = hasQ, cP = cQ, c = cQ, litP = lit;
+        tP = tQ, sP = sQ, mP = mQ, hasP = hasQ, cP = cQ, c = cQ;
 #pragma unroll
         for (int a = 0; a < 3; ++a) CP[a] = CQ[a];
         if (last || T < P.t_thresh) break;
     }
-    if (TABLE && kSH) n_sh -= tags_finish(S, tags);
 #pragma unroll
     for (int a = 0; a < 3; ++a) O.rgb[3 * r + a] = acc[a];
     O.T[r] = T;
@@ -1049,15 +989,15 @@ __global__ void __launch_bounds__(256) index_pack_kernel(const int* __restrict__
     }
 }
 
-// The fused blend over the indexed edge records: one ray per lane (EXACT: the exact colour mode's statistics).
-template <bool HALF, bool TRACE, bool TABLE, bool EXACT>
+// The fused blend with a finite cut-off over the indexed edge records: one ray per lane.
+template <bool HALF, bool TRACE>
 int launch_indexed(const FoamScene& S, const FoamParams& P, const FoamRays& R, const FoamOut& O, hipStream_t stream) {
     const dim3 grid(grid_for(R.n, kBlock)), block(kBlock);
     switch (P.sh_deg) {
-        case 0: hipLaunchKernelGGL((foam_infer_kernel<2, kFusedIdx, HALF, 0, TRACE, TABLE, EXACT>), grid, block, 0, stream, S, P, R, O); break;
-        case 1: hipLaunchKernelGGL((foam_infer_kernel<2, kFusedIdx, HALF, 1, TRACE, TABLE, EXACT>), grid, block, 0, stream, S, P, R, O); break;
-        case 2: hipLaunchKernelGGL((foam_infer_kernel<2, kFusedIdx, HALF, 2, TRACE, TABLE, EXACT>), grid, block, 0, stream, S, P, R, O); break;
-        default: hipLaunchKernelGGL((foam_infer_kernel<2, kFusedIdx, HALF, 3, TRACE, TABLE, EXACT>), grid, block, 0, stream, S, P, R, O);
+        case 0: hipLaunchKernelGGL((foam_infer_kernel<2, kFusedIdx, HALF, 0, TRACE, false>), grid, block, 0, stream, S, P, R, O); break;
+        case 1: hipLaunchKernelGGL((foam_infer_kernel<2, kFusedIdx, HALF, 1, TRACE, false>), grid, block, 0, stream, S, P, R, O); break;
+        case 2: hipLaunchKernelGGL((foam_infer_kernel<2, kFusedIdx, HALF, 2, TRACE, false>), grid, block, 0, stream, S, P, R, O); break;
+        default: hipLaunchKernelGGL((foam_infer_kernel<2, kFusedIdx, HALF, 3, TRACE, false>), grid, block, 0, stream, S, P, R, O);
     }
     return launch_status("foam_infer_kernel (indexed edges)");
 }
@@ -1082,8 +1022,9 @@ int launch(const FoamScene& S, const FoamParams& P, const FoamRays& R, const Foa
                            dim3(grid_for(R.n, kBlock / 8)), dim3(kBlock), 0, stream, S, P, R, O);
         return launch_status("foam_group_kernel");
     }
-    hipLaunchKernelGGL((foam_infer_kernel<STAGE, COLOR, HALF, DEG, TRACE, TABLE>), dim3(grid_for(R.n, kBlock)),
-                       dim3(kBlock), 0, stream, S, P, R, O);
+    // TABLE says that the cut-off is +inf: such a fused blend with one ray per lane runs in foam_tile.hip
+    hipLaunchKernelGGL((foam_infer_kernel<STAGE, COLOR, HALF, DEG, TRACE, TABLE && COLOR == kLazy>),
+                       dim3(grid_for(R.n, kBlock)), dim3(kBlock), 0, stream, S, P, R, O);
     return launch_status("foam_infer_kernel");
 }
 
@@ -1118,19 +1059,6 @@ int dispatch(int stage, int color_mode, bool half, const FoamScene& S, const Foa
                     : launch_sh<kLazy, false, TRACE>(S, P, R, O, lanes, table, stream);
     return half ? launch_sh<kFused, true, TRACE>(S, P, R, O, lanes, table, stream)
                 : launch_sh<kFused, false, TRACE>(S, P, R, O, lanes, table, stream);
-}
-
-template <bool HALF>
-int dispatch_indexed(bool trace, bool table, bool exact, const FoamScene& S, const FoamParams& P, const FoamRays& R,
-                     const FoamOut& O, hipStream_t s) {
-    if (exact)  // always with the slot table
-        return trace ? launch_indexed<HALF, true, true, true>(S, P, R, O, s)
-                     : launch_indexed<HALF, false, true, true>(S, P, R, O, s);
-    if (trace)
-        return table ? launch_indexed<HALF, true, true, false>(S, P, R, O, s)
-                     : launch_indexed<HALF, true, false, false>(S, P, R, O, s);
-    return table ? launch_indexed<HALF, false, true, false>(S, P, R, O, s)
-                 : launch_indexed<HALF, false, false, false>(S, P, R, O, s);
 }
 
 // Slot table of the reference's per-ray colour cache: for site k, the first and the last entry of every slot
@@ -1172,19 +1100,17 @@ inline int default_lanes(int64_t stage, int64_t color_mode) {
     return stage < 2 || color_mode == kLazy ? 4 : 1;
 }
 
-// Below this many rays the default layout of the full rendering (stage 2) is 16 lanes per ray (foam_wide.hip): one ray
+// Up to this many rays the default layout of the full rendering (stage 2) is 16 lanes per ray (foam_wide.hip): one ray
 // per lane, or four lanes, leaves a launch as long as its longest ray's chain of dependent reads, whatever its size.
 // Measured on a scene of 131k sites with large cells (90 samples per ray) and one of 1M (160 samples), 8x8 tiles, ms of
 // the render call, 16 lanes against the other layout:
-//   exact and fused colours, fp32 SH  8192 rays 0.65 : 9.9, 1.1 : 23.7; 131072 6.8 : 7.4, 8.9 : 20.0; 262144 10.1 : 8.3,
-//                                     14.0 : 21.4
+//   exact and fused colours, fp32 SH  8192 rays 0.66 : 2.8, 1.1 : 7.1; 65536 2.8 : 2.5, 4.0 : 7.1; 131072 6.8 : 2.8,
+//   (foam_tile.hip)                   8.8 : 6.3 (rows of pixels instead of tiles: 3.9 : 7.2, 7.4 : 10.6)
 //   baked colours                     8192 rays 0.53 : 1.83, 1.09 : 4.3; 65536 1.33 : 1.92, 2.4 : 5.0; 131072 2.7 : 2.1,
 //                                     4.2 : 5.2
 //   exact with a finite cut-off       65536 rays 2.7 : 3.6, 3.8 : 8.7; 131072 6.5 : 5.4, 8.5 : 11.8
-// The lines lie where the worse of the two scenes breaks even.
-inline int64_t wide_rays(int64_t color_mode, bool finite_cut) {
-    return color_mode == kBaked || (color_mode == kLazy && finite_cut) ? 98304 : 131072;
-}
+// The line lies between the sizes where the two scenes break even, for each of them.
+constexpr int64_t kWideRays = 98304;
 
 int foam_entry(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t* nbr, const float* edge,
                int64_t n_edges, const float* attr, const void* sh, int32_t sh_half, int64_t sh_deg, const float* o,
@@ -1196,13 +1122,13 @@ int foam_entry(const float* points, int64_t n_sites, const int32_t* offsets, con
                const float* rows = nullptr, int64_t row_floats = 16) {
     VGR_REQUIRE(n_rays >= 0, "foam_infer: n_rays must be >= 0 (got %lld)", static_cast<long long>(n_rays));
     // The indexed edge records serve the fused blend with one ray per lane (its default layout), and with the slot
-    // table and the colour cut-off +inf the exact colours too, run by that blend (foam_infer_kernel, EXACT).
+    // table and the colour cut-off +inf the exact colours too, run by that blend (foam_tile.hip).
     const bool one_lane = lanes == kDefaultLanes || lanes == 1;
     const bool exact_blend = edge_i != nullptr && attr_i != nullptr && slots != nullptr && stage == 2 &&
                              color_mode == kLazy && one_lane && std::isinf(color_cut) && color_cut > 0;
     const bool indexed = exact_blend || (edge_i != nullptr && attr_i != nullptr && stage == 2 &&
                                          color_mode == kFused && one_lane);
-    const bool wide = lanes == kDefaultLanes && stage == 2 && n_rays <= wide_rays(color_mode, !(std::isinf(color_cut) && color_cut > 0));
+    const bool wide = lanes == kDefaultLanes && stage == 2 && n_rays <= kWideRays;
     if (indexed) lanes = 1;
     if (lanes == kDefaultLanes) lanes = default_lanes(stage, color_mode);
     VGR_REQUIRE(lanes == 1 || lanes == 2 || lanes == 4 || lanes == 8,
@@ -1229,6 +1155,10 @@ int foam_entry(const float* points, int64_t n_sites, const int32_t* offsets, con
     // Fused and baked blends with a finite colour cut skip a neighbour against the running minimum of the terms
     // before it in edge order; a lane of a group sees only its own share of them, so these run one ray per lane.
     if (stage == 2 && color_mode != kLazy && !(color_cut > 1e30)) lanes = 1;
+    // Without a cut-off no colour decides which other one is looked up, so one ray per lane queues its samples and
+    // evaluates them by cell (foam_tile.hip); with a finite one the running minimum does, and the lookup runs in the pass.
+    const bool tile =
+        stage == 2 && lanes == 1 && std::isinf(color_cut) && color_cut > 0 && (indexed || color_mode == kFused);
     // The site rows serve the group layouts' fused blend (config 5's 8-lane batch: 2538.6 -> 2437.6 ms with the
     // 64-byte rows); the two-pass exact colours with 4 lanes per ray ran slower on them (268.9 against 258.3 ms on
     // config 3) and keep the attr rows, as the one-ray-per-lane kernels do. Site blocks also supply those kernels'
@@ -1261,9 +1191,12 @@ int foam_entry(const float* points, int64_t n_sites, const int32_t* offsets, con
     // 256 bytes of LDS per wave there: config 5's batch ran 2437.6 ms with the table, 2298.0 ms with the tags.
     const bool table = slots != nullptr && std::isinf(color_cut) && color_cut > 0 && lanes != 8;
     if (wide) return launch_foam_wide(S, P, R, O, int(color_mode), sh_half != 0, s);
-    if (indexed)
-        return sh_half != 0 ? dispatch_indexed<true>(trace != nullptr, table, exact_blend, S, P, R, O, s)
-                            : dispatch_indexed<false>(trace != nullptr, table, exact_blend, S, P, R, O, s);
+    if (tile) return launch_foam_tile(S, P, R, O, indexed, exact_blend, sh_half != 0, s);
+    if (indexed) {
+        if (sh_half != 0)
+            return trace != nullptr ? launch_indexed<true, true>(S, P, R, O, s) : launch_indexed<true, false>(S, P, R, O, s);
+        return trace != nullptr ? launch_indexed<false, true>(S, P, R, O, s) : launch_indexed<false, false>(S, P, R, O, s);
+    }
     if (trace != nullptr)
         return dispatch<true>(int(stage), int(color_mode), sh_half != 0, S, P, R, O, int(lanes), table, s);
     return dispatch<false>(int(stage), int(color_mode), sh_half != 0, S, P, R, O, int(lanes), table, s);

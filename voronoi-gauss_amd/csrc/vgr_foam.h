@@ -54,6 +54,11 @@ struct FoamOut {
 int launch_foam_wide(const FoamScene& S, const FoamParams& P, const FoamRays& R, const FoamOut& O, int color_mode,
                      bool half, hipStream_t stream);
 
+// Fused colours (exact: the exact colour mode's statistics) with the colour cut-off +inf, one ray per lane, colours evaluated
+// cell by cell on the matrix cores (foam_tile.hip). indexed: S.edge and S.attr are the indexed records.
+int launch_foam_tile(const FoamScene& S, const FoamParams& P, const FoamRays& R, const FoamOut& O, bool indexed, bool exact,
+                     bool half, hipStream_t stream);
+
 namespace {
 
 // Running normalised colour blend (fused / baked modes).
