@@ -1,4 +1,4 @@
-"""The inference renderer's one-ray-per-lane layout for colours without a cut-off (samples queued per ray, evaluated cell by
+"""The inference renderer's one-ray-per-lane layout of fused and exact colours (samples queued per ray, evaluated cell by
 cell) against the oracle and the group layout: T, traces and statistics bit-identical to the latter, rgb to rounding, at the
 sizes and neighbourhoods where it branches: partial and several waves, neighbourhoods that are and are not multiples of four
 and far beyond, rays whose queues fill at different times, no lit sample at all."""
@@ -28,13 +28,14 @@ def hub(gpu):
 	return f, f.rays(B=257, seed=11)
 
 
-def run(dev, pk, deg, rays, tt, wt, mode, lanes=1, indexed=False, slots=False, cap=None, order=None, trace_cap=512):
+def run(dev, pk, deg, rays, tt, wt, mode, lanes=1, indexed=False, slots=False, cap=None, order=None, trace_cap=512,
+		cut=math.inf):
 	t = lambda a: torch.as_tensor(np.ascontiguousarray(a), device=dev)  # noqa: E731
 	empty = torch.empty(0, dtype=torch.int32, device=dev)
 	scene = [t(pk[k]) for k in ('points', 'offsets', 'nbr', 'edge', 'attr', 'sh')]
 	orig = pk.get('orig')
 	out = ext.foam_infer_extension().foam_infer(
-		*scene, deg, *(t(a) for a in rays), tt, wt, math.inf, mode, 2, empty if cap is None else t(cap),
+		*scene, deg, *(t(a) for a in rays), tt, wt, cut, mode, 2, empty if cap is None else t(cap),
 		t(orig) if orig is not None and len(orig) else empty, trace_cap=trace_cap, lanes=lanes,
 		order=None if order is None else t(order), indexed=ext.index_pack(*scene[1:5]) if indexed else None,
 		slots=ext.slot_table(scene[1], scene[2]) if slots else None)
@@ -87,3 +88,23 @@ def test_tile_layout_degrees_orders_and_caps(gpu, hub, sh_deg, sh_half):
 		for k in g:
 			np.testing.assert_array_equal(h[k].view(np.int32), g[k].view(np.int32), err_msg=k)
 		assert (g['T'][:3] == 1).all() and (g['rgb'][:3] == 0).all() and (g['stats'][:3] == 0).all()
+
+
+@pytest.mark.parametrize('n_rays', [1, 65, 257])
+@pytest.mark.parametrize('indexed', [False, True])
+@pytest.mark.parametrize('sh_half', [False, True])
+@pytest.mark.parametrize('cut', [0.0, 2.0, 2 * math.log(1e3)])
+def test_tile_layout_cut_off(gpu, hub, n_rays, indexed, sh_half, cut):
+	"""A finite cut-off admits a term against the running minimum of the terms before it: the counted lookups and the
+	colours against the oracle and the 16-lane layout, which decide the same way in the same order."""
+	f, (o, d, start, near, _, far) = hub
+	rays = tuple(a[:n_rays] for a in (o, d, start, near, far))
+	pk = f.pack(eps_density=1e-3, sh_half=sh_half)
+	for tt, wt in ((0.0, -1.0), (1e-4, 0.05)):
+		g = run(gpu, pk, 3, rays, tt, wt, 2, indexed=indexed, cut=cut)
+		wide = run(gpu, pk, 3, rays, tt, wt, 2, lanes=None, cut=cut)
+		for k in ('T', 'stats', 'trace'):
+			np.testing.assert_array_equal(g[k].view(np.int32), wide[k].view(np.int32), err_msg=k)
+		np.testing.assert_allclose(g['rgb'], wide['rgb'], atol=1e-5, rtol=0)  # as in check
+		r = ref_foam(pk, 3, *rays, tt, wt, color_cut=cut, color_mode=2, trace_cap=512)
+		compare(g, r, exact_trace=tt == 0.0, stats_frac=0.98, w_thresh=max(wt, 1e-4))

@@ -12,8 +12,8 @@
 // A second layout, a group of 2, 4 or 8 lanes per ray (foam_group_kernel below), splits each cell's
 // neighbourhood over the group's lanes; it is the faster one for traversal, density and lazy colours, one ray per
 // lane for fused and baked colours (default_lanes). Two more layouts have files of their own: small batches run 16 lanes
-// per ray (foam_wide.hip, the rule at kWideRays), fused and exact colours without a cut-off evaluate a wave's samples by
-// cell (foam_tile.hip, the rule in foam_entry).
+// per ray (foam_wide.hip, the rule at kWideRays); fused colours with one ray per lane, and exact ones run by that blend,
+// evaluate a wave's samples by cell (foam_tile.hip).
 #include <cmath>
 
 #include "vgr_foam.h"
@@ -22,11 +22,6 @@ namespace vgr {
 namespace {
 
 constexpr int kBlock = 64;  // one wave64 per workgroup = one 8x8 ray tile
-// Fused colours over the indexed edge records (vgr_foam_index_pack): the neighbour's index in the fourth word of its
-// edge record and its cut-off word in attr[:, 7], so a neighbour round loads no separate index. An internal mode of
-// this file: it blends exactly as kFused.
-constexpr int kFusedIdx = 3;
-
 // ------------------------------------------------------------------ traversal arithmetic (never contracted)
 
 // Colour blocks of site k for this ray come through the wave-shared LDS cache of SH coefficient blocks: SLOTS
@@ -332,10 +327,7 @@ __device__ __forceinline__ int table_hits(const FoamScene& S, int c, int g, Slot
     return hits;
 }
 
-
-// Greedy walk to the lexicographic argmin of (|x - p|^2, tie order) over {c} U adj(c), repeated. IDX: the edge
-// records carry the neighbour index (indexed pack).
-template <bool IDX = false>
+// Greedy walk to the lexicographic argmin of (|x - p|^2, tie order) over {c} U adj(c), repeated.
 __device__ int walk_to(const FoamScene& S, int c, float x0, float x1, float x2, int& steps) {
     for (int it = 0; it < kWalkCap; ++it) {
         const float4 pc = S.points[c];
@@ -344,7 +336,7 @@ __device__ int walk_to(const FoamScene& S, int c, float x0, float x1, float x2, 
         const int e0 = S.offsets[c], e1 = S.offsets[c + 1];
         for (int e = e0 + 1; e < e1; ++e) {
             const float4 ed = S.edge[e];
-            const int k = IDX ? __float_as_int(ed.w) : S.nbr[e];
+            const int k = S.nbr[e];
             const float v0 = x0 - ed.x, v1 = x1 - ed.y, v2 = x2 - ed.z;
             const float dk = v0 * v0 + v1 * v1 + v2 * v2;
             if (dk < bd || (dk == bd && before(S, k, bk))) bd = dk, bk = k;
@@ -413,28 +405,13 @@ __device__ __forceinline__ SiteRec site_rec(const FoamScene& S, int k) {
 // Mahalanobis distance (lazy) or running colour blend (fused, baked), and, when want_exit, the exit face.
 // Pipelined (Tune): the edge record of e + 2 and the site records of e + 1 are loaded while edge e is evaluated,
 // indices clamped to the cell so every load stays in bounds.
-template <int STAGE, int COLOR, bool HALF, int DEG>
+template <int STAGE, int COLOR>
 __device__ void eval_cell(const FoamScene& S, const FoamParams& P, int c, float t, const float (&o)[3],
-                          const float (&d)[3], const float (&b)[16], ColorCache<COLOR>& cache,
-                          bool want_exit, CellEval& R, int& n_dens, int& n_sh) {
+                          const float (&d)[3], bool want_exit, CellEval& R, int& n_dens) {
     constexpr bool BLEND = STAGE >= 2 && COLOR != kLazy;
-    // Fused blend: the edge record of e + 1 (and, on the reference records, its neighbour index) is requested in
-    // round e, after the density term and before the colour lookup, whose latency then covers it; round e + 1
-    // starts with its neighbour index in hand. (Issued at the top of the round it spills the loop's registers; at
-    // its end it arrives too late to help. Baked colours, with no lookup to cover it, run slower with it.) The
-    // first record requested is the cell's own (self-first), which holds its position: on the reference records
-    // the cell position is taken from it (fewer spilled VGPRs there; on the indexed records the separate load is
-    // faster).
-    constexpr bool IDX = COLOR == kFusedIdx, PREF = STAGE >= 2 && (COLOR == kFused || IDX);
     const int e0 = S.offsets[c], e1 = S.offsets[c + 1];
     const int last = e1 - 1;
-    float4 edn;
-    int kn = 0;
-    if constexpr (PREF) {
-        edn = S.edge[entry_in(e0, e1)];
-        if constexpr (!IDX) kn = S.nbr[entry_in(e0, e1)];
-    }
-    const float4 pc = PREF && !IDX ? edn : S.points[c];
+    const float4 pc = S.points[c];
     float x[3];
     sample_point(o, d, t, x);
     R.sigma = 0.f, R.mmin = kInf, R.t_exit = kInf, R.next = INT_MAX;
@@ -457,9 +434,6 @@ __device__ void eval_cell(const FoamScene& S, const FoamParams& P, int c, float 
             const int e2 = min(e + 2, last);
             ed2 = S.edge[e2], k2 = S.nbr[e2];
             qn = site_rec<STAGE>(S, k1);
-        } else if constexpr (PREF) {
-            ed = edn, k = IDX ? __float_as_int(ed.w) : kn;
-            q = site_rec<STAGE>(S, k);
         } else {
             ed = S.edge[e], k = S.nbr[e];
             q = site_rec<STAGE>(S, k);
@@ -468,15 +442,10 @@ __device__ void eval_cell(const FoamScene& S, const FoamParams& P, int c, float 
         if (STAGE >= 1) {
             float v0, v1, v2, r2;
             offset_of(x, ed, v0, v1, v2, r2);
-            const float2 cut = cutoffs(COLOR == kFusedIdx ? q.q1.w : ed.w);
+            const float2 cut = cutoffs(ed.w);
             if (r2 <= cut.x) {
                 R.sigma += density_term(q.q0, q.q1, v0, v1, v2);
                 ++n_dens;
-            }
-            if constexpr (PREF) {
-                const int en = min(e + 1, last);
-                edn = S.edge[en];
-                if constexpr (!IDX) kn = S.nbr[en];
             }
             if (STAGE >= 2) {
                 const float lb = r2 * cut.y;
@@ -485,15 +454,8 @@ __device__ void eval_cell(const FoamScene& S, const FoamParams& P, int c, float 
                     if (lb <= lim) {
                         const float m = maha_f(q.q2, q.q3, v0, v1, v2);
                         if (m <= lim) {
-                            float c3[3];
-                            if (COLOR == kBaked) {
-                                const float4 q4 = S.attr[5 * static_cast<int64_t>(k) + 4];
-                                c3[0] = q4.x, c3[1] = q4.y, c3[2] = q4.z;
-                            } else {
-                                n_sh += ray_tag_miss(cache, k);
-                                cached_colour<HALF, sh_vec4<HALF, DEG>()>(cache, S.sh, HALF ? 6 : 12, k, b, c3);
-                            }
-                            blend_add(R.B, m, c3[0], c3[1], c3[2]);
+                            const float4 q4 = S.attr[5 * static_cast<int64_t>(k) + 4];
+                            blend_add(R.B, m, q4.x, q4.y, q4.z);
                         }
                     }
                 } else if (lb < R.mmin) {
@@ -557,6 +519,7 @@ __device__ void color_lazy(const FoamScene& S, const FoamParams& P, int c, float
 }
 
 // The register allocation is bounded for waves_for waves per SIMD (Tune<COLOR>::waves unless the LDS allows fewer).
+// The fused figures below and in Tune were taken with this kernel; one ray per lane runs them in foam_tile.hip now.
 // Six waves per SIMD is the fastest occupancy measured for the fused fp32 degree-3 kernel on config 3 although it
 // spills: 80 VGPRs, the rest of the ray's state (accumulated colour and depth, the basis) stored to scratch once
 // per sample, outside the neighbourhood loop; at 4 waves it needs no spills and ran 27 % slower, at 7 it spills
@@ -564,7 +527,7 @@ __device__ void color_lazy(const FoamScene& S, const FoamParams& P, int c, float
 template <int STAGE, int COLOR, bool HALF, int DEG, bool TRACE, bool TABLE>
 __global__ void __launch_bounds__(kBlock, (waves_for<COLOR, kBlock, TABLE>(STAGE >= 2 && COLOR != kBaked)))
     foam_infer_kernel(FoamScene S, FoamParams P, FoamRays R, FoamOut O) {
-    static_assert(!TABLE || COLOR == kLazy, "a blend without a cut-off runs in foam_tile.hip");
+    static_assert(COLOR != kFused && (!TABLE || COLOR == kLazy), "fused colours: foam_tile.hip");
     constexpr bool kSH = STAGE >= 2 && COLOR != kBaked;
     constexpr bool BLEND = STAGE >= 2 && COLOR != kLazy;
     __shared__ float4 cache_lds[cache_vec4<COLOR, kBlock, TABLE>(kSH)];
@@ -594,10 +557,10 @@ __global__ void __launch_bounds__(kBlock, (waves_for<COLOR, kBlock, TABLE>(STAGE
     int walk_steps = 0, n_dens = 0, n_sh = 0;
     SlotTags<1> tags;
     tags_init(tags);
-    int c = walk_to<COLOR == kFusedIdx>(S, start, o[0] + t_near * d[0], o[1] + t_near * d[1], o[2] + t_near * d[2],
+    int c = walk_to(S, start, o[0] + t_near * d[0], o[1] + t_near * d[1], o[2] + t_near * d[2],
                                         walk_steps);
     CellEval E;
-    eval_cell<STAGE, COLOR, HALF, DEG>(S, P, c, t_near, o, d, b, cache, true, E, n_dens, n_sh);
+    eval_cell<STAGE, COLOR>(S, P, c, t_near, o, d, true, E, n_dens);
     trace_cell<TRACE>(S, O, r, 0, c);
     float sP = E.sigma, mP = E.mmin, tP = t_near, CP[3] = {0.f, 0.f, 0.f};
     bool hasP = false;
@@ -612,7 +575,7 @@ __global__ void __launch_bounds__(kBlock, (waves_for<COLOR, kBlock, TABLE>(STAGE
         const bool last = E.next == INT_MAX || E.t_exit >= t_far || n_samples + 1 >= max_samples;
         const float tQ = last ? t_far : fmaxf(E.t_exit, tP);
         const int cQ = last ? c : E.next;
-        eval_cell<STAGE, COLOR, HALF, DEG>(S, P, cQ, tQ, o, d, b, cache, !last, E, n_dens, n_sh);
+        eval_cell<STAGE, COLOR>(S, P, cQ, tQ, o, d, !last, E, n_dens);
         trace_cell<TRACE>(S, O, r, n_samples, cQ);
         ++n_samples;
         const float sQ = E.sigma, mQ = E.mmin;
@@ -989,19 +952,6 @@ __global__ void __launch_bounds__(256) index_pack_kernel(const int* __restrict__
     }
 }
 
-// The fused blend with a finite cut-off over the indexed edge records: one ray per lane.
-template <bool HALF, bool TRACE>
-int launch_indexed(const FoamScene& S, const FoamParams& P, const FoamRays& R, const FoamOut& O, hipStream_t stream) {
-    const dim3 grid(grid_for(R.n, kBlock)), block(kBlock);
-    switch (P.sh_deg) {
-        case 0: hipLaunchKernelGGL((foam_infer_kernel<2, kFusedIdx, HALF, 0, TRACE, false>), grid, block, 0, stream, S, P, R, O); break;
-        case 1: hipLaunchKernelGGL((foam_infer_kernel<2, kFusedIdx, HALF, 1, TRACE, false>), grid, block, 0, stream, S, P, R, O); break;
-        case 2: hipLaunchKernelGGL((foam_infer_kernel<2, kFusedIdx, HALF, 2, TRACE, false>), grid, block, 0, stream, S, P, R, O); break;
-        default: hipLaunchKernelGGL((foam_infer_kernel<2, kFusedIdx, HALF, 3, TRACE, false>), grid, block, 0, stream, S, P, R, O);
-    }
-    return launch_status("foam_infer_kernel (indexed edges)");
-}
-
 // lanes: 1 = one ray per lane (foam_infer_kernel), 2, 4 or 8 = a group of that many lanes per ray
 // (foam_group_kernel). TABLE: the reference's cache tags from the slot table (colour cut-off +inf).
 template <int STAGE, int COLOR, bool HALF, int DEG, bool TRACE, bool TABLE = false>
@@ -1022,9 +972,11 @@ int launch(const FoamScene& S, const FoamParams& P, const FoamRays& R, const Foa
                            dim3(grid_for(R.n, kBlock / 8)), dim3(kBlock), 0, stream, S, P, R, O);
         return launch_status("foam_group_kernel");
     }
-    // TABLE says that the cut-off is +inf: such a fused blend with one ray per lane runs in foam_tile.hip
-    hipLaunchKernelGGL((foam_infer_kernel<STAGE, COLOR, HALF, DEG, TRACE, TABLE && COLOR == kLazy>),
-                       dim3(grid_for(R.n, kBlock)), dim3(kBlock), 0, stream, S, P, R, O);
+    if constexpr (COLOR == kFused)
+        return launch_foam_tile(S, P, R, O, false, false, HALF, stream);
+    else
+        hipLaunchKernelGGL((foam_infer_kernel<STAGE, COLOR, HALF, DEG, TRACE, TABLE>), dim3(grid_for(R.n, kBlock)),
+                           dim3(kBlock), 0, stream, S, P, R, O);
     return launch_status("foam_infer_kernel");
 }
 
@@ -1155,10 +1107,6 @@ int foam_entry(const float* points, int64_t n_sites, const int32_t* offsets, con
     // Fused and baked blends with a finite colour cut skip a neighbour against the running minimum of the terms
     // before it in edge order; a lane of a group sees only its own share of them, so these run one ray per lane.
     if (stage == 2 && color_mode != kLazy && !(color_cut > 1e30)) lanes = 1;
-    // Without a cut-off no colour decides which other one is looked up, so one ray per lane queues its samples and
-    // evaluates them by cell (foam_tile.hip); with a finite one the running minimum does, and the lookup runs in the pass.
-    const bool tile =
-        stage == 2 && lanes == 1 && std::isinf(color_cut) && color_cut > 0 && (indexed || color_mode == kFused);
     // The site rows serve the group layouts' fused blend (config 5's 8-lane batch: 2538.6 -> 2437.6 ms with the
     // 64-byte rows); the two-pass exact colours with 4 lanes per ray ran slower on them (268.9 against 258.3 ms on
     // config 3) and keep the attr rows, as the one-ray-per-lane kernels do. Site blocks also supply those kernels'
@@ -1191,12 +1139,7 @@ int foam_entry(const float* points, int64_t n_sites, const int32_t* offsets, con
     // 256 bytes of LDS per wave there: config 5's batch ran 2437.6 ms with the table, 2298.0 ms with the tags.
     const bool table = slots != nullptr && std::isinf(color_cut) && color_cut > 0 && lanes != 8;
     if (wide) return launch_foam_wide(S, P, R, O, int(color_mode), sh_half != 0, s);
-    if (tile) return launch_foam_tile(S, P, R, O, indexed, exact_blend, sh_half != 0, s);
-    if (indexed) {
-        if (sh_half != 0)
-            return trace != nullptr ? launch_indexed<true, true>(S, P, R, O, s) : launch_indexed<true, false>(S, P, R, O, s);
-        return trace != nullptr ? launch_indexed<false, true>(S, P, R, O, s) : launch_indexed<false, false>(S, P, R, O, s);
-    }
+    if (indexed) return launch_foam_tile(S, P, R, O, true, exact_blend, sh_half != 0, s);
     if (trace != nullptr)
         return dispatch<true>(int(stage), int(color_mode), sh_half != 0, S, P, R, O, int(lanes), table, s);
     return dispatch<false>(int(stage), int(color_mode), sh_half != 0, S, P, R, O, int(lanes), table, s);

@@ -1,5 +1,5 @@
-// Inference renderer, one ray per lane with colours evaluated cell by cell on the matrix cores, gfx950: fused and exact
-// colours without a colour cut-off (+inf), for batches that fill the GPU.
+// Inference renderer, one ray per lane with colours evaluated cell by cell on the matrix cores, gfx950: fused colours, and
+// exact ones without a colour cut-off (+inf), for batches that fill the GPU.
 //
 // Same function as csrc/foam_infer.cu:286-361. A wave renders 64 consecutive rays (an 8 x 8 tile of the host's order). The
 // walk, the exit faces and the density run one ray per lane, as in foam_infer.hip. A colour does not steer a ray: only the
@@ -19,7 +19,11 @@
 // An SH row is then read once per quad and its 48 multiply-adds run on the matrix cores, where a lookup per (sample,
 // neighbour) through LDS took 12 LDS reads and 48 FMAs of every lane; samples of segments below w_thresh cost no colour.
 //
-// stats[:, 4], the reference's cache misses: every pass looks up all entries of a cell, so the count needs the cells only:
+// A finite cut-off (CUT) leaves a term out against the running minimum of the terms before it in edge order. A pass then
+// also takes the colour distances, since the lookups they admit are counted (stats[:, 4]), and the evaluation, which visits
+// a cell's entries in the same order with the same operations, admits the same terms.
+//
+// stats[:, 4], the reference's cache misses: without a cut-off every pass looks up all entries of a cell, so the count needs the cells only:
 // from the slot table with the ray's 8 tags in registers, or, without a table, from tags per lookup in LDS. EXACT: the exact
 // (lazy) colour mode by the same one-pass blend. Its colour, sum_k exp(-(m_k - m_min) / 2) c_k / sum_k exp(-(m_k - m_min) / 2)
 // over every neighbour, is the blend's two sums up to rounding; its statistics count a colour pass only where the reference
@@ -29,11 +33,13 @@
 // issue of the geometry pass, about half of the time of the 800 x 800 view (measured with the colours left out). One MI355X, ms of
 // a render call, the one-ray-per-lane kernel of foam_infer.hip -> this one: 2M sites, 8.29M rays, fused, 69 % of the segments
 // heavier than w_thresh, 179.9 -> 113.5; 1920 x 1080 rays of 1M sites, fused, 38 %, 78.4 -> 47.5; 800 x 800, exact,
-// 29 %, 23.2 -> 11.5.
+// 29 %, 23.2 -> 11.5. With a cut-off of eps 1e-3: the first scene 169.8 -> 154.0, with fp16 SH 142.6 -> 125.5; 1237 x 822
+// rays, fp16, 40.1 -> 26.1.
 // Not taken (two such views, 11.2 / 51.3 ms): 16 samples of a cell against 16 entries per v_mfma_f32_16x16x4_f32 13.7 / 60.2 (a
 // cell's queue holds 6 samples on average, the rest is padding); the row's loads predicated on the entry instead of clamped
 // to one of the cell's 16.8 / 81.6 (each becomes a branch with its own wait); the ray's state parked in LDS during the
 // evaluation 11.7 / 53.5.
+#include <cmath>
 #include <type_traits>
 
 #include "vgr_foam.h"
@@ -94,10 +100,11 @@ struct Pass {
 
 // Density at o + t d over the neighbourhood of c and, when want_exit, the exit face: foam_infer.hip's sequential pass (the
 // same operations in the same order). The next edge record is requested while the current entry is evaluated.
-// TAGS (no slot table): the lookups that miss the ray's tags, which start at `tags`, 64 ints apart.
-template <bool IDX, bool TAGS>
+// TAGS (no slot table): the lookups that miss the ray's tags, which start at `tags`, 64 ints apart. CUT: a finite colour
+// cut-off, so a lookup is an entry within it of the running minimum of the entries before.
+template <bool IDX, bool TAGS, bool CUT>
 __device__ __forceinline__ Pass pass(const FoamScene& S, int c, float t, const float (&o)[3], const float (&d)[3],
-                                     bool want_exit, int& n_dens, int& n_sh, lds_int* tags) {
+                                     bool want_exit, int& n_dens, int& n_sh, lds_int* tags, float color_cut) {
     const int e0 = S.offsets[c], e1 = S.offsets[c + 1];
     float4 edn = S.edge[entry_in(e0, e1)];
     int kn = 0;
@@ -106,11 +113,14 @@ __device__ __forceinline__ Pass pass(const FoamScene& S, int c, float t, const f
     float x[3];
     sample_point(o, d, t, x);
     Pass R{0.f, kInf, INT_MAX, e1 - e0};
+    float low = kInf;
     for (int e = e0; e < e1; ++e) {
         const float4 ed = edn;
         const int k = IDX ? __float_as_int(ed.w) : kn;
         const float4* a = S.attr + 5 * static_cast<int64_t>(k);
         const float4 q0 = a[0], q1 = a[1];
+        float4 q2, q3;
+        if constexpr (CUT) q2 = a[2], q3 = a[3];
         const int en = min(e + 1, e1 - 1);
         edn = S.edge[en];
         if constexpr (!IDX) kn = S.nbr[en];
@@ -127,11 +137,22 @@ __device__ __forceinline__ Pass pass(const FoamScene& S, int c, float t, const f
         }
         float v0, v1, v2, r2;
         offset_of(x, ed, v0, v1, v2, r2);
-        if (r2 <= cutoffs(IDX ? q1.w : ed.w).x) {
+        const float2 cut = cutoffs(IDX ? q1.w : ed.w);
+        if (r2 <= cut.x) {
             R.sigma += density_term(q0, q1, v0, v1, v2);
             ++n_dens;
         }
-        if constexpr (TAGS) {
+        bool look = true;
+        if constexpr (CUT) {
+            const float lim = low + color_cut;
+            look = r2 * cut.y <= lim;
+            if (look) {
+                const float m = maha_f(q2, q3, v0, v1, v2);
+                look = m <= lim;
+                low = look && m < low ? m : low;
+            }
+        }
+        if (TAGS && look) {
             lds_int* p = tags + (k & (kRayTagSlots - 1)) * kBlock;
             n_sh += *p != k ? 1 : 0;
             *p = k;
@@ -157,8 +178,8 @@ __device__ __forceinline__ int table_hits(const FoamScene& S, int c, int (&tag)[
 
 // Blends of 64 samples, one per lane, the four samples of a quad in one cell (`cell`, -1 for a quad without samples): lane l
 // reads entry base + l % 4 of its quad's cell, the quad's four lanes share the four entries. `dir` is the sample's direction.
-template <bool IDX, bool HALF, int DEG>
-__device__ __forceinline__ void blend_quads(const FoamScene& S, int cell, const float (&x)[3], const float (&dir)[3],
+template <bool IDX, bool HALF, int DEG, bool CUT>
+__device__ __forceinline__ void blend_quads(const FoamScene& S, float color_cut, int cell, const float (&x)[3], const float (&dir)[3],
                                             float (&C)[3]) {
     constexpr int NB = (DEG + 1) * (DEG + 1), NV = sh_vec4<HALF, DEG>();
     const int lane = static_cast<int>(threadIdx.x);
@@ -194,19 +215,31 @@ __device__ __forceinline__ void blend_quads(const FoamScene& S, int cell, const 
             c1 = __builtin_amdgcn_mfma_f32_4x4x1f32(coef(3 * j + 1), b[j], c1, 0, 0, 0);
             c2 = __builtin_amdgcn_mfma_f32_4x4x1f32(coef(3 * j + 2), b[j], c2, 0, 0, 0);
         }
-        const auto distance = [&](auto perm, int r) {  // of entry base + r, from the quad's lane r
+        float lam = 0.f;  // the entry's bound: m >= lam r2
+        if constexpr (CUT) lam = cutoffs(IDX ? at[1].w : ed.w).y;
+        const auto distance = [&](auto perm, int r, float& lb) {  // of entry base + r, from the quad's lane r
             constexpr int P = decltype(perm)::value;
             const float4 p = make_float4(row_perm<P>(ed.x), row_perm<P>(ed.y), row_perm<P>(ed.z), 0.f);
             const float4 a = make_float4(row_perm<P>(q2.x), row_perm<P>(q2.y), row_perm<P>(q2.z), row_perm<P>(q2.w));
             const float4 c = make_float4(row_perm<P>(q3.x), row_perm<P>(q3.y), 0.f, 0.f);
             float v0, v1, v2, r2;
             offset_of(x, p, v0, v1, v2, r2);
-            const float d = maha_f(a, c, v0, v1, v2);
-            return base + r < e1 && d <= __builtin_huge_valf() ? d : __builtin_huge_valf();  // neither absent nor NaN
+            if constexpr (CUT) lb = r2 * row_perm<P>(lam);
+            return maha_f(a, c, v0, v1, v2);
         };
-        const float mk[4] = {distance(std::integral_constant<int, 0x00>{}, 0), distance(std::integral_constant<int, 0x55>{}, 1),
-                             distance(std::integral_constant<int, 0xAA>{}, 2), distance(std::integral_constant<int, 0xFF>{}, 3)};
-        const float low = fminf(m, fminf(fminf(mk[0], mk[1]), fminf(mk[2], mk[3])));
+        float lb[4], mk[4];
+        mk[0] = distance(std::integral_constant<int, 0x00>{}, 0, lb[0]);
+        mk[1] = distance(std::integral_constant<int, 0x55>{}, 1, lb[1]);
+        mk[2] = distance(std::integral_constant<int, 0xAA>{}, 2, lb[2]);
+        mk[3] = distance(std::integral_constant<int, 0xFF>{}, 3, lb[3]);
+        float low = m;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {  // a term left out (absent, NaN, or beyond the cut-off): +inf, weight 0
+            const float lim = CUT ? low + color_cut : kInf;
+            const bool in = base + r < e1 && (!CUT || lb[r] <= lim) && mk[r] <= lim;
+            mk[r] = in ? mk[r] : kInf;
+            low = fminf(low, mk[r]);
+        }
         const float keep = weight_of(m, low);
         A *= keep, cr *= keep, cg *= keep, cb *= keep, m = low;
 #pragma unroll
@@ -222,8 +255,8 @@ __device__ __forceinline__ void blend_quads(const FoamScene& S, int cell, const 
 // Evaluates every queued sample (the whole wave takes part): `queued` of each ray, sample s of ray r at 64 s + r. The samples
 // are grouped by cell through a hash table in LDS (a cell's entry counts its samples and gives each its rank; an exclusive
 // scan of the counts, rounded up to quads, gives the cells their places), then evaluated 64 places at a time.
-template <bool IDX, bool HALF, int DEG>
-__device__ __forceinline__ void evaluate(const FoamScene& S, Queue& Q, int queued, const float (&d)[3]) {
+template <bool IDX, bool HALF, int DEG, bool CUT>
+__device__ __forceinline__ void evaluate(const FoamScene& S, float color_cut, Queue& Q, int queued, const float (&d)[3]) {
     const int lane = static_cast<int>(threadIdx.x);
     constexpr int PER = kHash / kBlock;
 #pragma unroll
@@ -275,7 +308,7 @@ __device__ __forceinline__ void evaluate(const FoamScene& S, Queue& Q, int queue
         const int ray = from % kBlock;
         const float dir[3] = {__shfl(d[0], ray), __shfl(d[1], ray), __shfl(d[2], ray)};
         float C[3];
-        blend_quads<IDX, HALF, DEG>(S, lead >= 0 ? Q.cell[from] : -1, x, dir, C);
+        blend_quads<IDX, HALF, DEG, CUT>(S, color_cut, lead >= 0 ? Q.cell[from] : -1, x, dir, C);
         if (at >= 0) Q.x[at] = make_float4(q.w * C[0], q.w * C[1], q.w * C[2], 0.f);
     }
     __builtin_amdgcn_wave_barrier();
@@ -284,7 +317,7 @@ __device__ __forceinline__ void evaluate(const FoamScene& S, Queue& Q, int queue
 // IDX: the indexed edge records (vgr_foam_index_pack). TABLE: cache misses from the slot table. EXACT: the exact colour
 // mode's statistics (its colour passes: segments with weight > w_thresh, the far sample's cell and, when the segment before
 // was not coloured, the near sample's); always with the table.
-template <bool IDX, bool HALF, int DEG, bool TABLE, bool EXACT>
+template <bool IDX, bool HALF, int DEG, bool CUT, bool TABLE, bool EXACT>
 __global__ void __launch_bounds__(kBlock, kWaves) foam_tile_kernel(FoamScene S, FoamParams P, FoamRays R, FoamOut O) {
     __shared__ Queue Q;
     __shared__ int lds_tags[TABLE ? 1 : kRayTagSlots * kBlock];
@@ -315,7 +348,7 @@ __global__ void __launch_bounds__(kBlock, kWaves) foam_tile_kernel(FoamScene S, 
         t_far = R.t_far[r], tA = R.t_near[r];
         if (R.cap != nullptr) max_samples = R.cap[r];
         cA = walk<IDX>(S, start, o[0] + tA * d[0], o[1] + tA * d[1], o[2] + tA * d[2], walk_steps);
-        E = pass<IDX, !TABLE>(S, cA, tA, o, d, true, n_dens, n_sh, my_tags);
+        E = pass<IDX, !TABLE, CUT>(S, cA, tA, o, d, true, n_dens, n_sh, my_tags, P.color_cut);
         nA = E.n;
         if (TABLE && !EXACT) n_sh += E.n - table_hits(S, cA, tag);
         if (O.trace != nullptr) trace_cell<true>(S, O, r, 0, cA);
@@ -332,7 +365,7 @@ __global__ void __launch_bounds__(kBlock, kWaves) foam_tile_kernel(FoamScene S, 
             const bool last = E.next == INT_MAX || E.t_exit >= t_far || n_samples + 1 >= max_samples;
             const float tB = last ? t_far : fmaxf(E.t_exit, tA);
             const int cB = last ? cA : E.next;
-            E = pass<IDX, !TABLE>(S, cB, tB, o, d, !last, n_dens, n_sh, my_tags);
+            E = pass<IDX, !TABLE, CUT>(S, cB, tB, o, d, !last, n_dens, n_sh, my_tags, P.color_cut);
             if (TABLE && !EXACT) n_sh += E.n - table_hits(S, cB, tag);
             if (O.trace != nullptr) trace_cell<true>(S, O, r, n_samples, cB);
             ++n_samples;
@@ -366,7 +399,7 @@ __global__ void __launch_bounds__(kBlock, kWaves) foam_tile_kernel(FoamScene S, 
         const bool done = !wave_any(alive || ended);
         if (done || wave_any(queued == kDepth)) {
             __builtin_amdgcn_wave_barrier();
-            evaluate<IDX, HALF, DEG>(S, Q, queued, d);
+            evaluate<IDX, HALF, DEG, CUT>(S, P.color_cut, Q, queued, d);
             for (int s = 0; s < queued; ++s) {
                 const float4 v = Q.x[kBlock * s + lane];
                 acc[0] += v.x, acc[1] += v.y, acc[2] += v.z;
@@ -384,14 +417,14 @@ __global__ void __launch_bounds__(kBlock, kWaves) foam_tile_kernel(FoamScene S, 
     st[0] = n_samples, st[1] = n_color, st[2] = walk_steps, st[3] = n_dens, st[4] = n_sh;
 }
 
-template <bool IDX, bool HALF, bool TABLE, bool EXACT>
+template <bool IDX, bool HALF, bool CUT, bool TABLE, bool EXACT>
 void launch(const FoamScene& S, const FoamParams& P, const FoamRays& R, const FoamOut& O, hipStream_t stream) {
     const dim3 grid(grid_for(R.n, kBlock)), block(kBlock);
     switch (P.sh_deg) {
-        case 0: hipLaunchKernelGGL((foam_tile_kernel<IDX, HALF, 0, TABLE, EXACT>), grid, block, 0, stream, S, P, R, O); break;
-        case 1: hipLaunchKernelGGL((foam_tile_kernel<IDX, HALF, 1, TABLE, EXACT>), grid, block, 0, stream, S, P, R, O); break;
-        case 2: hipLaunchKernelGGL((foam_tile_kernel<IDX, HALF, 2, TABLE, EXACT>), grid, block, 0, stream, S, P, R, O); break;
-        default: hipLaunchKernelGGL((foam_tile_kernel<IDX, HALF, 3, TABLE, EXACT>), grid, block, 0, stream, S, P, R, O);
+        case 0: hipLaunchKernelGGL((foam_tile_kernel<IDX, HALF, 0, CUT, TABLE, EXACT>), grid, block, 0, stream, S, P, R, O); break;
+        case 1: hipLaunchKernelGGL((foam_tile_kernel<IDX, HALF, 1, CUT, TABLE, EXACT>), grid, block, 0, stream, S, P, R, O); break;
+        case 2: hipLaunchKernelGGL((foam_tile_kernel<IDX, HALF, 2, CUT, TABLE, EXACT>), grid, block, 0, stream, S, P, R, O); break;
+        default: hipLaunchKernelGGL((foam_tile_kernel<IDX, HALF, 3, CUT, TABLE, EXACT>), grid, block, 0, stream, S, P, R, O);
     }
 }
 
@@ -399,13 +432,17 @@ template <bool HALF>
 void launch_half(const FoamScene& S, const FoamParams& P, const FoamRays& R, const FoamOut& O, bool indexed, bool exact,
                  hipStream_t stream) {
     const bool table = S.slots != nullptr;
-    if (exact)  // always indexed, with the slot table
-        launch<true, HALF, true, true>(S, P, R, O, stream);
+    if (!(std::isinf(P.color_cut) && P.color_cut > 0))  // lookups depend on the distances: tags per lookup
+        indexed ? launch<true, HALF, true, false, false>(S, P, R, O, stream)
+                : launch<false, HALF, true, false, false>(S, P, R, O, stream);
+    else if (exact)  // always indexed, with the slot table
+        launch<true, HALF, false, true, true>(S, P, R, O, stream);
     else if (indexed)
-        table ? launch<true, HALF, true, false>(S, P, R, O, stream) : launch<true, HALF, false, false>(S, P, R, O, stream);
+        table ? launch<true, HALF, false, true, false>(S, P, R, O, stream)
+              : launch<true, HALF, false, false, false>(S, P, R, O, stream);
     else
-        table ? launch<false, HALF, true, false>(S, P, R, O, stream)
-              : launch<false, HALF, false, false>(S, P, R, O, stream);
+        table ? launch<false, HALF, false, true, false>(S, P, R, O, stream)
+              : launch<false, HALF, false, false, false>(S, P, R, O, stream);
 }
 
 }  // namespace
