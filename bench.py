@@ -396,7 +396,7 @@ def bench_foam(args):
 							'(counts every L1/L2/LDS hit as a fetch, so it can exceed the HBM peak)',
 							'foam_tile_kernel' if tile else 'foam_infer_kernel' if lanes == 1 else 'foam_group_kernel')
 	if roofline['frac'] is not None and tile:
-		roofline['limiter'] = ('not HBM: the texture data path is busy 94 % of the launch and the L2 serves 93 % of '
+		roofline['limiter'] = ('not HBM: the texture data path is busy 96 % of the launch and the L2 serves 97 % of '
 							   'the gathers (profiles/foam_infer_config3_counters.md)')
 
 	cpu = None

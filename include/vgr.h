@@ -78,7 +78,10 @@ int vgr_foam_infer_traced(const float* points, int64_t n_sites, const int32_t* o
  * a group of that many lanes per ray (each lane takes every lanes_per_ray-th edge of a cell's neighbourhood; the
  * group combines exit faces by a lexicographic minimum, so the visited cells are the same, and density and colour
  * terms by sums, so only their summation order differs), 0 the library's default (the layout vgr_foam_infer runs:
- * 4 lanes per ray for stages 0 and 1 and lazy colours, one ray per lane for fused and baked colours). Fused and
+ * for the full rendering of up to 98304 rays 16 lanes per ray, whose densities are summed in the order of one ray per
+ * lane, so T, traces and stats have that layout's bits; beyond, and for stages 0 and 1, 4 lanes per ray for stages 0 and 1
+ * and lazy colours, one ray per lane for fused and baked colours). One ray per lane evaluates fused colours for the
+ * samples of segments with weight > w_thresh only; without a cut-off its stats[:, 4] counts every entry of a pass. Fused and
  * baked colours with a finite color_cut always run one ray per lane (their neighbour skipping follows the edge
  * order). trace may be NULL (then trace_cap is ignored). order (NULL = the batch order): a permutation of
  * 0 .. B - 1 giving the order in which the rays are traced (vgr_ray_order); results are the same in any order, an
@@ -427,7 +430,8 @@ int vgr_foam_index_pack(const int32_t* offsets, const int32_t* nbr, const float*
  * VGR_COLOR_FUSED) with one ray per lane (lanes_per_ray 0 or 1) reads edge_i and attr_i in place of nbr, edge and
  * attr, one record stream per neighbourhood entry instead of two. The outputs are bit-identical to
  * vgr_foam_infer_lanes on the same pack. Exact colours (VGR_COLOR_LAZY, stage 2) with one ray per lane, slots
- * given and color_cut +inf run as that same fused blend: rgb, T, depth and stats[:, 0..3] bit-identical to
+ * given and color_cut +inf run as that same fused blend (lanes_per_ray 0 and up to 98304 rays: the 16-lane layout of
+ * vgr_foam_infer_lanes, on the reference records): rgb, T, depth and stats[:, 0..3] bit-identical to
  * VGR_COLOR_FUSED (rgb within rounding of the two-pass exact colour: the same normalised sum over every neighbour,
  * kept relative to a running minimum), stats[:, 4] the exact mode's cache misses (its colour passes: segments of
  * weight > w_thresh). Every other stage, colour mode or layout runs vgr_foam_infer_lanes on the reference records

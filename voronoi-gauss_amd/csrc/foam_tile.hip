@@ -23,21 +23,22 @@
 // also takes the colour distances, since the lookups they admit are counted (stats[:, 4]), and the evaluation, which visits
 // a cell's entries in the same order with the same operations, admits the same terms.
 //
-// stats[:, 4], the reference's cache misses: without a cut-off every pass looks up all entries of a cell, so the count needs the cells only:
+// stats[:, 4], the reference's cache misses: without a cut-off every pass looks up all entries, so the count needs the cells:
 // from the slot table with the ray's 8 tags in registers, or, without a table, from tags per lookup in LDS. EXACT: the exact
 // (lazy) colour mode by the same one-pass blend. Its colour, sum_k exp(-(m_k - m_min) / 2) c_k / sum_k exp(-(m_k - m_min) / 2)
 // over every neighbour, is the blend's two sums up to rounding; its statistics count a colour pass only where the reference
 // runs one: for the far sample of a segment heavier than w_thresh and, when the segment before was not, its near sample.
 //
-// Bound by the latency of the gathers behind a chain of (cell -> edge record -> SH row) at 4 waves per SIMD, and by the
-// issue of the geometry pass, about half of the time of the 800 x 800 view (measured with the colours left out). One MI355X, ms of
-// a render call, the one-ray-per-lane kernel of foam_infer.hip -> this one: 2M sites, 8.29M rays, fused, 69 % of the segments
-// heavier than w_thresh, 179.9 -> 113.5; 1920 x 1080 rays of 1M sites, fused, 38 %, 78.4 -> 47.5; 800 x 800, exact,
-// 29 %, 23.2 -> 11.5. With a cut-off of eps 1e-3: the first scene 169.8 -> 154.0, with fp16 SH 142.6 -> 125.5; 1237 x 822
-// rays, fp16, 40.1 -> 26.1.
-// Not taken (two such views, 11.2 / 51.3 ms): 16 samples of a cell against 16 entries per v_mfma_f32_16x16x4_f32 13.7 / 60.2 (a
-// cell's queue holds 6 samples on average, the rest is padding); the row's loads predicated on the entry instead of clamped
-// to one of the cell's 16.8 / 81.6 (each becomes a branch with its own wait); the ray's state parked in LDS during the
+// Bound by the texture data path, through which every gather returns: on the 2M-site scene below TD is busy 96 % of the
+// launch, the L2 hits 97 %, and the VALU issues less than half of what the lookup per lane issued (4.7e10 against 1.0e11);
+// in a view with fewer heavy segments the geometry pass is about half of the time (measured with the colours left out).
+// One MI355X, ms of a render call, the one-ray-per-lane kernel of foam_infer.hip -> this one: 2M sites, 8.29M rays, fused,
+// 69 % of the segments heavier than w_thresh, 179.9 -> 113.5; 1920 x 1080 rays of 2M sites, fused, 38 %, 78.4 -> 47.5;
+// 800 x 800, exact, 29 %, 23.2 -> 11.5. With a cut-off of eps 1e-3: the first scene 169.8 -> 154.0, with fp16 SH 142.6 ->
+// 125.5; 1237 x 822 rays, fp16, 40.1 -> 26.1.
+// Not taken (two such views, 11.2 / 51.3 ms): 16 samples of a cell against 16 entries per v_mfma_f32_16x16x4_f32 13.7 /
+// 60.2 (a cell's queue holds 6 samples on average, the rest is padding); the row's loads predicated on the entry instead of
+// clamped to one of the cell's 16.8 / 81.6 (each becomes a branch with its own wait); the ray's state parked in LDS during the
 // evaluation 11.7 / 53.5.
 #include <cmath>
 #include <type_traits>
@@ -49,10 +50,11 @@ namespace {
 
 constexpr int kBlock = 64;
 constexpr int kRayTagSlots = 8;
-// Queued samples per ray: 11.2 / 51.3 ms on the two views of the variants above; 3: 11.6 / 54.1 (smaller batches), 5: 12.0 / 55.1 (LDS).
+// Queued samples per ray: 11.2 / 51.3 ms on the two views of the variants above; 3: 11.6 / 54.1 (smaller batches), 5: 12.0 /
+// 55.1 (LDS).
 constexpr int kDepth = 4;
-// Waves per SIMD: 4 (128 VGPRs) hold the row, the basis and the ray without spills (SH degree 3 with a slot table); 3 with
-// 8 samples per ray 12.8 / 57.0, 5 spill: 19.9 / 86.7.
+// Waves per SIMD: 4 (128 VGPRs) hold the row, the basis and the ray with 18 spills (fp32, SH degree 3; none with fp16);
+// 3 with 8 samples per ray 12.8 / 57.0, 5 spill: 19.9 / 86.7.
 constexpr int kWaves = 4;
 
 typedef float float4v __attribute__((ext_vector_type(4)));
