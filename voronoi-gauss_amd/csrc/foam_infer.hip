@@ -213,18 +213,18 @@ __device__ __forceinline__ void cached_colour(ColorCache<COLOR>& C, const float4
         const bool hit = pending && C.tag[home] == k;
         const bool miss = pending && !hit;
         if (miss) C.claim[home] = lane;
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
         if (hit) C.claim[home] = -1;  // pin, after the claims
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
         const bool win = miss && C.claim[home] == lane;
         if (win) C.tag[home] = k;
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
         const bool lose = miss && !win && C.tag[home] != k;  // the slot holds another site in this lookup
         int block = home;
         bool served = hit || (miss && !lose), lead_fetch = false;
         if (OVF > 0 && __ballot(lose) != 0) {
             if (lose) C.claim[home] = lane;
-            __builtin_amdgcn_wave_barrier();
+            wave_sync();
             const bool lead = lose && C.claim[home] == lane;
             const uint64_t leads = __ballot(lead);
             if (lead) {
@@ -232,7 +232,7 @@ __device__ __forceinline__ void cached_colour(ColorCache<COLOR>& C, const float4
                 lead_fetch = o < OVF;
                 C.ovf_k[home] = k, C.ovf_b[home] = lead_fetch ? SLOTS + o : -1;
             }
-            __builtin_amdgcn_wave_barrier();
+            wave_sync();
             if (lose) {
                 const int ok = C.ovf_k[home], ob = C.ovf_b[home];
                 if (ok == k && ob >= 0) block = ob, served = true;
@@ -245,7 +245,7 @@ __device__ __forceinline__ void cached_colour(ColorCache<COLOR>& C, const float4
                 const int r = lanes_below(fetches);
                 C.req_k[r] = k, C.req_b[r] = block;
             }
-            __builtin_amdgcn_wave_barrier();
+            wave_sync();
             const int total = NV * __popcll(fetches);
             for (int base = 0; base < total; base += n_active) {
                 const int j = base + rank;
@@ -255,7 +255,7 @@ __device__ __forceinline__ void cached_colour(ColorCache<COLOR>& C, const float4
                     C.data[q * BLOCKS + C.req_b[r]] = sh[stride * static_cast<int64_t>(kr) + q];
                 }
             }
-            __builtin_amdgcn_wave_barrier();
+            wave_sync();
         }
         if (served) {
             float b[16];
@@ -275,7 +275,7 @@ __device__ __forceinline__ void cached_colour(ColorCache<COLOR>& C, const float4
             c[0] = fmaxf(c[0], 0.f), c[1] = fmaxf(c[1], 0.f), c[2] = fmaxf(c[2], 0.f);
         }
         pending = pending && !served;
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
         if (__ballot(pending) == 0) break;
     }
 }

@@ -58,6 +58,7 @@ constexpr int kDepth = 4;
 constexpr int kWaves = 4;
 
 typedef float float4v __attribute__((ext_vector_type(4)));
+typedef short short2v __attribute__((ext_vector_type(2), may_alias));  // two places of a queue's list
 
 // LDS words as such (through a generic pointer they would be flat accesses, which wait for all outstanding loads).
 typedef __attribute__((address_space(3))) volatile int lds_int;
@@ -70,7 +71,7 @@ struct Queue {
     int cell[kQueued];
     int key[kHash];     // cells found (-1: free)
     int count[kHash];   // their samples, then the first place of the cell in `list`
-    short list[4 * kQueued];  // samples by cell, every cell beginning a quad; -1: an empty place
+    alignas(4) short list[4 * kQueued];  // samples by cell, every cell beginning a quad; -1: an empty place
 };
 
 // The walk of foam_infer.hip's one-ray-per-lane kernel.
@@ -264,8 +265,8 @@ __device__ __forceinline__ void evaluate(const FoamScene& S, float color_cut, Qu
 #pragma unroll
     for (int u = 0; u < PER; ++u) Q.key[kBlock * u + lane] = -1, Q.count[kBlock * u + lane] = 0;
 #pragma unroll
-    for (int u = 0; u < 2 * kDepth; ++u) reinterpret_cast<int*>(Q.list)[kBlock * u + lane] = -1;
-    __builtin_amdgcn_wave_barrier();
+    for (int u = 0; u < 2 * kDepth; ++u) reinterpret_cast<short2v*>(Q.list)[kBlock * u + lane] = short2v{-1, -1};
+    wave_sync();
     int slot[kDepth], rank[kDepth];
 #pragma unroll
     for (int s = 0; s < kDepth; ++s) {
@@ -281,7 +282,7 @@ __device__ __forceinline__ void evaluate(const FoamScene& S, float color_cut, Qu
             slot[s] = h, rank[s] = atomicAdd(Q.count + h, 1);
         }
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
     int places[PER], sum = 0;
 #pragma unroll
     for (int u = 0; u < PER; ++u) places[u] = (Q.count[PER * lane + u] + 3) & ~3, sum += places[u];
@@ -293,14 +294,14 @@ __device__ __forceinline__ void evaluate(const FoamScene& S, float color_cut, Qu
     }
     const int total = __builtin_amdgcn_readlane(run, kBlock - 1);
     run -= sum;
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
 #pragma unroll
     for (int u = 0; u < PER; ++u) Q.count[PER * lane + u] = run, run += places[u];
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
 #pragma unroll
     for (int s = 0; s < kDepth; ++s)
         if (s < queued) Q.list[Q.count[slot[s]] + rank[s]] = static_cast<short>(kBlock * s + lane);
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
     for (int first = 0; first < total; first += kBlock) {
         const int at = first + lane < total ? Q.list[first + lane] : -1;
         const int lead = row_perm<0x00>(at);  // the quad's first sample, there if any is
@@ -313,7 +314,7 @@ __device__ __forceinline__ void evaluate(const FoamScene& S, float color_cut, Qu
         blend_quads<IDX, HALF, DEG, CUT>(S, color_cut, lead >= 0 ? Q.cell[from] : -1, x, dir, C);
         if (at >= 0) Q.x[at] = make_float4(q.w * C[0], q.w * C[1], q.w * C[2], 0.f);
     }
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
 }
 
 // IDX: the indexed edge records (vgr_foam_index_pack). TABLE: cache misses from the slot table. EXACT: the exact colour
@@ -400,7 +401,7 @@ __global__ void __launch_bounds__(kBlock, kWaves) foam_tile_kernel(FoamScene S, 
         }
         const bool done = !wave_any(alive || ended);
         if (done || wave_any(queued == kDepth)) {
-            __builtin_amdgcn_wave_barrier();
+            wave_sync();
             evaluate<IDX, HALF, DEG, CUT>(S, P.color_cut, Q, queued, d);
             for (int s = 0; s < queued; ++s) {
                 const float4 v = Q.x[kBlock * s + lane];

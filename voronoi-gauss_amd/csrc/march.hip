@@ -601,9 +601,9 @@ __device__ void grad_pass_wave(const MarchField& F, const MarchGradOut& G, int i
                 row = true;
             }
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
         add_rows(G, slots, __ballot(row), k, nb, rank, n_act);
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
     }
 }
 
@@ -1241,9 +1241,9 @@ __device__ void march_ray_group_backward(const MarchField& F, const MarchParams&
 #pragma unroll
                 for (int ch = 0; ch < 3; ++ch) mine[13 + ch] = S[s].col && Cc.c[s][ch] > 0.f ? gR[ch] * S[s].aw : 0.f;
             }
-            __builtin_amdgcn_wave_barrier();
+            wave_sync();
             add_rows(G, slots, __ballot(row), Cc.k[s], nb, rank, n_act);
-            __builtin_amdgcn_wave_barrier();
+            wave_sync();
             clear_slot(S[s]);
         }
     };
@@ -1427,9 +1427,9 @@ __device__ void march_visits(const MarchField& F, const MarchParams& M, const Ma
 #pragma unroll
                 for (int ch = 0; ch < 3; ++ch) mine[13 + ch] = S[s].col && Cc.c[s][ch] > 0.f ? gR[ch] * S[s].aw : 0.f;
             }
-            __builtin_amdgcn_wave_barrier();
+            wave_sync();
             add_rows_wave(G, slots, __ballot(row), Cc.k[s], RL);
-            __builtin_amdgcn_wave_barrier();
+            wave_sync();
         }
     }
 }
@@ -1703,10 +1703,10 @@ __device__ void train_scatter(const MarchField& F, const MarchGradOut& G, const 
                 for (int ch = 0; ch < 3; ++ch) mine[13 + ch] = dc[ch];
             }
         }
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
         if constexpr (WAVE) add_rows_wave(G, slots, __ballot(row), k, RL);
         else add_rows(G, slots, __ballot(row), k, nb, rank, n_act);
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
     }
 }
 

@@ -184,7 +184,7 @@ __global__ void __launch_bounds__(kBlock)
     const int my_start = has ? start[i0 + lane] : static_cast<int>(w_end);  // past the rows: never <= an entry
     const int my_old = has ? old_of(P, static_cast<int>(i0 + lane)) : 0;
     const int my_e0 = has ? P.offsets[my_old] : 0;
-    __builtin_amdgcn_wave_barrier();
+    wave_sync();
     constexpr int U = 4;  // entries a lane has in flight: their loads (adj, inv, site4) depend on each other in turn
     for (int64_t base = w_begin; base < w_end; base += 64 * U) {
         int s[U], e[U], j[U];
@@ -224,7 +224,7 @@ __global__ void __launch_bounds__(kBlock)
         }
     }
     if (SLOTS) {
-        __builtin_amdgcn_wave_barrier();
+        wave_sync();
         for (int t = lane; t < 4 * cnt; t += 64) {  // one int4 (two slots) per lane
             const unsigned long long* m = mine + 16 * (t / 4) + 2 * (t % 4);
             const auto first = [](unsigned long long k) { return k == ~0ull ? -2 : static_cast<int>(k & 0xffffffffu); };

@@ -53,6 +53,15 @@ __device__ __forceinline__ float row_perm(float v) {
     return __int_as_float(row_perm<CTRL>(__float_as_int(v)));
 }
 
+// Hands LDS data from the lanes of a wave to each other: what a lane stored before is stored for every lane's accesses after.
+// The lanes run in step, so no instruction is emitted; the barrier alone orders no memory, and without the fences the
+// compiler may move an access across it that it can prove independent of the lane's own accesses (of another type, say).
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Real spherical-harmonics basis up to degree 3 (3DGS constants and signs), zero beyond `deg`.
 __device__ inline void sh_basis(float x, float y, float z, int deg, float (&b)[16]) {
     b[0] = 0.28209479177387814f;
