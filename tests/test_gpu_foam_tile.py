@@ -108,3 +108,31 @@ def test_tile_layout_cut_off(gpu, hub, n_rays, indexed, sh_half, cut):
 		np.testing.assert_allclose(g['rgb'], wide['rgb'], atol=1e-5, rtol=0)  # as in check
 		r = ref_foam(pk, 3, *rays, tt, wt, color_cut=cut, color_mode=2, trace_cap=512)
 		compare(g, r, exact_trace=tt == 0.0, stats_frac=0.98, w_thresh=max(wt, 1e-4))
+
+
+@pytest.mark.parametrize('sh_half', [False, True])
+@pytest.mark.parametrize('indexed', [False, True])
+def test_terms_left_out_add_nothing(gpu, hub, sh_half, indexed):
+	"""A term left out of a blend adds nothing whatever its colour is: sites of infinite colour (fp16 SH past 65504) beyond
+	the cut-off of a ray's samples, and cells whose terms are all left out (conics of infinities: distances NaN), whose
+	colour is 0 / 0 as in the other layouts. Against 16 lanes per ray, which skip those terms."""
+	f, (o, d, start, near, _, far) = hub
+	rays = (o, d, start, near, far)
+	pk = f.pack(eps_density=1e-3, sh_half=sh_half)
+	pk['sh'] = pk['sh'].copy()  # the field's own array
+	pk['sh'][::23, 0] = np.inf
+	kw = dict(indexed=indexed, cut=0.5)
+	g, wide = run(gpu, pk, 3, rays, 1e-4, 1e-3, 2, **kw), run(gpu, pk, 3, rays, 1e-4, 1e-3, 2, lanes=None, cut=0.5)
+	ok = np.isfinite(wide['rgb'])  # the others: an infinite term that counts, as inf or, if its weight underflows, NaN
+	assert not ok.all() and ok.all(1).sum() > 20
+	np.testing.assert_array_equal(np.isfinite(g['rgb']), ok)
+	np.testing.assert_allclose(g['rgb'][ok], wide['rgb'][ok], atol=1e-5, rtol=1e-6)  # as in check
+	pk = f.pack(eps_density=1e-3, sh_half=sh_half)
+	inside = np.abs(f.points).max(1) < 0.45  # whole neighbourhoods of these sites
+	pk['attr'][inside, 8:14] = np.inf
+	for cut in (math.inf, 2 * math.log(1e3)):
+		kw = dict(indexed=indexed, cut=cut)
+		g, wide = run(gpu, pk, 3, rays, 1e-4, 1e-3, 2, **kw), run(gpu, pk, 3, rays, 1e-4, 1e-3, 2, lanes=None, cut=cut)
+		bad = np.isnan(wide['rgb']).any(1)
+		assert bad.any() and not bad.all()
+		np.testing.assert_allclose(g['rgb'], wide['rgb'], atol=1e-5, rtol=1e-6)

@@ -192,7 +192,7 @@ __device__ __forceinline__ void blend_quads(const FoamScene& S, float color_cut,
     if (cell >= 0) base = S.offsets[cell], e1 = S.offsets[cell + 1];
     float m = kInf, A = 0.f, cr = 0.f, cg = 0.f, cb = 0.f;
     for (; wave_any(base < e1); base += 4) {
-        const int e = entry_in(base + lane % 4, e1);  // an absent entry: another's records, weight 0
+        const int e = entry_in(base + lane % 4, e1);  // an absent entry: another's records, left out
         const float4 ed = S.edge[e];
         const int k = IDX ? __float_as_int(ed.w) : S.nbr[e];
         const float4* row = S.sh + S.sh_stride * static_cast<int64_t>(k);
@@ -237,7 +237,7 @@ __device__ __forceinline__ void blend_quads(const FoamScene& S, float color_cut,
         mk[3] = distance(std::integral_constant<int, 0xFF>{}, 3, lb[3]);
         float low = m;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {  // a term left out (absent, NaN, or beyond the cut-off): +inf, weight 0
+        for (int r = 0; r < 4; ++r) {  // a term left out (absent, NaN, or beyond the cut-off): kInf, weight 0
             const float lim = CUT ? low + color_cut : kInf;
             const bool in = base + r < e1 && (!CUT || lb[r] <= lim) && mk[r] <= lim;
             mk[r] = in ? mk[r] : kInf;
@@ -247,11 +247,14 @@ __device__ __forceinline__ void blend_quads(const FoamScene& S, float color_cut,
         A *= keep, cr *= keep, cg *= keep, cb *= keep, m = low;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const float c[3] = {fmaxf(c0[r], 0.f), fmaxf(c1[r], 0.f), fmaxf(c2[r], 0.f)};
+            // max(c, 0); the colour of a term left out is also kept finite, lest 0 * inf make a NaN of the blend
+            const float top = mk[r] < kInf ? __builtin_huge_valf() : kInf;
+            const float c[3] = {__builtin_amdgcn_fmed3f(c0[r], 0.f, top), __builtin_amdgcn_fmed3f(c1[r], 0.f, top),
+                                __builtin_amdgcn_fmed3f(c2[r], 0.f, top)};
             accumulate(A, cr, cg, cb, weight_of(mk[r], low), c);
         }
     }
-    const float inv = 1.f / A;
+    const float inv = m < kInf ? 1.f / A : __builtin_nanf("");  // every term left out: 0 / 0, as in the other layouts
     C[0] = cr * inv, C[1] = cg * inv, C[2] = cb * inv;
 }
 
