@@ -81,9 +81,11 @@ int vgr_foam_infer_traced(const float* points, int64_t n_sites, const int32_t* o
  * for the full rendering of up to 98304 rays 16 lanes per ray, whose densities are summed in the order of one ray per
  * lane, so T, traces and stats have that layout's bits; beyond, and for stages 0 and 1, 4 lanes per ray for stages 0 and 1
  * and lazy colours, one ray per lane for fused and baked colours). One ray per lane evaluates fused colours for the
- * samples of segments with weight > w_thresh only; without a cut-off its stats[:, 4] counts every entry of a pass. Fused and
- * baked colours with a finite color_cut always run one ray per lane (their neighbour skipping follows the edge
- * order). trace may be NULL (then trace_cap is ignored). order (NULL = the batch order): a permutation of
+ * samples of segments with weight > w_thresh only. stats[:, 4] counts the lookups of entries whose colour distance is a
+ * number and within the cut-off, in every layout (with slots and 2 or 4 lanes per ray: of all entries beside a site whose
+ * distances are none). Fused and baked colours with a finite color_cut run one ray per lane where a group was asked for
+ * (their neighbour skipping follows the edge order; 16 lanes per ray follow it too). trace may be NULL (then trace_cap is
+ * ignored). order (NULL = the batch order): a permutation of
  * 0 .. B - 1 giving the order in which the rays are traced (vgr_ray_order); results are the same in any order, an
  * entry outside [0, B) is skipped. slots (NULL = none): the slot table of vgr_foam_slot_table for this pack; with
  * color_cut = +inf the reference's cache misses (stats[:, 4]) then come from it once per neighbourhood pass instead
@@ -419,6 +421,8 @@ int vgr_ray_order(const float* o, const float* d, int64_t n_rays, int32_t dir_re
  * 183-184, 212-213, 269-272). This layout carries both in one record: edge_i[e] = (p_j, the bits of j = nbr[e])
  * and attr_i = attr with column 7 (zero padding in the reference layout) holding the bits of site k's cut-off word
  * half2(r2_k, lam_k), which every record pointing at k carries in edge[:, 3] (the self entry's, edge[offsets[k]]).
+ * The sign of r2_k, which is never negative, marks a site whose colour distances need not be numbers: a coefficient of its
+ * colour conic not finite or above 1e18, its position not finite or beyond 1e9, or lam_k not a number.
  *   offsets i32 (N + 1), nbr i32 (E), edge f32 (E, 4), attr f32 (N, 20) as for vgr_foam_infer
  *   -> edge_i f32 (E, 4), attr_i f32 (N, 20); a snapshot: rebuild after changing the pack.
  */

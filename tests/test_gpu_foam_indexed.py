@@ -75,6 +75,26 @@ def test_index_pack_layout(gpu, small):
 		np.testing.assert_array_equal(ai[:, keep].view(np.int32), pk['attr'][:, keep].view(np.int32))
 
 
+def test_index_pack_marks_degenerate_sites(gpu, small):
+	"""The word of a site whose colour distances need not be numbers (a conic coefficient not finite or above 1e18, a position
+	not finite or beyond 1e9, lam not a number) carries the mark 0x8000, and nothing else changes."""
+	pk = small[0].pack(eps_density=1e-3)
+	t = lambda a: torch.as_tensor(np.ascontiguousarray(a), device=gpu)  # noqa: E731
+	even, attr = ext.index_pack(*[t(pk[k]) for k in ('offsets', 'nbr', 'edge', 'attr')])
+	for k, col, v in ((3, 8, np.inf), (4, 13, np.nan), (5, 10, -2e18), (6, 11, 1e18)):
+		pk['attr'][k, col] = v
+	own = pk['offsets'][:-1]
+	pk['edge'][own[7], 0], pk['edge'][own[8], 2], pk['edge'][own[9], 1] = 2e9, np.nan, -1e9
+	pk['edge'].view(np.uint32)[own[10], 3] = 0x7e003c00  # lam NaN
+	ei, ai = ext.index_pack(*[t(pk[k]) for k in ('offsets', 'nbr', 'edge', 'attr')])
+	word = pk['edge'].view(np.int32)[own, 3]
+	word[[3, 4, 5, 7, 8, 10]] |= 0x8000
+	np.testing.assert_array_equal(ai.cpu().numpy()[:, 7].view(np.int32), word)
+	keep = [c for c in range(20) if c != 7]
+	np.testing.assert_array_equal(ai.cpu().numpy()[:, keep], pk['attr'][:, keep])
+	np.testing.assert_array_equal(ei.cpu().numpy()[:, 3].view(np.int32), even.cpu().numpy()[:, 3].view(np.int32))
+
+
 @pytest.mark.parametrize('sh_deg', [0, 1, 2, 3])
 @pytest.mark.parametrize('sh_half', [False, True])
 def test_indexed_identical_small_field(gpu, small, sh_deg, sh_half):

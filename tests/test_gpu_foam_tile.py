@@ -136,3 +136,33 @@ def test_terms_left_out_add_nothing(gpu, hub, sh_half, indexed):
 		bad = np.isnan(wide['rgb']).any(1)
 		assert bad.any() and not bad.all()
 		np.testing.assert_allclose(g['rgb'], wide['rgb'], atol=1e-5, rtol=1e-6)
+
+
+@pytest.mark.parametrize('indexed,slots,mode', CASES)
+@pytest.mark.parametrize('reorder', [False, True])
+def test_lookups_whose_distance_is_no_number(gpu, hub, indexed, slots, mode, reorder):
+	"""Without a cut-off the counted lookups are the entries whose colour distance is a number: all, except beside sites of
+	degenerate colour conics (all or one coefficient not finite, or finite ones whose distance overflows) and at samples so
+	far out, or at no place at all, that distances overflow. The same counts as 16 lanes per ray, which look entry by entry,
+	so that a batch's size does not change them; the oracle's for fused colours and the conics."""
+	f, (o, d, start, near, _, far) = hub
+	pk = f.pack(reorder=reorder)
+	start = pk['inv'][start].astype(np.int32) if reorder else start
+	pk['attr'][5::37, 8:14] = np.inf
+	pk['attr'][7::41, 9] = np.nan
+	pk['attr'][11::43, 8] = 3e38
+	rays = (o, d, start, near, far)
+	all_entries = run(gpu, f.pack(reorder=reorder), 3, rays, 0.0, -1.0, mode, indexed=indexed, slots=slots)['stats']
+	for tt, wt in ((0.0, -1.0), (1e-4, 1e-3)):
+		g = run(gpu, pk, 3, rays, tt, wt, mode, indexed=indexed, slots=slots)
+		wide = run(gpu, pk, 3, rays, tt, wt, mode, lanes=None)
+		np.testing.assert_array_equal(g['stats'], wide['stats'])
+	g = run(gpu, pk, 3, rays, 0.0, -1.0, mode, indexed=indexed, slots=slots)
+	assert (g['stats'][:, 4] < all_entries[:, 4]).sum() > 50
+	if mode == 2:  # the oracle's two-pass exact colours take such a term in, and are NaN
+		np.testing.assert_array_equal(g['stats'], ref_foam(pk, 3, *rays, 0.0, -1.0, color_mode=2)['stats'])
+	out = far.copy()
+	out[::3], out[1::5], out[2::7] = 3e19, np.inf, np.nan
+	g = run(gpu, pk, 3, (o, d, start, near, out), 0.0, -1.0, mode, indexed=indexed, slots=slots)
+	wide = run(gpu, pk, 3, (o, d, start, near, out), 0.0, -1.0, mode, lanes=None)
+	np.testing.assert_array_equal(g['stats'], wide['stats'])

@@ -165,3 +165,22 @@ def test_derived_records_of_the_pack_match_their_own_kernels(gpu, n, sh_half):
 		if reorder:
 			assert torch.equal(a['perm'], torch.sort(render.morton_codes(m.graph.points), stable=True)[1])
 			assert torch.equal(a['inv'][a['perm']], torch.arange(f.n, device=gpu))
+
+
+@pytest.mark.parametrize('reorder', [False, True])
+def test_derived_records_mark_degenerate_sites(gpu, reorder):
+	"""pack_foam(index=True) marks the sites that index_pack marks: colour conics that are not numbers (a NaN quaternion)."""
+	from helpers import Field
+	from vgr.model import VoronoiGaussField
+	f = Field(seed=4, n=300)
+	T = lambda a: torch.as_tensor(a, device=gpu)  # noqa: E731
+	m = VoronoiGaussField(T(f.points), T(f.offsets), T(f.adj), torch.zeros(f.n, 3, device=gpu),
+						  torch.ones(f.n, device=gpu))
+	with torch.no_grad():
+		m.c_quat[::17] = float('nan')
+	a = render.pack_foam(m, eps_density=1e-3, reorder=reorder)
+	b = render.index_pack(render.pack_foam(m, eps_density=1e-3, reorder=reorder, index=False))
+	marked = (a['attr_i'].view(torch.int32)[:, 7] & 0x8000) != 0
+	assert torch.equal(marked, torch.isnan(a['attr'][:, 8])) and 0 < marked.sum() < f.n // 8
+	for k in ('attr_i', 'rows', 'edge_i', 'edge'):
+		assert torch.equal(a[k].view(torch.int32), b[k].view(torch.int32)), k

@@ -929,7 +929,8 @@ __global__ void __launch_bounds__(kBlock, (waves_for<COLOR, kBlock / G, TABLE>(S
 
 // Indexed edge records from a pack: edge_i[e] = (p_j, the bits of j = nbr[e]) for every entry, and attr_i = attr with
 // column 7 (padding in the reference's layout) holding site k's cut-off word, which every edge record pointing at k
-// carries in the reference's layout (the self entry's, edge[offsets[k]].w). One lane per float4 written.
+// carries in the reference's layout (the self entry's, edge[offsets[k]].w), with the site's mark (kOddSite). One lane per
+// float4 of edge_i, per float of attr_i.
 __global__ void __launch_bounds__(256) index_pack_kernel(const int* __restrict__ offsets, const int* __restrict__ nbr,
                                                          const float4* __restrict__ edge, const float* __restrict__ attr,
                                                          int64_t n_sites, int64_t n_edges, float4* __restrict__ edge_i,
@@ -948,7 +949,12 @@ __global__ void __launch_bounds__(256) index_pack_kernel(const int* __restrict__
         attr_i[j] = attr[j];
     } else {  // the self entry's word; 0 for a site without entries (never a neighbour of a consistent graph)
         const int e0 = offsets[k];
-        attr_i[j] = e0 < offsets[k + 1] && e0 < n_edges ? edge[e0].w : 0.f;
+        if (e0 < offsets[k + 1] && e0 < n_edges) {
+            const float4 ed = edge[e0];
+            attr_i[j] = mark_site(ed.w, attr + 20 * k + 8, ed.x, ed.y, ed.z);
+        } else {
+            attr_i[j] = 0.f;
+        }
     }
 }
 

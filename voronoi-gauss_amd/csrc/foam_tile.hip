@@ -23,8 +23,9 @@
 // also takes the colour distances, since the lookups they admit are counted (stats[:, 4]), and the evaluation, which visits
 // a cell's entries in the same order with the same operations, admits the same terms.
 //
-// stats[:, 4], the reference's cache misses: without a cut-off every pass looks up all entries, so the count needs the cells:
-// from the slot table with the ray's 8 tags in registers, or, without a table, from tags per lookup in LDS. EXACT: the exact
+// stats[:, 4], the reference's cache misses: without a cut-off a pass looks up all entries whose colour distance is a number,
+// which but for degenerate sites is all of them, so that the count needs the cells: from the slot table with the ray's 8 tags
+// in registers (count_lookups), or, without a table, from tags per lookup in LDS. EXACT: the exact
 // (lazy) colour mode by the same one-pass blend. Its colour, sum_k exp(-(m_k - m_min) / 2) c_k / sum_k exp(-(m_k - m_min) / 2)
 // over every neighbour, is the blend's two sums up to rounding; its statistics count a colour pass only where the reference
 // runs one: for the far sample of a segment heavier than w_thresh and, when the segment before was not, its near sample.
@@ -98,8 +99,14 @@ __device__ int walk(const FoamScene& S, int c, float x0, float x1, float x2, int
 
 struct Pass {
     float sigma, t_exit;
-    int next, n;  // exit neighbour, entries of the cell
+    int next;  // exit neighbour
+    int n;     // entries of the cell; ~entries when the pass may not look all of them up (count_lookups)
 };
+
+// Every pass looks up the entries of its cell whose colour distance is a number (without a cut-off). That is every entry,
+// except beside a site whose colour conic is not finite, or so far out that the distance overflows. Where distances are not
+// taken, such a pass is told by vgr_foam.h's kOddSite, which the indexed records carry per site, and by the sample's position.
+constexpr float kOddPosition = 1e9f;  // as kOddSite: 9 terms of at most 1e18 * (2e9)^2 stay below FLT_MAX
 
 // Density at o + t d over the neighbourhood of c and, when want_exit, the exit face: foam_infer.hip's sequential pass (the
 // same operations in the same order). The next edge record is requested while the current entry is evaluated.
@@ -108,6 +115,7 @@ struct Pass {
 template <bool IDX, bool TAGS, bool CUT>
 __device__ __forceinline__ Pass pass(const FoamScene& S, int c, float t, const float (&o)[3], const float (&d)[3],
                                      bool want_exit, int& n_dens, int& n_sh, lds_int* tags, float color_cut) {
+    constexpr bool DIST = CUT || TAGS || !IDX;  // the pass takes the colour distances
     const int e0 = S.offsets[c], e1 = S.offsets[c + 1];
     float4 edn = S.edge[entry_in(e0, e1)];
     int kn = 0;
@@ -117,13 +125,15 @@ __device__ __forceinline__ Pass pass(const FoamScene& S, int c, float t, const f
     sample_point(o, d, t, x);
     Pass R{0.f, kInf, INT_MAX, e1 - e0};
     float low = kInf;
+    uint32_t words = 0;
+    bool odd = !DIST && !(fabsf(x[0]) <= kOddPosition && fabsf(x[1]) <= kOddPosition && fabsf(x[2]) <= kOddPosition);
     for (int e = e0; e < e1; ++e) {
         const float4 ed = edn;
         const int k = IDX ? __float_as_int(ed.w) : kn;
         const float4* a = S.attr + 5 * static_cast<int64_t>(k);
         const float4 q0 = a[0], q1 = a[1];
         float4 q2, q3;
-        if constexpr (CUT) q2 = a[2], q3 = a[3];
+        if constexpr (DIST) q2 = a[2], q3 = a[3];
         const int en = min(e + 1, e1 - 1);
         edn = S.edge[en];
         if constexpr (!IDX) kn = S.nbr[en];
@@ -140,20 +150,23 @@ __device__ __forceinline__ Pass pass(const FoamScene& S, int c, float t, const f
         }
         float v0, v1, v2, r2;
         offset_of(x, ed, v0, v1, v2, r2);
-        const float2 cut = cutoffs(IDX ? q1.w : ed.w);
-        if (r2 <= cut.x) {
+        const float word = IDX ? q1.w : ed.w;
+        const float2 cut = cutoffs(word);
+        if (!DIST) words |= __float_as_uint(word);
+        if (r2 <= (IDX ? fabsf(cut.x) : cut.x)) {
             R.sigma += density_term(q0, q1, v0, v1, v2);
             ++n_dens;
         }
         bool look = true;
-        if constexpr (CUT) {
-            const float lim = low + color_cut;
+        if constexpr (DIST) {
+            const float lim = CUT ? low + color_cut : color_cut;
             look = r2 * cut.y <= lim;
             if (look) {
                 const float m = maha_f(q2, q3, v0, v1, v2);
                 look = m <= lim;
-                low = look && m < low ? m : low;
+                if (CUT) low = look && m < low ? m : low;
             }
+            odd = odd || !look;
         }
         if (TAGS && look) {
             lds_int* p = tags + (k & (kRayTagSlots - 1)) * kBlock;
@@ -161,6 +174,7 @@ __device__ __forceinline__ Pass pass(const FoamScene& S, int c, float t, const f
             *p = k;
         }
     }
+    if (!TAGS && (odd || (words & kOddSite) != 0)) R.n = ~R.n;
     return R;
 }
 
@@ -177,6 +191,34 @@ __device__ __forceinline__ int table_hits(const FoamScene& S, int c, int (&tag)[
         tag[2 * q + 1] = v.w >= 0 ? v.w : tag[2 * q + 1];
     }
     return hits;
+}
+
+// The reference's cache misses of the pass over cell c at o + t d, without a cut-off: of all n entries by the slot table, or
+// (n = ~entries, rare) of those whose colour distance is a number, entry by entry.
+template <bool IDX>
+__device__ __forceinline__ int count_lookups(const FoamScene& S, int c, int n, float t, const float (&o)[3],
+                                             const float (&d)[3], int (&tag)[kRayTagSlots]) {
+    if (n >= 0) return n - table_hits(S, c, tag);
+    float x[3];
+    sample_point(o, d, t, x);
+    int misses = 0;
+    const int e0 = S.offsets[c];
+    for (int e = e0; e < e0 + ~n; ++e) {
+        const float4 ed = S.edge[e];
+        const int k = IDX ? __float_as_int(ed.w) : S.nbr[e];
+        const float4* a = S.attr + 5 * static_cast<int64_t>(k);
+        float v0, v1, v2, r2;
+        offset_of(x, ed, v0, v1, v2, r2);
+        const float lb = r2 * cutoffs(IDX ? a[1].w : ed.w).y, m = maha_f(a[2], a[3], v0, v1, v2);
+        if (lb != lb || m != m) continue;
+#pragma unroll
+        for (int s = 0; s < kRayTagSlots; ++s) {
+            const bool here = (k & (kRayTagSlots - 1)) == s;
+            misses += here && tag[s] != k ? 1 : 0;
+            tag[s] = here ? k : tag[s];
+        }
+    }
+    return misses;
 }
 
 // Blends of 64 samples, one per lane, the four samples of a quad in one cell (`cell`, -1 for a quad without samples): lane l
@@ -356,7 +398,7 @@ __global__ void __launch_bounds__(kBlock, kWaves) foam_tile_kernel(FoamScene S, 
         cA = walk<IDX>(S, start, o[0] + tA * d[0], o[1] + tA * d[1], o[2] + tA * d[2], walk_steps);
         E = pass<IDX, !TABLE, CUT>(S, cA, tA, o, d, true, n_dens, n_sh, my_tags, P.color_cut);
         nA = E.n;
-        if (TABLE && !EXACT) n_sh += E.n - table_hits(S, cA, tag);
+        if (TABLE && !EXACT) n_sh += count_lookups<IDX>(S, cA, E.n, tA, o, d, tag);
         if (O.trace != nullptr) trace_cell<true>(S, O, r, 0, cA);
         n_samples = 1;
     }
@@ -372,7 +414,7 @@ __global__ void __launch_bounds__(kBlock, kWaves) foam_tile_kernel(FoamScene S, 
             const float tB = last ? t_far : fmaxf(E.t_exit, tA);
             const int cB = last ? cA : E.next;
             E = pass<IDX, !TABLE, CUT>(S, cB, tB, o, d, !last, n_dens, n_sh, my_tags, P.color_cut);
-            if (TABLE && !EXACT) n_sh += E.n - table_hits(S, cB, tag);
+            if (TABLE && !EXACT) n_sh += count_lookups<IDX>(S, cB, E.n, tB, o, d, tag);
             if (O.trace != nullptr) trace_cell<true>(S, O, r, n_samples, cB);
             ++n_samples;
             const float delta = tB - tA;
@@ -382,8 +424,9 @@ __global__ void __launch_bounds__(kBlock, kWaves) foam_tile_kernel(FoamScene S, 
             const float half = lit ? 0.5f * w : 0.f;
             if (lit) {
                 if constexpr (EXACT) {
-                    if (!lit_before) n_sh += nA - table_hits(S, cA, tag);
-                    n_sh += E.n - table_hits(S, cB, tag);
+#pragma unroll 1  // one copy of the rare part: two spill 17 more VGPRs
+                    for (int far = lit_before ? 1 : 0; far < 2; ++far)
+                        n_sh += count_lookups<IDX>(S, far ? cB : cA, far ? E.n : nA, far ? tB : tA, o, d, tag);
                 }
                 dep += w * 0.5f * (tA + tB);
                 ++n_color;

@@ -26,6 +26,7 @@
 
 #include "vgr_abi.h"
 #include "vgr_device.h"
+#include "vgr_foam.h"
 #include "vgr_scan.h"
 #include "vgr_bbox.h"
 
@@ -59,7 +60,7 @@ __device__ __forceinline__ int old_of(const PackIn& P, int i) {
 // What the pack writes beside the reference's records (any of them may be null).
 struct PackIndex {
     float4* __restrict__ edge_i;  // (E) p_j, the bits of j
-    float4* __restrict__ attr_i;  // (N, 5) attr with column 7 = the site's cut-off word
+    float4* __restrict__ attr_i;  // (N, 5) attr with column 7 = the site's cut-off word with its mark (kOddSite)
     int4* __restrict__ slots;     // (N, 4) slot table
     float4* __restrict__ rows;    // (N, row_vec) site rows: the first 16 columns of attr_i, then (row_vec 16) the SH row
     int row_vec;                  // 4 or 16 float4
@@ -115,7 +116,7 @@ __global__ void __launch_bounds__(kBlock)
         float* a = rec + kSiteStride * threadIdx.x;
 #pragma unroll
         for (int k = 0; k < 6; ++k) a[k] = P.dA[6 * o + k], a[8 + k] = P.cA[6 * o + k];
-        a[6] = raw, a[7] = cut;
+        a[6] = raw, a[7] = mark_site(cut, a + 8, x, y, z);
 #pragma unroll
         for (int k = 14; k < 20; ++k) a[k] = 0.f;
     }

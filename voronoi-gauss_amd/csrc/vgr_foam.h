@@ -24,6 +24,19 @@ struct FoamScene {
     int sh_stride;   // float4 from one SH row to the next: 12 (fp32), 6 (fp16) or 16 (the SH rows of site blocks)
 };
 
+// Mark of a site in its word of the indexed records (the sign of half2(r2, lam)'s r2, which is never negative): a colour
+// distance to it need not be a number. Its colour conic is not finite or above 1e18, its position not finite or beyond 1e9, or
+// its bound lam not a number; of every other site, from samples within 1e9, the distance and its bound are finite.
+constexpr uint32_t kOddSite = 0x8000u;
+
+__device__ __forceinline__ float mark_site(float word, const float* conic, float px, float py, float pz) {
+    const uint32_t u = __float_as_uint(word), lam = u >> 16;
+    bool even = (lam & 0x7c00u) != 0x7c00u && fabsf(px) <= 1e9f && fabsf(py) <= 1e9f && fabsf(pz) <= 1e9f;
+#pragma unroll
+    for (int q = 0; q < 6; ++q) even = even && fabsf(conic[q]) <= 1e18f;
+    return __uint_as_float(even ? u : u | kOddSite);
+}
+
 struct FoamParams {
     float t_thresh, w_thresh, color_cut;
     int sh_deg;
