@@ -265,3 +265,29 @@ def test_site_rows_identical_in_group_layouts(gpu, small, lanes):
 		ext.foam_infer_extension().foam_infer(
 			tens['points'], tens['offsets'], tens['nbr'], tens['edge'], tens['attr'], tens['sh'].half(), 3, t(o), t(d),
 			t(st), t(near), t(far), 1e-4, 1e-4, math.inf, 2, 2, empty, orig, lanes=lanes, indexed=(ei, ai, blocks))
+
+
+@pytest.mark.parametrize('sh_half', [False, True])
+@pytest.mark.parametrize('cut', [math.inf, 2 * math.log(1e3)])
+def test_site_rows_identical_in_the_default_layout(gpu, small, sh_half, cut):
+	"""Small batches by the default layout (16 lanes per ray): every colour mode with site rows or blocks, which some modes
+	read and others leave aside, gives the outputs of the attr rows bit for bit."""
+	f, (o, d, start, near, _, far) = small
+	t = lambda a: torch.as_tensor(np.ascontiguousarray(a), device=gpu)  # noqa: E731
+	empty = torch.empty(0, dtype=torch.int32, device=gpu)
+	pk = f.pack(eps_density=1e-3, sh_half=sh_half)
+	pk['attr'][:, 16:19] = np.random.default_rng(3).uniform(0, 1, (f.n, 3))
+	scene = [t(pk[k]) for k in ('points', 'offsets', 'nbr', 'edge', 'attr', 'sh')]
+	ei, ai = ext.index_pack(*scene[1:5])
+	rows = ai[:, :16].contiguous()
+	records = [(ei, ai), (ei, ai, rows)]
+	if not sh_half:
+		records.append((ei, ai, torch.cat([rows, scene[5].reshape(-1, 48)], 1).contiguous()))
+	for mode in (0, 1, 2):
+		outs = []
+		for idx in records:
+			out = ext.foam_infer_extension().foam_infer(*scene, 3, t(o), t(d), t(start), t(near), t(far), 1e-4, 1e-4, cut, mode, 2,
+														empty, empty, trace_cap=256, indexed=idx)
+			outs.append(dict(zip(FIELDS, [x.cpu().numpy() for x in out])))
+		for other in outs[1:]:
+			assert_identical(outs[0], other)

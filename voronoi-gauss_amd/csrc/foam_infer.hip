@@ -1115,10 +1115,18 @@ int foam_entry(const float* points, int64_t n_sites, const int32_t* offsets, con
     if (stage == 2 && color_mode != kLazy && !(color_cut > 1e30)) lanes = 1;
     // The site rows serve the group layouts' fused blend (config 5's 8-lane batch: 2538.6 -> 2437.6 ms with the
     // 64-byte rows); the two-pass exact colours with 4 lanes per ray ran slower on them (268.9 against 258.3 ms on
-    // config 3) and keep the attr rows, as the one-ray-per-lane kernels do. Site blocks also supply those kernels'
-    // SH rows, 16 float4 apart after each 4-float4 record.
+    // config 3) and keep the attr rows, as the one-ray-per-lane kernels do. Site blocks also supply the SH rows of the
+    // kernels that read them, 16 float4 apart after each 4-float4 record.
+    // 16 lanes per ray read 64-byte rows (fp16 SH, 65536 incoherent rays 1.98 -> 1.80 ms, coherent ones the same), and blocks
+    // where the SH row follows the record: exact and fused colours. Baked colours have no SH row, and exact ones with a
+    // cut-off read few of them: there a coherent batch pays for lines it does not use (8x8 tiles, baked: 98304 rays 1.67 ms
+    // with blocks, 1.44 without, 1.59 with one ray per lane; exact, eps 1e-3: 65536 rays 3.2 and 3.8 ms with blocks, 2.4 and
+    // 2.9 without, 2.7 and 3.4 with 4 lanes per ray; incoherent rays 1.82 and 1.25 ms, 2.2 and 2.4).
+    const bool cut_off = !(std::isinf(color_cut) && color_cut > 0);
+    const bool wide_rows =
+        wide && (row_floats == 16 ? color_mode != kBaked : color_mode == kFused || (color_mode == kLazy && !cut_off));
     const bool rows_used =
-        rows != nullptr && stage == 2 && (wide || (!indexed && color_mode == kFused && lanes > 1));
+        rows != nullptr && stage == 2 && (wide ? wide_rows : !indexed && color_mode == kFused && lanes > 1);
     const bool blocks = rows_used && row_floats == 64;
     const FoamScene S{reinterpret_cast<const float4*>(points),
                       offsets,
