@@ -87,7 +87,7 @@ def test_nearest_sites_dispatch_and_errors(gpu):
 	dev = sites.nearest_sites(T(pts, gpu), T(q, gpu))
 	assert isinstance(host, np.ndarray) and dev.is_cuda and dev.dtype == torch.int32
 	np.testing.assert_array_equal(dev.cpu().numpy(), host)
-	# a batch above 65,536 queries is answered in its Z-order: the same answers
+	# a batch above 65,536 queries is answered cell by cell: the same answers
 	qb = rng.uniform(-1.2, 1.2, (100000, 3)).astype(np.float32)
 	np.testing.assert_array_equal(sites.nearest_sites(T(pts, gpu), T(qb, gpu)).cpu().numpy(),
 								  sites.nearest_sites(pts, qb))
@@ -148,3 +148,24 @@ def test_points_box(gpu, n, stride):
 		want = torch.cat([pts[:, :3].amin(0), pts[:, :3].amax(0)])
 		assert torch.equal(torch.isnan(box[:6]), torch.isnan(want))
 		assert torch.equal(box[:6].nan_to_num(7.0), want.nan_to_num(7.0))
+
+
+@pytest.mark.parametrize('m', [65536, 65537, 131072])
+@pytest.mark.parametrize('per_cell', [2.0, 0.02])
+def test_binning_follows_queries_and_cells(gpu, m, per_cell, monkeypatch):
+	"""A batch is binned above 65,536 queries where it is not small beside the grid's cells (1.5M of them with 0.02 sites per
+	cell: one query per 16 cells from 93,750 on), with the same answers on both sides of the line."""
+	from vgr import _lib
+	rng = np.random.default_rng(16)
+	pts = rng.uniform(-1, 1, (30000, 3)).astype(np.float32)
+	q = rng.uniform(-1.1, 1.1, (m, 3)).astype(np.float32)
+	g = grid.SiteGrid(T(pts, gpu), per_cell=per_cell)
+	n_cells = len(g.cell_start) - 1
+	assert (n_cells > 16 * 65537) == (per_cell < 1) and n_cells <= 16 * 131072
+	names, call = [], _lib.call
+	monkeypatch.setattr(_lib, 'call', lambda name, *a: (names.append(name), call(name, *a))[1])
+	got = g.nearest(T(q, gpu))
+	assert names == ['vgr_grid_nearest_binned' if m > 65536 and 16 * m >= n_cells else 'vgr_grid_nearest_points']
+	monkeypatch.undo()
+	assert torch.equal(got, torch.cat([g.nearest(T(q[a:a + 65536], gpu)) for a in range(0, m, 65536)]))
+	np.testing.assert_array_equal(got.cpu().numpy()[:500], dense.nearest_brute(pts, q[:500]))

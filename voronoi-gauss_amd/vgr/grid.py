@@ -13,8 +13,14 @@ import torch
 from . import _lib
 
 
-# Batches above this many queries are binned before they are answered.
-BINNED_QUERIES = 65536
+# Batches above this many queries, and of at least one query per BINNED_CELLS cells, are binned before they are answered. The
+# binning clears and scans a counter per cell and writes the queries again; it pays where queries differ in how many cells
+# they scan. One MI355X, ms query by query : binned, of a grid that is kept:
+#   clustered sites, queries around them   20k sites 65537 queries 0.24 : 0.19, 1M sites 2.3 : 1.6, 1M queries 7.8 : 3.7
+#   uniform sites, queries over the cube   1M sites 65537 queries 0.07 : 0.10, 1M 0.23 : 0.24, 4M 0.79 : 0.67; a batch of
+#                                          near ones costs up to 0.1 more binned, one whose queries lie outside half
+#   31M sites, 15.6M cells                 65537 queries 0.06 : 0.17 uniform, 4.4 : 4.7 clustered; 1M 0.34 : 0.47, 15.7 : 10.6
+BINNED_QUERIES, BINNED_CELLS = 65536, 16
 
 
 class SiteGrid:
@@ -60,8 +66,8 @@ class SiteGrid:
 	def nearest(self, queries, order=None):
 		"""Index (int32) of the nearest site of every query point: queries (m, 3) float32 CUDA tensor. order:
 		optional int32 (m,) permutation of 0 .. m - 1, the order in which the queries are answered (query_order
-		gives a coherent one); the answers do not depend on it. Without an order, batches above 65,536 queries are
-		binned into the grid's cells first and answered cell by cell."""
+		gives a coherent one); the answers do not depend on it. Without an order, batches above 65,536 queries and
+		a sixteenth of the grid's cells are binned into the cells first and answered cell by cell."""
 		if not (isinstance(queries, torch.Tensor) and queries.is_cuda):
 			raise RuntimeError('queries must be a CUDA tensor')
 		if queries.dtype != torch.float32 or queries.dim() != 2 or queries.shape[1] != 3 or not queries.is_contiguous():
@@ -70,8 +76,9 @@ class SiteGrid:
 									  and order.shape == (len(queries),) and order.is_contiguous()):
 			raise RuntimeError('order must be a contiguous int32 CUDA tensor of one entry per query')
 		out = torch.empty(len(queries), dtype=torch.int32, device=queries.device)
-		if order is None and BINNED_QUERIES < len(queries) < 2 ** 31:
-			wb = int(_lib.load().vgr_grid_binned_work_size(len(queries), len(self.cell_start) - 1))
+		n_cells = len(self.cell_start) - 1
+		if order is None and BINNED_QUERIES < len(queries) < 2 ** 31 and BINNED_CELLS * len(queries) >= n_cells:
+			wb = int(_lib.load().vgr_grid_binned_work_size(len(queries), n_cells))
 			work = torch.empty(wb, dtype=torch.uint8, device=queries.device)
 			_lib.call('vgr_grid_nearest_binned', _lib.ptr(self.cell_points), self.n, *self._geom,
 					  _lib.ptr(self.cell_start), _lib.ptr(queries), len(queries), _lib.ptr(work), wb, _lib.ptr(out),
