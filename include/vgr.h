@@ -171,7 +171,7 @@ int vgr_march_backward(const float* points, int64_t n_sites, const int32_t* offs
 
 /*
  * The march of a training step with 16 lanes per ray (vgr_march_forward_lanes) that leaves visit records for its backward:
- * visits f32 (B, visit_cap, 8), per run of at most 32 samples in one cell (cell bits, index of its first sample bits,
+ * visits f32 (B, visit_cap, 8), per run of at most 34 samples in one cell (cell bits, index of its first sample bits,
  * transmittance and composited rgb before it, unused x 2), and n_visits i32 (B), the runs of each ray (0: not traced, more
  * than visit_cap: its records are incomplete). vgr_march_backward_visits replays the runs independently of each other, rays
  * with incomplete records as vgr_march_backward does, and takes the forward's stats; n_rays <= 2^22.

@@ -122,7 +122,7 @@ def test_march_backward_edge_cases(gpu):
 @pytest.mark.parametrize('cap', [1, 24, 256])
 @pytest.mark.parametrize('dt', [1 / 16, 1 / 256])
 def test_backward_of_recorded_visits(gpu, n_rays, cap, dt):
-	"""The backward from the forward's visit records (runs of up to 32 samples in a cell, replayed on their own) against the
+	"""The backward from the forward's visit records (runs of up to 34 samples in a cell, replayed on their own) against the
 	backward that marches every ray again: records that all fit, some and none, steps longer than a cell and many steps per
 	cell. The samples replay with the forward's bits and the sums run in another order: 1e-5. The forward's outputs do not
 	depend on the records."""
@@ -148,3 +148,30 @@ def test_backward_of_recorded_visits(gpu, n_rays, cap, dt):
 	want = fx.march_backward(*args, outs[0], outs[1], *up, lanes=16)
 	for a, b in zip(got, want):
 		assert torch.isfinite(a).all() and (a.double() - b.double()).norm() <= 1e-5 * b.double().norm() + 1e-30
+
+
+@pytest.mark.parametrize('n_rays', [1, 4099, (1 << 19) - 1, 1 << 19])
+def test_march_without_gradients(gpu, n_rays):
+	"""ext.march without gradients takes the layout by batch size and leaves no records: the bits of the forward under
+	autograd below 2^19 rays (16 lanes per ray in both), and from there on one ray per lane, whose sums run in the order of
+	the neighbourhood: the same samples, colours of at most ~3 by sums of at most ~30 terms each to a few ulps."""
+	f = Field(seed=9, n=300)
+	o, d, start, near, mid, far = f.rays(B=min(n_rays, 4099), seed=9)
+	dA, cA = f.conics(0.01)
+	rays = [torch.as_tensor(np.resize(a, (n_rays,) + a.shape[1:]), device=gpu) for a in (o, d, start, near, mid, far)]
+	graph = ext.Graph(*[T(a, gpu) for a in (f.points, f.offsets, f.adj)])
+	params = [T(a, gpu) for a in (f.raw, dA, cA, f.sh)]
+	plain = ext.march(graph, *params, 3, *rays, DT, NBG)
+	with torch.no_grad():
+		off = ext.march(graph, *[p.clone().requires_grad_() for p in params], 3, *rays, DT, NBG)
+	grad = ext.march(graph, *[p.clone().requires_grad_() for p in params], 3, *rays, DT, NBG)
+	for a, b, c in zip(plain, off, grad):
+		assert not a.requires_grad and torch.equal(a, b)
+		if n_rays < 1 << 19:
+			assert torch.equal(a, c.detach())
+		elif a.dtype == torch.int32:
+			assert (a == c).all(1).float().mean() > 0.999  # a weight within ulps of the threshold is coloured or not
+		else:
+			# such a segment moves its ray by its weight, 1e-4
+			near_ = (a - c.detach()).abs()
+			assert near_.max() < 5e-4 and (near_ < 1e-5).float().mean() > 0.999

@@ -1012,9 +1012,10 @@ __device__ __forceinline__ void group_colour_n(const MarchField& F, GroupCell& C
     }
 }
 
-// The visits a forward leaves for its backward: per ray up to `cap` records of 8 floats, one per run of at most
-// kVisitSamples samples in one cell: the cell and the index of its first sample (bits), the transmittance and the colour
-// composited before it. n: the records of each ray (more than cap: the ray's records are incomplete).
+// The visits a forward leaves for its backward: per ray up to `cap` records of 8 floats, one per run of samples in one cell (a
+// run ends with the round that takes it to kVisitSamples samples, so it has at most kGroupBatch - 1 more): the cell and the
+// index of its first sample (bits), the transmittance and the colour composited before it. n: the records of each ray (more
+// than cap: the ray's records are incomplete).
 constexpr int kVisitSamples = 32;
 constexpr int kVisitFloats = 8;
 struct MarchVisits {
@@ -1942,11 +1943,14 @@ extern "C" int64_t vgr_march_backward_work_size(int64_t n_sites, int64_t sh_deg)
 namespace vgr {
 namespace {
 // Launches of fewer rays take the 16-lane group layout, for forward and backward alike (the backward replays the
-// forward's sums). Config 5, ms forward / backward, one ray per lane against 16 lanes per ray: 4,096 rays 34 / 85
-// against 5 / 16; 65,536 rays 41 / 189 against 19 / 70; 262,144 rays 75 / 408 against 67 / 251; 1,048,576 rays
-// 236 / 1531 against 255 / 974. A training step (forward + backward) is faster in the group layout at every size
-// measured, a forward alone from about half a million rays in one ray per lane (the whole 16.7M-ray inference
-// batch: 3,350 against 5,264 ms), hence the switch at 2^19 rays.
+// forward's sums). A training step (forward + backward) is faster in the group layout at every size measured and asks for
+// it. A forward alone, ms one ray per lane : 16 lanes, steps of 1/512, scenes of 1M sites (surfaces), 256k (clusters) and
+// 131k (thin):
+//   views in 8x8 tiles   65,536 rays 22 : 12, 15 : 12, 16 : 13; 262,144 rays 38 : 44, 27 : 42, 31 : 46;
+//                        524,176 rays 57 : 80, 48 : 99, 54 : 114; 1M rays 99 : 168, 75 : 160, 84 : 174
+//   incoherent rays      65,536 rays 18 : 8, 13 : 8, 14 : 9; 262,144 rays 33 : 25, 25 : 28, 30 : 32;
+//                        524,176 rays 51 : 49, 40 : 55, 47 : 63; 1M rays 89 : 97, 73 : 108, 86 : 125
+// From 2^19 rays on one ray per lane is at least as fast on all of them; below, it depends on the rays.
 constexpr int64_t kGroupRays = 524288;
 
 int64_t march_lanes(int64_t lanes, int64_t n_rays) { return lanes != 0 ? lanes : n_rays < kGroupRays ? kGroup : 1; }
@@ -2094,9 +2098,8 @@ int march_backward(const float* points, int64_t n_sites, const int32_t* offsets,
     // against 193 ms)
     if (march_lanes(lanes_per_ray, n_rays) == kGroup) {
         if (V.rec != nullptr)
-            hipLaunchKernelGGL(march_visits_kernel, dim3(static_cast<unsigned>(n_rays * kVisitWaves)), dim3(kBlock),
-                0, s, F,
-                               M, R, GI, G, V, stats);
+            hipLaunchKernelGGL(march_visits_kernel, dim3(static_cast<unsigned>(n_rays * kVisitWaves)), dim3(kBlock), 0, s,
+                               F, M, R, GI, G, V, stats);
         hipLaunchKernelGGL(march_group_backward_kernel, dim3(grid_for(n_rays * kGroup, kBlock)), dim3(kBlock), 0, s,
                            F, M, R, GI, G, V);
     } else if (n_rays >= kCoopRays)
@@ -2137,8 +2140,8 @@ extern "C" int vgr_march_backward_visits(const float* points, int64_t n_sites, c
                                         int32_t* n_visits, const int32_t* stats, void* stream) {
     VGR_REQUIRE(n_rays == 0 || (visits && n_visits && stats && visit_cap > 0 && visit_cap <= INT_MAX),
                 "march_backward_visits: visits, n_visits and stats are required, visit_cap in [1, 2^31)");
-    VGR_REQUIRE(n_rays <= vgr::kSplitRays, "march_backward_visits: at most %lld rays", static_cast<long
-        long>(vgr::kSplitRays));
+    VGR_REQUIRE(n_rays <= vgr::kSplitRays, "march_backward_visits: at most %lld rays",
+                static_cast<long long>(vgr::kSplitRays));
     return vgr::march_backward(points, n_sites, offsets, adj, n_adj, raw, dA, cA, sh, sh_deg, o, d, start, near_t,
         mid_t, far_t, n_rays, dt, n_bg, t_thresh, w_thresh, rgb, T, g_rgb, g_T, g_raw, g_dA, g_cA, g_sh, vgr::kGroup,
         blocks_ready, work, work_bytes, vgr::MarchVisits{const_cast<float*>(visits), const_cast<int32_t*>(n_visits),
@@ -2245,10 +2248,9 @@ int foam_backward(const float* points, int64_t n_sites, const int32_t* offsets, 
         VGR_REQUIRE(reinterpret_cast<uintptr_t>(rec) % 16 == 0, "foam_backward: rec must be 16-byte aligned");
         float4* grads = static_cast<float4*>(scratch);
         count = reinterpret_cast<int*>(grads + n_rays * record_cap);
-        hipLaunchKernelGGL(train_grads_kernel, dim3(grid_for(n_rays, kBlock)), dim3(kBlock), 0, s, M, start,
-                           int(n_sites), GI, reinterpret_cast<const float4*>(rec), int(record_cap), stats, n_rays, grads, count);
-        hipLaunchKernelGGL(train_samples_kernel, dim3(static_cast<unsigned>(n_rays * kSampleWaves)), dim3(kBlock), 0,
-            s, F,
+        hipLaunchKernelGGL(train_grads_kernel, dim3(grid_for(n_rays, kBlock)), dim3(kBlock), 0, s, M, start, int(n_sites),
+                           GI, reinterpret_cast<const float4*>(rec), int(record_cap), stats, n_rays, grads, count);
+        hipLaunchKernelGGL(train_samples_kernel, dim3(static_cast<unsigned>(n_rays * kSampleWaves)), dim3(kBlock), 0, s, F,
                            R, G, rec, int(record_cap), grads, count);
     }
     hipLaunchKernelGGL(train_backward_kernel, dim3(grid_for(n_rays * kGroup, kBlock)), dim3(kBlock), 0, s, F, M, R,
