@@ -54,17 +54,23 @@ def copy_probe(dev):
 
 def source_hash(*names):
 	"""16 hex digits of SHA-256 over the named kernel sources (foam_infer.hip: with the files its entry point launches
-	from and their header), the two headers every kernel includes and the hipcc flags: it names the build a DRAM-traffic
-	profile was measured on."""
+	from), the headers of csrc/ they include and the hipcc flags: it names the build a DRAM-traffic profile was measured
+	on."""
 	import hashlib
+	import re
 
 	from vgr import build
 	h = hashlib.sha256()
-	foam = {'foam_tile.hip', 'foam_wide.hip', 'vgr_foam.h'} if 'foam_infer.hip' in names else set()
-	for n in sorted(set(names) | foam | {'vgr_device.h', 'vgr_abi.h'}):
-		h.update(n.encode())
+	todo = set(names) | ({'foam_tile.hip', 'foam_wide.hip'} if 'foam_infer.hip' in names else set())
+	text = {}
+	while todo:
+		n = todo.pop()
 		with open(os.path.join(build.CSRC, n), 'rb') as f:
-			h.update(f.read())
+			text[n] = f.read()
+		todo |= set(re.findall(r'#include "(\w+\.h)"', text[n].decode())) - set(text)
+	for n in sorted(text):
+		h.update(n.encode())
+		h.update(text[n])
 	h.update(' '.join(build.HIPCC_FLAGS).encode())
 	return h.hexdigest()[:16]
 
@@ -389,14 +395,14 @@ def bench_foam(args):
 		key += '-rows64' if pack['rows'].size(1) == 16 else '-blocks256'
 	src = source_hash('foam_infer.hip')
 	log(f'kernel source hash (foam_infer.hip and its kernels): {src}; workload key {key}')
-	tile = lanes == 1 and not args.eps_color > 0 and (mode == 2 or exact_blend)
+	tile = lanes == 1 and (mode == 2 or exact_blend)
 	roofline = hbm_roofline(ms, key, src, abytes,
 							'cache-oblivious gather bytes from the per-ray counters: 56 B per ray + 24 B per sample + '
 							f'{80 if indexed else 84} B per neighbourhood edge + SH bytes per distinct blended site '
 							'(counts every L1/L2/LDS hit as a fetch, so it can exceed the HBM peak)',
 							'foam_tile_kernel' if tile else 'foam_infer_kernel' if lanes == 1 else 'foam_group_kernel')
-	if roofline['frac'] is not None and tile:
-		roofline['limiter'] = ('not HBM: the texture data path is busy 96 % of the launch and the L2 serves 97 % of '
+	if roofline['frac'] is not None and key == 'config3-scale1.0-fused-reorder1-l1-tiles8morton-idx':  # as measured
+		roofline['limiter'] = ('not HBM: the texture data path is busy 97 % of the launch and the L2 serves 97 % of '
 							   'the gathers (profiles/foam_infer_config3_counters.md)')
 
 	cpu = None
@@ -650,12 +656,13 @@ def bench_march_grad(args):
 		# one workspace for both passes, as ext.march's autograd uses it: the backward reuses the forward's blocks
 		work = torch.empty(int(_lib.load().vgr_march_backward_work_size(sc.n_sites, sc.sh_deg)), dtype=torch.uint8,
 						   device=dev)
-		for lanes in (1, 16):  # both ray layouts; the library's default picks 16 below 524288 rays
-			f_ms, out, _ = time_steps(lambda: me.march_forward(*fwd_args, lanes=lanes, work=work), args.steps,
+		for lanes in (1, 16):  # both ray layouts; ext.march's autograd runs 16 lanes per ray, with visit records
+			visits = ext.march_visits(B, dev) if lanes == 16 else None
+			f_ms, out, _ = time_steps(lambda: me.march_forward(*fwd_args, lanes=lanes, work=work, visits=visits), args.steps,
 									  args.warmup, stream)
 			rgb, T, _, stats = out
-			b_ms, grads, _ = time_steps(lambda: me.march_backward(*fwd_args, rgb, T, g_rgb, g_T, lanes=lanes,
-																  work=work), args.steps, args.warmup, stream)
+			b_ms, grads, _ = time_steps(lambda: me.march_backward(*fwd_args, rgb, T, g_rgb, g_T, lanes=lanes, work=work,
+																  visits=visits, stats=stats), args.steps, args.warmup, stream)
 			st = stats.double()
 			fwd_bytes = float(56 * B + st[:, 2].sum() * (8 + 16 * E) + st[:, 0].sum() * (8 + E * 44) +
 							  st[:, 1].sum() * E * (24 + SHB))
@@ -667,8 +674,7 @@ def bench_march_grad(args):
 			log(f'{B} rays, {lanes} lane(s) per ray: forward {L["fwd"]:.3f} ms, backward {L["bwd"]:.3f} ms '
 				f'({bwd_bytes / L["bwd"] / 1e6:.0f} GB/s algorithmic); samples/ray {L["samples"]:.1f}, coloured '
 				f'{L["coloured"]:.1f}')
-	auto = 16 if args.batch < 524288 else 1
-	L = legs[args.batch, auto]
+	L = legs[args.batch, 16]
 	ms = L['fwd'] + L['bwd']
 	cpu = None
 	if args.cpu_seconds > 0:
@@ -695,12 +701,12 @@ def bench_march_grad(args):
 	emit('Mrays/s through march forward + backward (training batch)', mrays_per_s(args.batch, ms), 'Mrays/s', args, ms,
 		 {'workload': f'config 5 uniform march training step: {args.batch} random rays of the config-5 batch, dt = '
 					  f'1/512, 64 bg steps, march_forward + march_backward', 'sites': sc.n_sites,
-		  'rays_per_step': args.batch, 'lanes_per_ray': auto, 'forward_ms': round(L['fwd'], 4),
+		  'rays_per_step': args.batch, 'lanes_per_ray': 16, 'forward_ms': round(L['fwd'], 4),
 		  'backward_ms': round(L['bwd'], 4), 'samples_per_ray': round(L['samples'], 2),
 		  'coloured_per_ray': round(L['coloured'], 2), 'layouts': layouts},
 		 hbm_roofline(L['bwd'], f'config5-march-grad-b{args.batch}', source_hash('march.hip'), L['bytes'],
 					  'cache-oblivious bytes of the backward launch (site blocks per neighbour visit, gradient rows)',
-					  'march_group_backward_kernel' if auto == 16 else 'march_backward_kernel'), cpu)
+					  'march_visits_kernel'), cpu)
 
 
 def sample_words(B, n):
@@ -714,10 +720,10 @@ def mrays_per_s(B, ms):
 
 def bench_locate(args):
 	"""Start-cell location for config 5: the nearest of 4,000,000 sites for each of the 16,777,216 ray origins
-	(vgr_grid_nearest_points over a grid and its cell-ordered sites built once, outside the timed region; the
-	origins answered in their Z-order, computed inside the timed step, unless --order off). CPU baseline: the
-	reference's own nearest_sites (scipy cKDTree, sites.py:38-39, single-threaded as called there) on a bounded
-	sample."""
+	(a grid and its cell-ordered sites built once, outside the timed region; the origins binned into the grid's cells as
+	nearest_sites does, inside the timed step; --order on: in their Z-order instead, computed inside the timed step,
+	--order off: as given). CPU baseline: the reference's own nearest_sites (scipy cKDTree, sites.py:38-39,
+	single-threaded as called there) on a bounded sample."""
 	import numpy as np
 	import torch
 
@@ -731,10 +737,13 @@ def bench_locate(args):
 	stream = torch.cuda.current_stream(dev)
 	build_ms, g, _ = time_steps(lambda: grid.SiteGrid(pts), 3, 1, stream)
 	n_cells = g.res[0] * g.res[1] * g.res[2]
-	ordered = args.order != 'off'  # the origins of a ray batch come in no spatial order
+	ordered = args.order == 'on'
 	pos_bits = args.order_pos_bits or 8
+	as_given = torch.arange(B, dtype=torch.int32, device=dev)
 	if ordered:
 		step = lambda: g.nearest(q, order=grid.query_order(q, pos_bits))  # noqa: E731
+	elif args.order == 'off':
+		step = lambda: g.nearest(q, order=as_given)  # noqa: E731
 	else:
 		step = lambda: g.nearest(q)  # noqa: E731
 	launch_ms, out, wall = time_steps(step, args.steps, args.warmup, stream)
@@ -771,8 +780,10 @@ def bench_locate(args):
 					  f'origins', 'sites': N, 'queries': B, 'grid_res': g.res,
 		  'grid_build_ms': round(float(np.mean(build_ms)), 3),
 		  'query_order': (f'Z-order of the origins, {pos_bits} bits per axis (vgr_ray_order, one direction bin), '
-						  f'inside the timed step' if ordered else 'as given')},
-		 hbm_roofline(ms, 'config5-locate' + (f'-order{pos_bits}' if ordered else ''), source_hash('grid.hip'), abytes,
+						  f'inside the timed step' if ordered else 'as given' if args.order == 'off' else
+						  'binned into the grid\'s cells (vgr_grid_nearest_binned) inside the timed step')},
+		 hbm_roofline(ms, 'config5-locate' + (f'-order{pos_bits}' if ordered else '-given' if args.order == 'off' else
+											  '-binned'), source_hash('grid.hip'), abytes,
 					  'compulsory bytes: each query point, site and grid word read once, each answer written once',
 					  'grid_nearest'), cpu)
 

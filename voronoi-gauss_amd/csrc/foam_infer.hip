@@ -41,7 +41,8 @@ constexpr int kBlock = 64;  // one wave64 per workgroup = one 8x8 ray tile
 //   registers and are checked and replaced once per pass, with static slot indices;
 // - otherwise 8 tags per ray in the wave's LDS, checked and replaced at every lookup in the reference's order.
 //
-// Tuning per colour mode, measured on config 3. Fused and baked colours: 24 slots and 4 overflow blocks (5.8 KB of
+// Tuning per colour mode, measured on config 3; the fused figures are those of one ray per lane, which foam_tile.hip runs now
+// (the group layouts keep these caches). Fused and baked colours: 24 slots and 4 overflow blocks (5.8 KB of
 // LDS per wave), so that 24 waves (6 per SIMD) fit in a CU's 160 KB, and no software pipelining: the registers that
 // pipelined loads hold are worth more as a sixth wave, whose loads cover the latency instead (48 slots at 4 waves,
 // 36 at 5 and 26 at 7 were all slower: 233, 216 and 257 ms against 207 without overflow blocks). Lazy colours take
@@ -1048,11 +1049,16 @@ __global__ void __launch_bounds__(256) slot_table_kernel(const int* __restrict__
 
 // Lanes per ray of vgr_foam_infer and vgr_foam_infer_traced, the faster layout per path on config 3 (8.29M rays,
 // 2M sites, SH degree 3). Traversal and density: 4 lanes per ray (stage 0: 42.6 ms against 60.6 with one ray per
-// lane; stage 1: 59.3 against 67.2); lazy colours: 4 (262.8 against 276.6 ms). Fused and baked colours: one ray
-// per lane (205.9 against 223.0, 249.9 and 290.6 ms at 2, 4 and 8 lanes; baked 107.6 against 109.3 at 2): their
-// colour lookups run for every neighbour of every sample, and the 64 rays of a tile, in the same cell, step through
-// its neighbours together, one site per lookup, where a group's lanes ask for different sites at once (29 % more
-// VALU and LDS instructions per launch at 4 lanes).
+// lane; stage 1: 59.3 against 67.2); lazy colours: 4 (262.8 against 276.6 ms). Fused colours: one ray per lane (foam_tile.hip,
+// 113.2 against 223.0, 249.9 and 290.6 ms at 2, 4 and 8 lanes), baked ones too (107.6 against 109.3 at 2). An incoherent
+// batch is faster with a group, which the caller asks for with an order (config 5: 8 lanes per ray): its rays share no cells,
+// so foam_tile.hip's quads hold one sample each. ms of 262144 and 1M rays in no order, one ray per lane : 8 lanes : the lookup
+// per lane that foam_tile.hip replaced
+//   fused, fp32 SH            131k sites 15.5 : 10.9 : 17.4, 62.7 : 39.8 : 59.9; 256k, thin, every sample coloured 21.0 :
+//                             14.2 : 22.5, 84.7 : 51.7 : 79.3; 1M, surfaces 18.7 : 15.9 : 27.9, 69.9 : 57.7 : 86.8
+//   the same, fp16            12.8 : 8.9 : 13.8, 51.3 : 33.1 : 50.4; 18.1 : 12.1 : 18.7, 72.7 : 45.3 : 69.9
+//   fp16, eps 1e-3            14.5 : - : 12.4, 54.3 : - : 46.8; 20.0 : - : 16.7, 76.3 : - : 63.0
+// so without an order, a cut-off in a thin scene costs up to 21 % more than before; 131072 rays cost 11 to 63 % less.
 constexpr int kDefaultLanes = 0;
 inline int default_lanes(int64_t stage, int64_t color_mode) {
     return stage < 2 || color_mode == kLazy ? 4 : 1;
@@ -1060,14 +1066,20 @@ inline int default_lanes(int64_t stage, int64_t color_mode) {
 
 // Up to this many rays the default layout of the full rendering (stage 2) is 16 lanes per ray (foam_wide.hip): one ray
 // per lane, or four lanes, leaves a launch as long as its longest ray's chain of dependent reads, whatever its size.
-// Measured on a scene of 131k sites with large cells (90 samples per ray) and one of 1M (160 samples), 8x8 tiles, ms of
-// the render call, 16 lanes against the other layout:
-//   exact and fused colours, fp32 SH  8192 rays 0.66 : 2.8, 1.1 : 7.1; 65536 2.8 : 2.5, 4.0 : 7.1; 131072 6.8 : 2.8,
-//   (foam_tile.hip)                   8.8 : 6.3 (rows of pixels instead of tiles: 3.9 : 7.2, 7.4 : 10.6)
-//   baked colours                     8192 rays 0.53 : 1.83, 1.09 : 4.3; 65536 1.33 : 1.92, 2.4 : 5.0; 131072 2.7 : 2.1,
-//                                     4.2 : 5.2
-//   exact with a finite cut-off       65536 rays 2.7 : 3.6, 3.8 : 8.7; 131072 6.5 : 5.4, 8.5 : 11.8
-// The line lies between the sizes where the two scenes break even, for each of them.
+// ms, 16 lanes : the other layout, a pack with derived records, scenes of 131k sites (clusters), 1M (surfaces) and 256k (thin):
+//                                   32768 rays                        98304 rays
+//   exact, fp32 SH       8x8 tiles  1.6 : 1.3, 3.0 : 3.0, 2.0 : 1.7   4.1 : 1.8, 8.0 : 4.2, 5.1 : 2.2
+//   (degree 3)           pixels     1.4 : 1.8, 1.8 : 3.7, 1.7 : 2.4   3.7 : 2.3, 4.7 : 4.7, 4.7 : 3.2
+//                        incoherent 1.2 : 2.9, 1.6 : 4.1, 1.5 : 3.7   3.0 : 4.9, 4.0 : 6.5, 3.9 : 6.8
+//   degree 0             8x8 tiles  0.7 : 1.1, 1.3 : 2.4, 0.8 : 1.4   1.6 : 1.3, 3.2 : 3.1, 2.0 : 1.6
+//                        incoherent 0.7 : 2.4, 1.1 : 3.3, 1.0 : 3.0   1.7 : 3.7, 2.4 : 5.1, 2.6 : 5.2
+//   fp16                 8x8 tiles  0.9 : 1.5, 1.6 : 3.3, 1.1 : 1.9   2.1 : 1.9, 4.3 : 4.3, 2.6 : 2.3
+//                        incoherent 0.9 : 3.0, 1.3 : 4.1, 1.2 : 3.9   2.3 : 4.2, 3.2 : 5.7, 3.2 : 5.9
+//   fused, fp16, eps 1e-3, tiles    0.9 : 1.8, 1.7 : 3.9, 1.1 : 2.2   2.2 : 2.3, 4.4 : 5.1, 2.7 : 2.8
+//   baked                8x8 tiles  0.5 : 1.1, 1.0 : 2.3, 0.6 : 1.3   1.2 : 1.4, 2.4 : 3.0, 1.5 : 1.7
+//   exact, eps 1e-3      8x8 tiles  1.1 : 1.9, 2.2 : 4.6, 1.4 : 2.5   2.8 : 3.1, 5.7 : 9.0, 3.6 : 4.4
+// The line is where coherent batches break even, except with fp32 SH of degree 3 and site blocks, which do near 32768 rays:
+// there it leans to the incoherent ones, whose caller cannot be told apart. Before these two layouts all of them took longer.
 constexpr int64_t kWideRays = 98304;
 
 int foam_entry(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t* nbr, const float* edge,

@@ -1,5 +1,6 @@
 // Inference renderer, one ray per lane with colours evaluated cell by cell on the matrix cores, gfx950: fused colours, and
-// exact ones without a colour cut-off (+inf), for batches that fill the GPU.
+// exact ones without a colour cut-off (+inf), for batches that fill the GPU with rays that share cells (the rule and what
+// incoherent ones cost: default_lanes in foam_infer.hip).
 //
 // Same function as csrc/foam_infer.cu:286-361. A wave renders 64 consecutive rays (an 8 x 8 tile of the host's order). The
 // walk, the exit faces and the density run one ray per lane, as in foam_infer.hip. A colour does not steer a ray: only the
@@ -54,7 +55,7 @@ constexpr int kRayTagSlots = 8;
 // Queued samples per ray: 11.2 / 51.3 ms on the two views of the variants above; 3: 11.6 / 54.1 (smaller batches), 5: 12.0 /
 // 55.1 (LDS).
 constexpr int kDepth = 4;
-// Waves per SIMD: 4 (128 VGPRs) hold the row, the basis and the ray with 18 spills (fp32, SH degree 3; none with fp16);
+// Waves per SIMD: 4 (128 VGPRs) hold the row, the basis and the ray with 13 spills (fp32, SH degree 3; none with fp16);
 // 3 with 8 samples per ray 12.8 / 57.0, 5 spill: 19.9 / 86.7.
 constexpr int kWaves = 4;
 
@@ -227,8 +228,8 @@ __device__ __forceinline__ int count_lookups(const FoamScene& S, int c, int n, f
 // Blends of 64 samples, one per lane, the four samples of a quad in one cell (`cell`, -1 for a quad without samples): lane l
 // reads entry base + l % 4 of its quad's cell, the quad's four lanes share the four entries. `dir` is the sample's direction.
 template <bool IDX, bool HALF, int DEG, bool CUT>
-__device__ __forceinline__ void blend_quads(const FoamScene& S, float color_cut, int cell, const float (&x)[3], const float (&dir)[3],
-                                            float (&C)[3]) {
+__device__ __forceinline__ void blend_quads(const FoamScene& S, float color_cut, int cell, const float (&x)[3],
+                                            const float (&dir)[3], float (&C)[3]) {
     constexpr int NB = (DEG + 1) * (DEG + 1), NV = sh_vec4<HALF, DEG>();
     const int lane = static_cast<int>(threadIdx.x);
     float b[16];
@@ -472,11 +473,15 @@ __global__ void __launch_bounds__(kBlock, kWaves) foam_tile_kernel(FoamScene S, 
 template <bool IDX, bool HALF, bool CUT, bool TABLE, bool EXACT>
 void launch(const FoamScene& S, const FoamParams& P, const FoamRays& R, const FoamOut& O, hipStream_t stream) {
     const dim3 grid(grid_for(R.n, kBlock)), block(kBlock);
+    const auto run = [&](auto deg) {
+        hipLaunchKernelGGL((foam_tile_kernel<IDX, HALF, decltype(deg)::value, CUT, TABLE, EXACT>), grid, block, 0, stream, S, P,
+                           R, O);
+    };
     switch (P.sh_deg) {
-        case 0: hipLaunchKernelGGL((foam_tile_kernel<IDX, HALF, 0, CUT, TABLE, EXACT>), grid, block, 0, stream, S, P, R, O); break;
-        case 1: hipLaunchKernelGGL((foam_tile_kernel<IDX, HALF, 1, CUT, TABLE, EXACT>), grid, block, 0, stream, S, P, R, O); break;
-        case 2: hipLaunchKernelGGL((foam_tile_kernel<IDX, HALF, 2, CUT, TABLE, EXACT>), grid, block, 0, stream, S, P, R, O); break;
-        default: hipLaunchKernelGGL((foam_tile_kernel<IDX, HALF, 3, CUT, TABLE, EXACT>), grid, block, 0, stream, S, P, R, O);
+        case 0: run(std::integral_constant<int, 0>{}); break;
+        case 1: run(std::integral_constant<int, 1>{}); break;
+        case 2: run(std::integral_constant<int, 2>{}); break;
+        default: run(std::integral_constant<int, 3>{});
     }
 }
 

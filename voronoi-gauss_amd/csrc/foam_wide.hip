@@ -4,8 +4,8 @@
 // known only once the cell before has been read, so a launch of few waves lasts as long as its longest chain and its
 // time is the latency of one cell times the cells of a ray. One ray per lane reads a cell's neighbourhood (mean 16.5
 // entries) entry by entry, about 16 dependent rounds; here a group of 16 lanes (one DPP row, 4 rays per wave) reads it
-// in one or two, so a cell costs two memory latencies (its edge records; its neighbours' site records and CSR offsets,
-// which the exit's lane hands on to the next cell) and, where the segment is coloured, a third (SH rows).
+// in one or two: two dependent reads per cell (its edge records; its neighbours' site records and CSR offsets, which the
+// exit's lane hands on to the next cell) and, where the segment is coloured, a third (SH rows).
 //
 // What the batch size decides and what does not:
 // - the cells visited are those of every other layout: the exit is the lexicographic minimum of (t, tie order);
@@ -20,10 +20,11 @@
 // - the reference's cache misses (stats[:, 4]): lane s < 8 of the group holds the ray's tag of slot s; the first and the
 //   last lookup of a slot in a round come from ballots of the low bits of the sites (colour_tags).
 //
-// Bound: latency of the chain up to a few thousand rays, then the vector-memory path (every lane of a wave reads its own
-// site): 16 loads of 16 bytes per entry of a coloured sample. A batch of 4096 rays of 8x8 tiles over 131k sites (90
-// samples per ray, 35 % of the segments coloured) takes 0.53 ms, 6 us per cell of a ray, where one ray per lane takes
-// 12.5 ms; 8192 rays 0.65 against 9.9 ms.
+// Bound: the chain of cells for a few thousand rays, then the vector-memory path (every lane of a wave reads its own site:
+// 16 loads of 16 bytes per entry of a coloured sample). 8192 rays in rows of pixels over 131k sites, exact colours, fp32 SH
+// (2 waves per SIMD, 0.47 ms of GPU time): the texture data path is busy 81 % of it, waves wait 56 % of their cycles, the
+// VALU issues 38 % of the time, the L2 hits 97.7 % and DRAM moves 51 MB. The rule at kWideRays (foam_infer.hip) holds the
+// comparison with the other layouts.
 #include <cmath>
 
 #include "vgr_foam.h"

@@ -21,7 +21,7 @@
 //
 // vgr_morton_codes gives the Z-order keys of the renumbering, with the arithmetic of morton_order (render.py:168-176):
 // q = trunc((p - lo) / max(hi - lo, 1e-12) * 1023) per axis over the bounding box [lo, hi], bit b of axis a at
-// bit 3 b + a of the key; the caller sorts them.
+// bit 3 b + a of the key; vgr_morton_order also sorts them (30-bit keys, a stable radix sort) and gives the permutation.
 #include <rocprim/device/device_radix_sort.hpp>
 
 #include "vgr_abi.h"

@@ -1,5 +1,5 @@
-// What the kernels of the inference renderer share (foam_infer.hip, foam_wide.hip): the scene, ray and output arguments,
-// the field arithmetic and the tie order of the exit faces.
+// What the kernels of the inference renderer share (foam_infer.hip, foam_wide.hip, foam_tile.hip): the scene, ray and output
+// arguments, the field arithmetic and the tie order of the exit faces.
 #pragma once
 
 #include "vgr_abi.h"
@@ -67,8 +67,8 @@ struct FoamOut {
 int launch_foam_wide(const FoamScene& S, const FoamParams& P, const FoamRays& R, const FoamOut& O, int color_mode,
                      bool half, hipStream_t stream);
 
-// Fused colours (exact: the exact colour mode's statistics) with the colour cut-off +inf, one ray per lane, colours evaluated
-// cell by cell on the matrix cores (foam_tile.hip). indexed: S.edge and S.attr are the indexed records.
+// Fused colours, one ray per lane, evaluated cell by cell on the matrix cores (foam_tile.hip); exact: the exact colour mode's
+// statistics (colour cut-off +inf, indexed records and slot table). indexed: S.edge and S.attr are the indexed records.
 int launch_foam_tile(const FoamScene& S, const FoamParams& P, const FoamRays& R, const FoamOut& O, bool indexed, bool exact,
                      bool half, hipStream_t stream);
 

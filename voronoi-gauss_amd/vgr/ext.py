@@ -402,7 +402,8 @@ class _FoamInferExtension:
 
 def index_pack(offsets, nbr, edge, attr):
 	"""Indexed edge records of a foam pack (vgr_foam_index_pack) -> (edge_i (E, 4), attr_i (N, 20)): edge_i[e] =
-	(p_j, the bits of j = nbr[e]), attr_i = attr with column 7 holding site k's cut-off word edge[offsets[k], 3].
+	(p_j, the bits of j = nbr[e]), attr_i = attr with column 7 holding site k's cut-off word edge[offsets[k], 3],
+	the sign of its r2 marking a site whose colour distances need not be numbers (degenerate conic or position).
 	A snapshot of the pack: rebuild it after changing edge or attr."""
 	for t, n, dt in ((offsets, 'offsets', torch.int32), (nbr, 'nbr', torch.int32), (edge, 'edge', torch.float32),
 					 (attr, 'attr', torch.float32)):
