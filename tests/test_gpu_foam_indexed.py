@@ -269,9 +269,10 @@ def test_site_rows_identical_in_group_layouts(gpu, small, lanes):
 
 @pytest.mark.parametrize('sh_half', [False, True])
 @pytest.mark.parametrize('cut', [math.inf, 2 * math.log(1e3)])
-def test_site_rows_identical_in_the_default_layout(gpu, small, sh_half, cut):
-	"""Small batches by the default layout (16 lanes per ray): every colour mode with site rows or blocks, which some modes
-	read and others leave aside, gives the outputs of the attr rows bit for bit."""
+def test_default_layout_reads_the_records_of_the_call(gpu, small, sh_half, cut):
+	"""Small batches by the default layout (16 lanes per ray) read the records and SH rows given to the call in every colour
+	mode, as larger ones do, not their copies in the site rows and blocks: a pack whose colours, conics or densities change
+	after index_pack renders as one without copies, bit for bit."""
 	f, (o, d, start, near, _, far) = small
 	t = lambda a: torch.as_tensor(np.ascontiguousarray(a), device=gpu)  # noqa: E731
 	empty = torch.empty(0, dtype=torch.int32, device=gpu)
@@ -280,9 +281,12 @@ def test_site_rows_identical_in_the_default_layout(gpu, small, sh_half, cut):
 	scene = [t(pk[k]) for k in ('points', 'offsets', 'nbr', 'edge', 'attr', 'sh')]
 	ei, ai = ext.index_pack(*scene[1:5])
 	rows = ai[:, :16].contiguous()
-	records = [(ei, ai), (ei, ai, rows)]
+	records = [None, (ei, ai), (ei, ai, rows)]
 	if not sh_half:
 		records.append((ei, ai, torch.cat([rows, scene[5].reshape(-1, 48)], 1).contiguous()))
+	scene[5] = scene[5].flip(0).contiguous()
+	scene[4][:, 6] -= 0.25
+	scene[4][:, 8:14] *= 1.5
 	for mode in (0, 1, 2):
 		outs = []
 		for idx in records:

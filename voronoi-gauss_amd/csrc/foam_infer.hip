@@ -1068,18 +1068,19 @@ inline int default_lanes(int64_t stage, int64_t color_mode) {
 // per lane, or four lanes, leaves a launch as long as its longest ray's chain of dependent reads, whatever its size.
 // ms, 16 lanes : the other layout, a pack with derived records, scenes of 131k sites (clusters), 1M (surfaces) and 256k (thin):
 //                                   32768 rays                        98304 rays
-//   exact, fp32 SH       8x8 tiles  1.6 : 1.3, 3.0 : 3.0, 2.0 : 1.7   4.1 : 1.8, 8.0 : 4.2, 5.1 : 2.2
-//   (degree 3)           pixels     1.4 : 1.8, 1.8 : 3.7, 1.7 : 2.4   3.7 : 2.3, 4.7 : 4.7, 4.7 : 3.2
-//                        incoherent 1.2 : 2.9, 1.6 : 4.1, 1.5 : 3.7   3.0 : 4.9, 4.0 : 6.5, 3.9 : 6.8
-//   degree 0             8x8 tiles  0.7 : 1.1, 1.3 : 2.4, 0.8 : 1.4   1.6 : 1.3, 3.2 : 3.1, 2.0 : 1.6
-//                        incoherent 0.7 : 2.4, 1.1 : 3.3, 1.0 : 3.0   1.7 : 3.7, 2.4 : 5.1, 2.6 : 5.2
-//   fp16                 8x8 tiles  0.9 : 1.5, 1.6 : 3.3, 1.1 : 1.9   2.1 : 1.9, 4.3 : 4.3, 2.6 : 2.3
-//                        incoherent 0.9 : 3.0, 1.3 : 4.1, 1.2 : 3.9   2.3 : 4.2, 3.2 : 5.7, 3.2 : 5.9
-//   fused, fp16, eps 1e-3, tiles    0.9 : 1.8, 1.7 : 3.9, 1.1 : 2.2   2.2 : 2.3, 4.4 : 5.1, 2.7 : 2.8
-//   baked                8x8 tiles  0.5 : 1.1, 1.0 : 2.3, 0.6 : 1.3   1.2 : 1.4, 2.4 : 3.0, 1.5 : 1.7
-//   exact, eps 1e-3      8x8 tiles  1.1 : 1.9, 2.2 : 4.6, 1.4 : 2.5   2.8 : 3.1, 5.7 : 9.0, 3.6 : 4.4
-// The line is where coherent batches break even, except with fp32 SH of degree 3 and site blocks, which do near 32768 rays:
-// there it leans to the incoherent ones, whose caller cannot be told apart. Before these two layouts all of them took longer.
+//   exact, fp32 SH       8x8 tiles  1.1 : 1.3, 2.2 : 3.0, 1.4 : 1.7   2.9 : 1.8, 5.9 : 4.2, 3.7 : 2.2
+//   (degree 3)           pixels     1.1 : 1.8, 1.5 : 3.7, 1.4 : 2.4   2.8 : 2.3, 3.8 : 4.7, 3.6 : 3.2
+//                        incoherent 1.2 : 2.9, 1.6 : 4.1, 1.7 : 3.7   3.4 : 4.9, 4.1 : 6.5, 4.6 : 6.8
+//   degree 0             8x8 tiles  0.6 : 1.1, 1.2 : 2.5, 0.7 : 1.4   1.4 : 1.3, 3.0 : 3.0, 1.8 : 1.6
+//                        incoherent 0.9 : 2.4, 1.3 : 3.3, 1.3 : 3.0   2.5 : 3.7, 3.3 : 5.2, 3.5 : 5.2
+//   fp16                 8x8 tiles  0.8 : 1.5, 1.6 : 3.3, 1.0 : 1.8   2.0 : 1.9, 4.1 : 4.3, 2.5 : 2.3
+//                        incoherent 1.0 : 3.1, 1.4 : 4.0, 1.4 : 3.9   2.5 : 4.3, 3.3 : 5.7, 3.6 : 5.9
+//   fused, fp16, eps 1e-3, tiles    0.8 : 1.8, 1.5 : 3.9, 1.0 : 2.2   2.0 : 2.3, 3.9 : 5.1, 2.5 : 2.8
+//   baked                8x8 tiles  0.5 : 1.1, 1.0 : 2.3, 0.6 : 1.3   1.2 : 1.4, 2.5 : 2.9, 1.5 : 1.8
+//   exact, eps 1e-3      8x8 tiles  1.1 : 2.0, 2.2 : 4.6, 1.4 : 2.5   2.8 : 3.2, 5.7 : 9.0, 3.6 : 4.4
+// The line is where coherent batches break even, except with fp32 SH of degree 3, which do between 32768 and 65536 rays (2.2 : 1.6,
+// 3.9 : 3.4, 2.8 : 1.9): there it leans to the incoherent ones, whose caller cannot be told apart. Before these two layouts
+// all of them took longer.
 constexpr int64_t kWideRays = 98304;
 
 int foam_entry(const float* points, int64_t n_sites, const int32_t* offsets, const int32_t* nbr, const float* edge,
@@ -1129,16 +1130,10 @@ int foam_entry(const float* points, int64_t n_sites, const int32_t* offsets, con
     // 64-byte rows); the two-pass exact colours with 4 lanes per ray ran slower on them (268.9 against 258.3 ms on
     // config 3) and keep the attr rows, as the one-ray-per-lane kernels do. Site blocks also supply the SH rows of the
     // kernels that read them, 16 float4 apart after each 4-float4 record.
-    // 16 lanes per ray read 64-byte rows (fp16 SH, 65536 incoherent rays 1.98 -> 1.80 ms, coherent ones the same), and blocks
-    // where the SH row follows the record: exact and fused colours. Baked colours have no SH row, and exact ones with a
-    // cut-off read few of them: there a coherent batch pays for lines it does not use (8x8 tiles, baked: 98304 rays 1.67 ms
-    // with blocks, 1.44 without, 1.59 with one ray per lane; exact, eps 1e-3: 65536 rays 3.2 and 3.8 ms with blocks, 2.4 and
-    // 2.9 without, 2.7 and 3.4 with 4 lanes per ray; incoherent rays 1.82 and 1.25 ms, 2.2 and 2.4).
-    const bool cut_off = !(std::isinf(color_cut) && color_cut > 0);
-    const bool wide_rows =
-        wide && (row_floats == 16 ? color_mode != kBaked : color_mode == kFused || (color_mode == kLazy && !cut_off));
-    const bool rows_used =
-        rows != nullptr && stage == 2 && (wide ? wide_rows : !indexed && color_mode == kFused && lanes > 1);
+    // 16 lanes per ray read the attr and SH rows of the call too: the rows are a snapshot, which only layouts that a caller
+    // asks for read. (Coherent batches are faster without: 8x8 tiles, 65536 rays of two scenes, exact 3.2 and 4.0 ms with
+    // blocks, 2.4 and 2.9 without; incoherent ones slower: 2.3 and 2.9, 2.5 and 3.3.)
+    const bool rows_used = rows != nullptr && stage == 2 && !wide && !indexed && color_mode == kFused && lanes > 1;
     const bool blocks = rows_used && row_floats == 64;
     const FoamScene S{reinterpret_cast<const float4*>(points),
                       offsets,

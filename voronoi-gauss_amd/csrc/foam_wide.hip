@@ -22,8 +22,8 @@
 //
 // Bound: the chain of cells for a few thousand rays, then the vector-memory path (every lane of a wave reads its own site:
 // 16 loads of 16 bytes per entry of a coloured sample). 8192 rays in rows of pixels over 131k sites, exact colours, fp32 SH
-// (2 waves per SIMD, 0.47 ms of GPU time): the texture data path is busy 81 % of it, waves wait 56 % of their cycles, the
-// VALU issues 38 % of the time, the L2 hits 97.7 % and DRAM moves 51 MB. The rule at kWideRays (foam_infer.hip) holds the
+// (2 waves per SIMD, 0.40 ms of GPU time): the texture data path is busy 78 % of it, waves wait 46 % of their cycles, the
+// VALU issues 44 % of the time, the L2 hits 97.5 % and DRAM moves 55 MB. The rule at kWideRays (foam_infer.hip) holds the
 // comparison with the other layouts.
 #include <cmath>
 
@@ -89,9 +89,7 @@ __device__ __forceinline__ void row_exit(const FoamScene& S, float& t, int& k) {
     min_step<kMirror>(S, t, k);
 }
 
-__device__ __forceinline__ const float4* record(const FoamScene& S, int k) {
-    return S.rows != nullptr ? S.rows + S.row_stride * static_cast<int64_t>(k) : S.attr + 5 * static_cast<int64_t>(k);
-}
+__device__ __forceinline__ const float4* record(const FoamScene& S, int k) { return S.attr + 5 * static_cast<int64_t>(k); }
 
 // One entry of a neighbourhood: its edge record and site, and whether the lane has one.
 struct Entry {
