@@ -121,6 +121,24 @@ def test_native_bake_matches_float64(model, gpu, deg):
 	ext.bake_colors(pk['points'][:0], pk['sh32'][:0], deg, center, pk['attr'][:0])
 
 
+@pytest.mark.parametrize('index', [False, True])
+def test_pack_asks_the_model_for_its_sh_rows(gpu, monkeypatch, index):
+	"""The packed SH rows are those of model.sh(), also where a subclass, the object or the class has another one."""
+	sc = scenes.make_scene(1, cache_dir=None, log=None)
+	m = VoronoiGaussField.from_scene(sc, gpu)
+	own = m.sh().detach()
+	dimmed = lambda self: 0.5 * torch.cat([self.sh_dc, self.sh_rest], 1)  # noqa: E731
+	assert torch.equal(render.pack_foam(m, index=index)['sh32'], own)
+	m.__class__ = type('Dimmed', (VoronoiGaussField,), {'sh': dimmed})
+	assert torch.equal(render.pack_foam(m, index=index)['sh32'], 0.5 * own)
+	m.__class__ = VoronoiGaussField
+	m.sh = lambda: dimmed(m)
+	assert torch.equal(render.pack_foam(m, index=index)['sh32'], 0.5 * own)
+	del m.sh
+	monkeypatch.setattr(VoronoiGaussField, 'sh', dimmed)
+	assert torch.equal(render.pack_foam(m, index=index)['sh32'], 0.5 * own)
+
+
 def test_native_pack_errors(gpu):
 	pts = torch.zeros(4, 3, device=gpu)
 	with pytest.raises(RuntimeError, match='float32|CUDA|sh must'):

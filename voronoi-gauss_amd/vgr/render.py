@@ -13,6 +13,8 @@ import torch.nn.functional as F
 from . import ext
 from .model import VoronoiGaussField
 
+_FIELD_SH = VoronoiGaussField.sh  # the field's own
+
 # ---------------------------------------------------------------------------------------------------- ray bounds
 
 
@@ -306,8 +308,9 @@ def pack_foam(model, scale_floor=0.0, eps_density=0.0, sh_half=False, reorder=Fa
 	perm = inv = orig = None
 	if reorder:
 		perm, inv, orig = ext.morton_order(g.points)
-	# a field's SH rows are read from its two parameters, without the copy that joins them
-	parts = isinstance(model, VoronoiGaussField) and type(model).sh is VoronoiGaussField.sh and index
+	# a field's SH rows are read from its two parameters, without the copy that joins them, unless its sh() is another one
+	# (of a subclass, set on the object or on the class)
+	parts = index and isinstance(model, VoronoiGaussField) and getattr(model.sh, '__func__', None) is _FIELD_SH
 	sh = (model.sh_dc.detach().contiguous(), model.sh_rest.detach().contiguous()) if parts else \
 		model.sh().detach().float().contiguous()
 	if parts and any(t.dtype != torch.float32 for t in sh):
